@@ -19,7 +19,45 @@ struct DeviceWorkspace {
 std::mutex g_ws_mutex;
 std::vector<DeviceWorkspace> g_ws;
 std::vector<int> g_cus;
+std::vector<hipMemPool_t> g_pools;
+
+// The current device's scratch pool (made on first use; NULL if that fails).
+hipMemPool_t scratch_pool() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  if ((size_t)dev >= g_pools.size()) g_pools.resize(dev + 1, nullptr);
+  if (!g_pools[dev]) {
+    hipMemPoolProps props = {};
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    hipMemPool_t p = nullptr;
+    if (hipMemPoolCreate(&p, &props) != hipSuccess) return nullptr;
+    uint64_t keep = kGqScratchMax;
+    if (hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+      (void)hipMemPoolDestroy(p);
+      return nullptr;
+    }
+    g_pools[dev] = p;
+  }
+  return g_pools[dev];
+}
 }  // namespace
+
+GqScratch::GqScratch(size_t bytes, hipStream_t s) : stream(s) {
+  if (bytes > kGqScratchMax) return;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  hipMemPool_t pool = nullptr;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone || !(pool = scratch_pool()) ||
+      hipMallocFromPoolAsync(&ptr, bytes, pool, s) != hipSuccess) {
+    ptr = nullptr;
+    (void)hipGetLastError();  // (the caller takes a route without scratch)
+  }
+}
+GqScratch::~GqScratch() {
+  if (ptr) (void)hipFreeAsync(ptr, stream);
+}
 
 int gq_hip_status(hipError_t e) {
   if (e == hipSuccess) return GQ_OK;
@@ -219,9 +257,18 @@ int gq_unpack_host(int fmt, const void *packed, size_t N, size_t K, void *gguf) 
 int gq_matmul(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K, void *stream) {
   if (M >= 1 && M <= GQ_MAX_BATCH)
     return gq_gemv(fmt, packed, a, c, N, K, (int)M, nullptr, 0, stream);
-  int ct = 0, nck = 0;
-  if (gq_fmt_is_q6k(fmt) && gq_gemm_skinny_plan(fmt, M, N, K, &ct, &nck) != GQ_OK) {
-    // K too long for the skinny kernel: batches of 16 rows through the GEMV
+  if (gq_fmt_is_q6k(fmt) && (K > 4096 || M == 0 || N == 0 || K == 0)) {
+    // gq_gemm refuses Q6_K past K = 4096: the tiled kernel on scratch memory,
+    // or batches of 16 rows through the GEMV where there is none.  Two or three
+    // GEMV passes over few columns also beat the tiled kernel, whose few
+    // workgroups each walk K in steps (17 / 33 / 48 / 64 rows, 4096 x 14336: GEMVs
+    // 38 / 66 / 82 / 109 us, tiled 79 / 79 / 80 / 82; 14336 x 14336: 83 / 132 / 143 /
+    // 190 against 95 / 96 / 98 / 100; 512 x 4096 x 14336: 861 against 99)
+    if ((M > 48 || (M > 32 && N >= 8192)) && M <= GQ_MAX_DIM && N > 0 && K > 0 && packed && a && c &&
+        gq_check_shape(fmt, N, K) == GQ_OK) {
+      const int r = gq_launch_matmul_q6k(fmt, packed, a, c, M, N, K, (hipStream_t)stream);
+      if (r != GQ_ERR_WORKSPACE && r != GQ_ERR_UNSUPPORTED) return r;
+    }
     for (size_t m0 = 0; m0 < M; m0 += GQ_MAX_BATCH) {
       const size_t mb = M - m0 < GQ_MAX_BATCH ? M - m0 : GQ_MAX_BATCH;
       GQ_TRY(gq_gemv(fmt, packed, a + m0 * K, c + m0 * N, N, K, (int)mb, nullptr, 0, stream));

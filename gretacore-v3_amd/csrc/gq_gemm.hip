@@ -460,6 +460,16 @@ struct RStep<GQ_FMT_Q4_K, NJ> {
   gq_u2 q[NJ][2];
   gq_u4 meta[NJ];  // d, dmin, W1, W2, W3 of the column's super-block
 };
+template <int NJ>
+struct RStep<GQ_FMT_Q6_K, NJ> {
+  gq_u2 q[NJ][2];      // low nibbles: the code groups of slots kh, 2 + kh
+  uint32_t hi[NJ][2];  // their high 2-bit fields
+  uint32_t sc[NJ];     // the step's four int8 scales (one per 16 k)
+  uint32_t d[NJ];      // the super-block's d (fp16 bits)
+};
+// loads of one column block and K step
+template <int FMT>
+constexpr int kRLoads = FMT == GQ_FMT_Q6_K ? 6 : 3;
 
 // Buffer resource over the 4 GiB from p (raw: stride 0, the offset in
 // bytes).  The register-B kernel addresses its operands as a 32-bit per-lane
@@ -478,6 +488,13 @@ GQ_DEV gq_u4 ld16_b(const void *base, uint32_t vo, uint32_t so) {
   return gq_u4{v[0], v[1], v[2], v[3]};
 }
 
+GQ_DEV uint32_t ld4_b(const void *base, uint32_t vo, uint32_t so) {
+  return __builtin_amdgcn_raw_buffer_load_b32(gq_rsrc(base), vo, so, 0);
+}
+GQ_DEV uint32_t ld2_b(const void *base, uint32_t vo, uint32_t so) {
+  return __builtin_amdgcn_raw_buffer_load_b16(gq_rsrc(base), vo, so, 0);
+}
+
 template <int FMT, int NJ>
 GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_t (&so)[NJ], int step,
                        RStep<FMT, NJ> &st) {
@@ -493,6 +510,17 @@ GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_
       st.q[j][0] = ld16_b(w, qo[j], b);
       st.q[j][1] = ld16_b(w, qo[j] + 512u, b);
       st.d[j] = ld8_b(w, so[j], (uint32_t)(step >> 1) * 128u);
+    } else if constexpr (FMT == GQ_FMT_Q6_K) {
+      // (d: from the row's scale bytes at 16 r to its d at 256 + 2 r)
+      const uint32_t m = (uint32_t)step & 3u, c = (uint32_t)step >> 2;
+      const uint32_t b = c * 3072u + ((m >> 1) << 10) + 8u * (m & 1u), bh = c * 3072u + 2048u + 4u * m;
+      const uint32_t r = threadIdx.x & 15u;
+      st.q[j][0] = ld8_b(w, qo[j], b);
+      st.q[j][1] = ld8_b(w, qo[j] + 512u, b);
+      st.hi[j][0] = ld4_b(w, qo[j], bh);
+      st.hi[j][1] = ld4_b(w, qo[j] + 512u, bh);
+      st.sc[j] = ld4_b(w, so[j], c * 288u + 4u * m);
+      st.d[j] = ld2_b(w, so[j] - 14u * r, c * 288u + 256u);
     } else {
       const int m = step & 3;
       const uint32_t b = ((uint32_t)(step >> 2) << 11) + ((uint32_t)(m >> 1) << 10) + 8u * (uint32_t)(m & 1);
@@ -564,14 +592,41 @@ GQ_DEV void q4k_factors(const RStep<GQ_FMT_Q4_K, NJ> &st, int step, QKf (&f)[NJ]
   }
 }
 
+// Q6_K: the scales d sc of the step's two 16-element groups this lane holds
+// (2 h + kh, h = 0, 1), each product rounded once to fp16.
+template <int NJ>
+GQ_DEV void q6k_factors(const RStep<GQ_FMT_Q6_K, NJ> &st, int kh, gq_half2 (&f)[NJ][2]) {
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)st.d[j]);
+    const uint32_t s = st.sc[j] >> (8 * kh);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const _Float16 hs = (_Float16)(d * (float)(int8_t)((s >> (16 * h)) & 0xFFu));
+      f[j][h] = gq_half2{hs, hs};
+    }
+  }
+}
+
 // B fragment of column block j, MFMA k-step ks, K step `step`: 8 fp16 values
-// (c - bias) * scale (Q4_K: d sc c - dmin m, factors from q4k_factors), each
-// rounded once.
+// (c - bias) * scale (Q4_K: d sc c - dmin m, factors from q4k_factors; Q6_K:
+// factors from q6k_factors), each rounded once.
 template <int FMT, int NJ>
-GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const QKf *qk, uint32_t mg) {
+GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const QKf *qk, const gq_half2 *q6,
+                      uint32_t mg) {
   const int h = ks >> 1;
   gq_half2 p[4];
-  if constexpr (FMT == GQ_FMT_Q8_0) {
+  if constexpr (FMT == GQ_FMT_Q6_K) {
+    // slots 8 (ks & 1) + 0..3 in the low nibbles, + 4..7 in the high ones; the
+    // high fields of the first four at bits 4 (ks & 1), of the next at + 2
+    const uint32_t w = st.q[j][h][ks & 1], hw = st.hi[j][h];
+    const uint32_t h0 = (ks & 1) ? hw : hw << 4, h1 = (ks & 1) ? hw >> 2 : hw << 2;
+    bytes_to_magic((w & 0x0F0F0F0Fu) | (h0 & 0x30303030u), p[0], p[1]);
+    bytes_to_magic(((w >> 4) & 0x0F0F0F0Fu) | (h1 & 0x30303030u), p[2], p[3]);
+    const gq_half2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};  // codes 0..63, -32
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = (p[i] + off) * q6[h];
+  } else if constexpr (FMT == GQ_FMT_Q8_0) {
     const gq_u4 &q = st.q[j][h];
     const uint32_t w0 = q[2 * (ks & 1)] ^ 0x80808080u, w1 = q[2 * (ks & 1) + 1] ^ 0x80808080u;
     const uint32_t db = st.d[j][h];
@@ -654,7 +709,7 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   constexpr int NA = BM / (8 * NW);  // activation-tile loads per thread and K step
   // loads a step may leave in flight at its end: the activation tiles of
   // steps s + 2 .. s + PD - 1 and the weights of steps s + 2 .. s + PD
-  constexpr int pend = (PD - 2) * NA + (PD - 1) * 3 * NJ;
+  constexpr int pend = (PD - 2) * NA + (PD - 1) * kRLoads<FMT> * NJ;
   static_assert(pend <= 63, "vmcnt immediate");
   constexpr int kWaitPend = 0x0F70 | (pend & 15) | ((pend >> 4) << 14);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -681,6 +736,9 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     } else if constexpr (FMT == GQ_FMT_Q8_0) {
       qo[j] = (tc << 11) + slot;
       so[j] = sc_off + tc * 128u + 8u * r;
+    } else if constexpr (FMT == GQ_FMT_Q6_K) {
+      qo[j] = tc * 3072u + slot;
+      so[j] = sc_off + tc * 288u + 16u * r;
     } else {
       qo[j] = (tc << 11) + slot;
       so[j] = sc_off + tc * 256u + 16u * r;
@@ -725,12 +783,14 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     read_a(0, 0);
     QKf qk[NJ][2];
     if constexpr (FMT == GQ_FMT_Q4_K) q4k_factors<NJ>(cur, step, qk);
+    gq_half2 q6[NJ][2];
+    if constexpr (FMT == GQ_FMT_Q6_K) q6k_factors<NJ>(cur, kh, q6);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks + 1 < KS) read_a(ks + 1, (ks + 1) & 1);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const gq_half8 bf = rfrag<FMT, NJ>(cur, j, ks, step, qk[j], mg);
+        const gq_half8 bf = rfrag<FMT, NJ>(cur, j, ks, step, qk[j], q6[j], mg);
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[i][j] = gq_mfma32(af[ks & 1][i], bf, acc[i][j]);
       }
@@ -1171,9 +1231,26 @@ int launch_fmt(const void *packed, const _Float16 *a16, int lda, void *c, const 
   }
 }
 
+// Q6_K: the shapes pick_tile chooses by itself for whole chunks of 256 k (the
+// step count is then a multiple of 4)
+template <int FMT, int CBF16>
+int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
+                  hipStream_t s) {
+  switch (pick_tile(FMT, M, N, K)) {
+  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 3);
+  case 13: return launch_rb<FMT, CBF16, 128, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s);
+  case 17: return launch_rb<FMT, CBF16, 128, 128, 1, 4, 2>(packed, a16, lda, c, rs, M, N, K, s);
+  default: return launch_rb<FMT, CBF16, 64, 128, 1, 4, 4>(packed, a16, lda, c, rs, M, N, K, s);
+  }
+}
+
 template <int FMT>
 int launch_gemm(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int c_dtype, int M, int N,
                 int K, hipStream_t s) {
+  if constexpr (FMT == GQ_FMT_Q6_K)
+    return c_dtype == GQ_DT_BF16 ? launch_fmt_kg<FMT, 1>(packed, a16, lda, c, rs, M, N, K, s)
+                                 : launch_fmt_kg<FMT, 0>(packed, a16, lda, c, rs, M, N, K, s);
+  else
   return c_dtype == GQ_DT_BF16 ? launch_fmt<FMT, 1>(packed, a16, lda, c, rs, M, N, K, s)
                                : launch_fmt<FMT, 0>(packed, a16, lda, c, rs, M, N, K, s);
 }
@@ -1197,8 +1274,11 @@ static bool gemm_converts_a(int fmt, size_t M, size_t N, size_t K, int a_dtype) 
   if (gq_gemm_skinny_plan(fmt, M, N, K, &ct, &nck) == GQ_OK) return true;
   const int tile = pick_tile(fmt, (int)M, (int)N, (int)K);
   const bool q4 = (fmt == GQ_FMT_Q4_0 || gq_fmt_is_q4k(fmt)) && tile != 1 && tile != 2 && tile != 3;
-  return a_dtype != GQ_DT_F16 || gq_kpad(fmt, K) != K || q4;
+  return a_dtype != GQ_DT_F16 || gq_kpad(fmt, K) != K || q4 || gq_fmt_is_q6k(fmt);
 }
+
+static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s);
 
 extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M,
                        size_t N, size_t K, void *ws, size_t ws_bytes, void *stream) {
@@ -1212,7 +1292,31 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
   GQ_CHECK(K > 0, GQ_ERR_INVALID_ARGS);
   // the kernel addresses the packed tensor with 32-bit offsets
   GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32), GQ_ERR_INVALID_ARGS);
-  hipStream_t s = (hipStream_t)stream;
+  // Q6_K: K <= 4096 (gq_matmul takes any K)
+  GQ_CHECK(!gq_fmt_is_q6k(fmt) || K <= 4096, GQ_ERR_UNSUPPORTED);
+  return gemm_core(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ws, ws_bytes, (hipStream_t)stream);
+}
+
+// gq_matmul's Q6_K rows beyond the GEMV batches, any K: blocks of rows whose
+// converted activations fit a scratch buffer.  GQ_ERR_WORKSPACE without one
+// (the stream is being captured, or no memory), GQ_ERR_UNSUPPORTED where the
+// tiled kernel's 32-bit offsets do not reach; nothing is launched then.
+int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,
+                         hipStream_t s) {
+  const size_t row = gq_kpad(fmt, K) * 2;
+  GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32) && 256 * row <= kGqScratchMax / 2, GQ_ERR_UNSUPPORTED);
+  const size_t fit = (kGqScratchMax / 2 / row) & ~(size_t)255, mb = M < fit ? M : fit;
+  const size_t bytes = gq_gemm_workspace_bytes(fmt, mb, K);
+  GqScratch ws(bytes, s);
+  GQ_CHECK(ws.ptr, GQ_ERR_WORKSPACE);
+  for (size_t m0 = 0; m0 < M; m0 += mb)
+    GQ_TRY(gemm_core(fmt, packed, a + m0 * K, GQ_DT_F32, c + m0 * N, GQ_DT_F32, M - m0 < mb ? M - m0 : mb, N, K,
+                     ws.ptr, bytes, s));
+  return GQ_OK;
+}
+
+static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s) {
   // Few rows: the tiled GEMM gives N / 64 .. N / 128 workgroups, each walking
   // all of K (37-55 us at 4096 x 4096 or 14336 x 4096 for any M <= 256); the
   // skinny kernel takes the shapes gq_gemm_skinny_plan accepts (4096 x 4096:
@@ -1240,8 +1344,6 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
     return gq_launch_gemm_skinny(fmt, packed, (const _Float16 *)ws, (int)ldo, c, rs, c_dtype == GQ_DT_BF16, (int)M, (int)N,
                                  (int)K, s);
   }
-  // Q6_K has no tiled kernel (gq_matmul runs the batch GEMV per 16 rows)
-  GQ_CHECK(!gq_fmt_is_q6k(fmt), GQ_ERR_UNSUPPORTED);
   const _Float16 *a16 = (const _Float16 *)a;
   const float *rs = nullptr;
   // the register-B kernel takes the 4-bit formats' B fragments in the
@@ -1267,6 +1369,8 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
   switch (fmt) {
   case GQ_FMT_Q4_0: return launch_gemm<GQ_FMT_Q4_0>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
   case GQ_FMT_Q8_0: return launch_gemm<GQ_FMT_Q8_0>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
+  case GQ_FMT_Q6_K:
+  case GQ_FMT_Q6_K_GGML: return launch_gemm<GQ_FMT_Q6_K>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
   default: return launch_gemm<GQ_FMT_Q4_K>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
   }
 }

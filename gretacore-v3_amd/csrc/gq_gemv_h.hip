@@ -1131,8 +1131,9 @@ extern "C" int gq_launch_gemm_mfma_mixed_f16f32(void *stream, const float *a, co
 int gq_gemm_skinny_plan(int fmt, size_t M, size_t N, size_t K, int *ct_out, int *nck_out) {
   const char *e = getenv("GQ_GEMM_SKINNY");
   if ((e && e[0] == '0') || getenv("GQ_GEMM_TILE")) return GQ_ERR_UNSUPPORTED;  // (a forced tiled shape)
-  // Q6_K (no tiled GEMM; the alternative is the batch GEMV per 16 rows): any
-  // M, at most 2 chunks per wave (K <= 4096; its chunks take 17 registers)
+  // Q6_K: at most 2 chunks per wave (K <= 4096; its chunks take 17
+  // registers), any M (512 x 1024 x 4096: 22 us against 32 on the tiled kernel,
+  // whose few workgroups each walk K alone)
   const bool q6 = gq_fmt_is_q6k(fmt);
   if (M == 0 || (!q6 && M > 256) || N == 0 || K == 0) return GQ_ERR_UNSUPPORTED;
   const int f = gq_fmt_is_q4k(fmt) ? GQ_FMT_Q4_K : q6 ? GQ_FMT_Q6_K : fmt;
@@ -1161,7 +1162,11 @@ int gq_gemm_skinny_plan(int fmt, size_t M, size_t N, size_t K, int *ct_out, int 
   // is (4096 x 4096 at 64 / 128 rows: 15.6 / 17.5 vs 20-23 us)
   // (GQ_GEMM_SKINNY=2: up to two per CU, for tuning)
   const size_t lim = (nckp >= 16 || (e && e[0] == '2')) ? 2 * cus : cus;
-  if (!q6 && wgs > lim) return GQ_ERR_UNSUPPORTED;
+  // Q6_K stays here for up to 40 rows, whose one row block reads the weights
+  // once either way (17 x 14336 x 4096: 22.5 us against 28.4 tiled; 48 rows: 29.3
+  // against 29.2), and where the tiled kernel's 32-bit activation offsets end
+  const bool q6_any = q6 && (M <= 40 || M * gq_kpad(fmt, K) * 2 >= ((size_t)1 << 32));
+  if (!q6_any && wgs > lim) return GQ_ERR_UNSUPPORTED;
   *ct_out = ct;
   *nck_out = nckp;
   return GQ_OK;

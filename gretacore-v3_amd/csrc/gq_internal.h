@@ -67,5 +67,25 @@ int gq_launch_f16_to_f32(const void *in, size_t n, float *out, hipStream_t s);
 
 // Library-owned per-device workspace (grown on demand, never shrunk).
 int gq_default_workspace(size_t bytes, void **ptr);
+// Scratch memory of one call on stream s, ordered with the stream: from a pool
+// of the current device that keeps at most kGqScratchMax bytes between calls
+// (more goes back to the device as its work ends).  Each call has its own
+// block, so calls on other streams and threads do not meet.  ptr is NULL where
+// no block is to be had: more than kGqScratchMax asked for, no memory left, or
+// a stream under capture (an allocation would become part of the graph).
+constexpr size_t kGqScratchMax = (size_t)256 << 20;
+struct GqScratch {
+  void *ptr = nullptr;
+  GqScratch(size_t bytes, hipStream_t s);
+  ~GqScratch();
+  GqScratch(const GqScratch &) = delete;
+  GqScratch &operator=(const GqScratch &) = delete;
+
+private:
+  hipStream_t stream;
+};
+// Q6_K rows of gq_matmul through the tiled GEMM (gq_gemm.hip)
+int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,
+                         hipStream_t s);
 // Compute units of the current device (cached per device; 0 without a device).
 int gq_device_cus(void);

@@ -47,10 +47,12 @@ extern "C" {
 /* accepted by gq_dequant_gguf only (loader conversions) */
 #define GQ_FMT_F16 1         /* one "block" = one fp16 value (weight_loader.cpp:91-110) */
 /* Q6_K (both layouts): T16 repack, dequant, gq_gemv (int8 matrix-core
-   kernel at batch 1..2, fp16 above) and gq_gemm for K <= 4096 (skinny kernel,
-   any M); gq_gemv_multi / gq_gemv_swiglu run their fallback for it (RMSNorm,
+   kernel at batch 1..2, fp16 above) and gq_gemm for K <= 4096 (skinny or tiled
+   kernel); gq_gemv_multi / gq_gemv_swiglu run their fallback for it (RMSNorm,
    one gq_gemv per matrix); gq_gemm with longer K and gq_gemv_prep / prepped
-   return GQ_ERR_UNSUPPORTED for it (gq_matmul then runs 16-row GEMV batches). */
+   return GQ_ERR_UNSUPPORTED for it.  gq_matmul takes any K: beyond 4096 the tiled
+   kernel on scratch memory of the call's own (stream-ordered), or 16-row GEMV
+   batches up to 48 rows and while the stream is being captured. */
 
 /* activation / output dtypes */
 #define GQ_DT_F32 0

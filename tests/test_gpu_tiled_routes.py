@@ -1,0 +1,95 @@
+"""Tiled-GEMM routes of Q6_K weights against float64 products of the
+dequantized weights (the oracle's), at the edges of each tile shape."""
+import threading
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+# A and W rounded once to fp16 each: relative error <= 2^-11 per factor, about
+# 3.5e-4 over a row in the 2-norm; 1e-3 bounds it
+TOL = 1e-3
+
+
+def _ref(fmt, w, a, n, k):
+    import torch
+    wd = torch.from_numpy(O.dequant(fmt, w).reshape(n, k)).cuda().double()
+    return a.double().cuda() @ wd.t()
+
+
+def _rel(c, ref):
+    return float((c.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("fmt", [O.Q6_K, O.Q6_K_GGML])
+@pytest.mark.parametrize("m,n,k", [
+    (4865, 5300, 256),   # 256 x 256 tiles, one row and 180 columns over
+    (700, 8300, 512),    # 128 x 256
+    (641, 4200, 1024),   # 128 x 128 in two K groups
+    (300, 4100, 256),    # 64 x 128 in four K groups, one step each
+])
+def test_q6k_tiled_gemm(dev, fmt, m, n, k):
+    import gq
+    import torch
+    w = O.gen_weights(fmt, n, k, seed=m)
+    packed = torch.from_numpy(gq.repack_host(fmt, w, n, k)).to(dev)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dev)
+    ref = _ref(fmt, w, a, n, k)
+    c = gq.gemm(fmt, packed, a, n, k)
+    assert _rel(c, ref) <= TOL
+    cb = gq.gemm(fmt, packed, a, n, k, out_dtype=torch.bfloat16)
+    assert torch.equal(cb, c.bfloat16())
+
+
+@pytest.mark.parametrize("m,n,k", [(49, 33, 4352), (33, 8192, 4352), (130, 8200, 4608), (300, 100, 14336)])
+def test_q6k_matmul_long_k(dev, m, n, k):
+    """K > 4096: the tiled kernel on scratch memory, the 16-row GEMVs under
+    capture; the same within the bound, replayed with eager calls between."""
+    import gq
+    import torch
+    w = O.gen_weights(O.Q6_K, n, k, seed=k)
+    packed = torch.from_numpy(gq.repack_host(O.Q6_K, w, n, k)).to(dev)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dev)
+    ref = _ref(O.Q6_K, w, a, n, k)
+    c = torch.empty(m, n, device=dev)
+    gq.matmul(O.Q6_K, packed, a, n, k, c=c)
+    assert _rel(c, ref) <= TOL
+    g = torch.cuda.CUDAGraph()
+    cg = torch.empty(m, n, device=dev)
+    with torch.cuda.graph(g):
+        gq.matmul(O.Q6_K, packed, a, n, k, c=cg)
+    for _ in range(3):
+        cg.zero_()
+        g.replay()
+        gq.matmul(O.Q6_K, packed, a, n, k, c=c)
+        torch.cuda.synchronize()
+        assert _rel(cg, ref) <= TOL and _rel(c, ref) <= TOL
+
+
+def test_scratch_routes_on_streams(dev):
+    """Calls of four threads on streams of their own: each has its own scratch."""
+    import gq
+    import torch
+    m, n, k = 100, 500, 5120
+    w = O.gen_weights(O.Q6_K, n, k, seed=1)
+    packed = torch.from_numpy(gq.repack_host(O.Q6_K, w, n, k)).to(dev)
+    a = [torch.randn(m, k, generator=torch.Generator().manual_seed(i)).to(dev) for i in range(4)]
+    want = [gq.matmul(O.Q6_K, packed, x, n, k) for x in a]
+    got = [torch.zeros(m, n, device=dev) for _ in a]
+    torch.cuda.synchronize()
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(10):
+                gq.matmul(O.Q6_K, packed, a[i], n, k, c=got[i])
+        s.synchronize()
+
+    th = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert all(np.array_equal(x.cpu().numpy(), y.cpu().numpy()) for x, y in zip(got, want))
