@@ -19,44 +19,112 @@ struct DeviceWorkspace {
 std::mutex g_ws_mutex;
 std::vector<DeviceWorkspace> g_ws;
 std::vector<int> g_cus;
-std::vector<hipMemPool_t> g_pools;
 
-// The current device's scratch pool (made on first use; NULL if that fails).
-hipMemPool_t scratch_pool() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(g_ws_mutex);
-  if ((size_t)dev >= g_pools.size()) g_pools.resize(dev + 1, nullptr);
-  if (!g_pools[dev]) {
-    hipMemPoolProps props = {};
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = dev;
-    hipMemPool_t p = nullptr;
-    if (hipMemPoolCreate(&p, &props) != hipSuccess) return nullptr;
-    uint64_t keep = kGqScratchMax;
-    if (hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
-      (void)hipMemPoolDestroy(p);
-      return nullptr;
-    }
-    g_pools[dev] = p;
-  }
-  return g_pools[dev];
+// Scratch blocks of a device.  A block is one call's from its acquisition to
+// the event recorded behind that call's last kernel; a later call waits for
+// the event on its own stream.  (hipMallocAsync / hipFreeAsync do the same but
+// cost 18 us a call.)
+struct ScratchBlock {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+  hipEvent_t done = nullptr;
+  hipStream_t last = nullptr;
+  bool busy = false;      // between acquisition and release
+  uint64_t used = 0;      // acquisition count at the last use
+};
+constexpr int kScratchBlocks = 4;          // of at most kGqScratchMax bytes each
+constexpr uint64_t kScratchIdle = 4096;    // acquisitions an idle block is kept for
+struct ScratchDevice {
+  ScratchBlock block[kScratchBlocks];
+  uint64_t count = 0;
+};
+std::mutex g_scratch_mutex;
+std::vector<ScratchDevice *> g_scratch;  // (never moved: releases refer to the blocks)
+
+// Event queries and allocations would spoil a capture that another thread has
+// under way in the global mode; in the relaxed mode this thread's do not.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+void scratch_free(ScratchBlock &b) {  // its work has ended
+  (void)hipFree(b.ptr);
+  b.ptr = nullptr;
+  b.bytes = 0;
 }
 }  // namespace
 
 GqScratch::GqScratch(size_t bytes, hipStream_t s) : stream(s) {
-  if (bytes > kGqScratchMax) return;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  hipMemPool_t pool = nullptr;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone || !(pool = scratch_pool()) ||
-      hipMallocFromPoolAsync(&ptr, bytes, pool, s) != hipSuccess) {
-    ptr = nullptr;
+  int dev = 0;
+  if (bytes > kGqScratchMax || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();  // (the caller takes a route without scratch)
+    return;
   }
+  RelaxedCapture relaxed;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  if ((size_t)dev >= g_scratch.size()) g_scratch.resize(dev + 1, nullptr);
+  if (!g_scratch[dev]) g_scratch[dev] = new ScratchDevice;
+  ScratchDevice &d = *g_scratch[dev];
+  ++d.count;
+  auto ended = [](const ScratchBlock &b) { return hipEventQuery(b.done) == hipSuccess; };
+  // the block this stream used last (its work is in order already), else one
+  // whose work has ended, else an empty place, else any that is large enough
+  ScratchBlock *best = nullptr;
+  int rank = 0;
+  for (ScratchBlock &b : d.block) {
+    if (b.busy) continue;
+    int r = 1;  // (a smaller block: replaced)
+    if (!b.ptr) r = 3;
+    else if (d.count - b.used > kScratchIdle && ended(b)) {
+      scratch_free(b);
+      r = 3;
+    } else if (b.bytes >= bytes) r = b.last == s ? 5 : ended(b) ? 4 : 2;
+    if (r > rank) {
+      rank = r;
+      best = &b;
+    }
+  }
+  if (!best) return;
+  if (best->ptr && best->bytes < bytes) {
+    if (hipEventSynchronize(best->done) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    scratch_free(*best);
+  }
+  if (!best->ptr) {
+    const size_t want = (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+    if ((!best->done && hipEventCreateWithFlags(&best->done, hipEventDisableTiming) != hipSuccess) ||
+        hipMalloc(&best->ptr, want) != hipSuccess) {
+      best->ptr = nullptr;
+      (void)hipGetLastError();
+      return;
+    }
+    best->bytes = want;
+  } else if (hipStreamWaitEvent(s, best->done, 0) != hipSuccess) {
+    // (also on the stream that used it last: a stream made anew may have an
+    // old one's handle)
+    (void)hipGetLastError();
+    return;
+  }
+  (void)hipGetLastError();  // (a query of running work)
+  best->busy = true;
+  best->last = s;
+  best->used = d.count;
+  block = best;
+  ptr = best->ptr;
 }
 GqScratch::~GqScratch() {
-  if (ptr) (void)hipFreeAsync(ptr, stream);
+  if (!block) return;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  ScratchBlock &b = *(ScratchBlock *)block;
+  // without the event the block stays out of use
+  if (hipEventRecord(b.done, stream) == hipSuccess) b.busy = false;
+  else (void)hipGetLastError();
 }
 
 int gq_hip_status(hipError_t e) {

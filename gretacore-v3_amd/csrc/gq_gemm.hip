@@ -467,9 +467,16 @@ struct RStep<GQ_FMT_Q6_K, NJ> {
   uint32_t sc[NJ];     // the step's four int8 scales (one per 16 k)
   uint32_t d[NJ];      // the super-block's d (fp16 bits)
 };
+// fp16 weights, row-major N x K (no T16 layout): the fragments as they are, one
+// 16-byte load each.  A wave's load touches 32 rows, 32 bytes of each; the
+// step's four loads together take whole 128-byte lines.
+template <int NJ>
+struct RStep<GQ_FMT_F16, NJ> {
+  gq_u4 q[NJ][4];  // MFMA k-step ks
+};
 // loads of one column block and K step
 template <int FMT>
-constexpr int kRLoads = FMT == GQ_FMT_Q6_K ? 6 : 3;
+constexpr int kRLoads = FMT == GQ_FMT_Q6_K ? 6 : FMT == GQ_FMT_F16 ? 4 : 3;
 
 // Buffer resource over the 4 GiB from p (raw: stride 0, the offset in
 // bytes).  The register-B kernel addresses its operands as a 32-bit per-lane
@@ -495,12 +502,32 @@ GQ_DEV uint32_t ld2_b(const void *base, uint32_t vo, uint32_t so) {
   return __builtin_amdgcn_raw_buffer_load_b16(gq_rsrc(base), vo, so, 0);
 }
 
+// (F16: so[0] is the matrix's size in bytes, K the row length.  The step's
+// halves of 32 k lie wholly inside the row or past it -- K % 32 == 0 -- and those
+// past it are read beyond the resource's range, which gives zeros.)
 template <int FMT, int NJ>
-GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_t (&so)[NJ], int step,
+GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_t (&so)[NJ], int K, int step,
                        RStep<FMT, NJ> &st) {
+  if constexpr (FMT == GQ_FMT_F16) {
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), (short)0, (int)so[0], 0x00020000);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t vo = (int)BK * step + 32 * h < K ? qo[j] : so[0];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, 128u * (uint32_t)step + 64u * h + 16u * e, 0);
+          st.q[j][2 * h + e] = gq_u4{v[0], v[1], v[2], v[3]};
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if constexpr (FMT == GQ_FMT_Q4_0) {
+    if constexpr (FMT == GQ_FMT_F16) {
+    } else if constexpr (FMT == GQ_FMT_Q4_0) {
       const uint32_t b = ((uint32_t)(step >> 1) << 10) + 8u * (uint32_t)(step & 1);
       st.q[j][0] = ld8_b(w, qo[j], b);
       st.q[j][1] = ld8_b(w, qo[j] + 512u, b);
@@ -614,6 +641,8 @@ GQ_DEV void q6k_factors(const RStep<GQ_FMT_Q6_K, NJ> &st, int kh, gq_half2 (&f)[
 template <int FMT, int NJ>
 GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const QKf *qk, const gq_half2 *q6,
                       uint32_t mg) {
+  if constexpr (FMT == GQ_FMT_F16) return __builtin_bit_cast(gq_half8, st.q[j][ks]);
+  else {
   const int h = ks >> 1;
   gq_half2 p[4];
   if constexpr (FMT == GQ_FMT_Q6_K) {
@@ -662,6 +691,7 @@ GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const Q
     o[2 * i + 1] = p[i][1];
   }
   return o;
+  }
 }
 
 // Workgroup tile BM x BN, WM x WN waves; a wave owns (BM / WM) x (BN / WN) of C
@@ -683,7 +713,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KG)
 __attribute__((amdgpu_waves_per_eu(WM * WN * KG / 4, WM * WN * KG / 4)))
 k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__restrict__ a16, int lda,
           void *__restrict__ c, const float *__restrict__ rs, int M, int N, int C, int nsteps, int tiles_m,
-          int gm) {
+          int gm, int sps, int stag) {
   constexpr int KS = BK / 16;
   constexpr int NW = WM * WN, TM = BM / WM / 32, NJ = BN / WN / 32;  // waves per group, MFMA tiles per wave
   static_assert(TM >= 1 && NJ >= 1 && BM % (8 * NW) == 0, "tile shape");
@@ -701,7 +731,11 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     constexpr int v = decltype(b)::value;
     return (v == 0 ? As_0 : v == 1 ? As_1 : v == 2 ? As_2 : As_3) + kg * (BM * BK);
   };
-  const int nl = nsteps / KG;  // this group's steps
+  // this workgroup's K steps: part blockIdx.y of sps steps (all of them where
+  // the grid has one part), its output the part's own M x N
+  const int s0 = (int)blockIdx.y * sps;
+  const int nl = (nsteps - s0 < sps ? nsteps - s0 : sps) / KG;  // this group's steps
+  c = reinterpret_cast<uint8_t *>(c) + (size_t)blockIdx.y * (size_t)M * (size_t)N * (CBF16 ? 2u : 4u);
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
   using B2 = std::integral_constant<int, 2>;
@@ -730,7 +764,11 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     if (t >= ntiles) t = ntiles - 1;  // clamped; those columns are never stored
     const uint32_t tc = (uint32_t)t * (uint32_t)C;
     const uint32_t slot = 16u * (16u * (uint32_t)kh + (uint32_t)r);
-    if constexpr (FMT == GQ_FMT_Q4_0) {
+    if constexpr (FMT == GQ_FMT_F16) {  // (C: the row length, sc_off: the matrix's bytes)
+      const int n = n0 + (BN / WN) * wn + 32 * j + (lane & 31);
+      qo[j] = (uint32_t)(n < N ? n : N - 1) * (2u * (uint32_t)C) + 32u * (uint32_t)kh;
+      so[j] = sc_off;
+    } else if constexpr (FMT == GQ_FMT_Q4_0) {
       qo[j] = (tc << 10) + slot;
       so[j] = sc_off + tc * 128u + 8u * r;
     } else if constexpr (FMT == GQ_FMT_Q8_0) {
@@ -761,7 +799,12 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   const int sw = a_swz(lane & 31);
 
   // the group's l-th step of K
-  auto gstep = [&](int l) { return l * KG + kg; };
+  const int off = stag ? (nt * stag) % nl : 0;  // (where this column tile's walk of K starts)
+  auto gstep = [&](int l) {
+    int i = l + off;
+    i = i < nl ? i : i - nl;
+    return s0 + i * KG + kg;
+  };
   // the group's step l (buffer and register stage l % PD; `step` the K step);
   // steps past the end are skipped by every wave alike
   auto run_step = [&](int l, auto buf_c) {
@@ -796,7 +839,7 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
       }
     }
     // the register stage of this step is free: request step + PD into it
-    load_rstep<FMT, NJ>(w, qo, so, s2, cur);
+    load_rstep<FMT, NJ>(w, qo, so, C, s2, cur);
     // the activation tile and the weights of step + 1 must have landed
     __builtin_amdgcn_s_waitcnt(kWaitPend);
     __syncthreads();
@@ -808,7 +851,7 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     constexpr int i = decltype(b)::value;
     const int st = gstep(i < nl ? i : nl - 1);
     if constexpr (i < PD - 1) load_a_lds_b<BM, NW>(a16, ao, st, wave, As_of(b));
-    load_rstep<FMT, NJ>(w, qo, so, st, wst[i]);
+    load_rstep<FMT, NJ>(w, qo, so, C, st, wst[i]);
   };
   // the tile's row scales, requested before the operands (the oldest load,
   // so the wait below covers it) and kept in LDS for the epilogue, whose
@@ -1108,15 +1151,58 @@ int launch_cfg(const void *packed, const _Float16 *a16, int lda, void *c, const 
   return gq_last_launch();
 }
 
+// Steps per part of a K split, in whole groups of four (the K groups of every
+// shape divide it), and the parts that leaves
+int split_steps(int nsteps, int splits) { return ((nsteps + splits - 1) / splits + 3) & ~3; }
+int split_parts(int nsteps, int splits) {
+  const int sps = split_steps(nsteps, splits);
+  return (nsteps + sps - 1) / sps;
+}
+
+// c[m][n] = rs[m] * (the sum of the K parts' [splits][M][N], in part order)
+__global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ part, const float *__restrict__ rs,
+                                                   float *__restrict__ c, size_t mn, int N, int splits) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= mn) return;
+  if (i + 4 <= mn && (mn & 3) == 0) {
+    gq_f4 v = *reinterpret_cast<const gq_f4 *>(part + i);
+    for (int p = 1; p < splits; ++p) {
+      const gq_f4 t = *reinterpret_cast<const gq_f4 *>(part + (size_t)p * mn + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += t[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] *= rs[(i + e) / (size_t)N];
+    // (c may start at any float)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[i + e] = v[e];
+    return;
+  }
+  for (size_t j = i; j < i + 4 && j < mn; ++j) {
+    float v = part[j];
+    for (int p = 1; p < splits; ++p) v += part[(size_t)p * mn + j];
+    c[j] = v * rs[j / (size_t)N];
+  }
+}
+
 // pd_default: the pipeline depth of the shape (GQ_GEMM_PD=2|3|4 overrides it,
 // for tuning)
+// splits > 1: K in that many parts of whole KG steps (split_steps), c the
+// parts' sums [splits][M][N] in fp32
 template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int KG = 1>
 int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
-              hipStream_t s, int pd_default = 4) {
-  const int C = (int)gq_chunks(FMT, K);
-  const int nsteps = (int)(gq_kpad(FMT, K) / BK);
+              hipStream_t s, int pd_default = 4, int splits = 1) {
+  const int C = FMT == GQ_FMT_F16 ? K : (int)gq_chunks(FMT, K);
+  const uint32_t sc_off = FMT == GQ_FMT_F16 ? (uint32_t)N * (uint32_t)K * 2u : (uint32_t)gq_sc_plane_offset(FMT, N, K);
+  const int nsteps = (int)((FMT == GQ_FMT_F16 ? gq_f16w_kpad(K) : gq_kpad(FMT, K)) / BK);
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   if ((size_t)tiles_m * (size_t)tiles_n > 0x7FFFFFFFu) return GQ_ERR_INVALID_ARGS;  // (one grid dimension)
+  const int sps = splits > 1 ? split_steps(nsteps, splits) : nsteps;
+  // fp16 rows at a power-of-two stride put every workgroup's step on the same
+  // few memory channels: each weight column tile starts its K walk one step
+  // further on (17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
+  // formats, whose tiles are contiguous, gain nothing)
+  const int stag = FMT == GQ_FMT_F16 ? 1 : 0;
   const char *e = getenv("GQ_GEMM_PD");
   const int pd = e ? atoi(e) : pd_default;
   // tile order in groups of 4 M tiles (GQ_GEMM_GM=n overrides, 0: plain
@@ -1125,9 +1211,10 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
   const char *eg = getenv("GQ_GEMM_GM");
   const int gm = eg ? atoi(eg) : 4;
 #define GQ_LAUNCH_RB(PD)                                                                                        \
-  hipLaunchKernelGGL((k_gemm_rb<FMT, CBF16, BM, BN, WM, WN, PD, KG>), dim3((unsigned)(tiles_m * tiles_n)),      \
-                     dim3(64 * WM * WN * KG), 0, s, (const uint8_t *)packed, (uint32_t)gq_sc_plane_offset(FMT, N, K), \
-                     a16, lda, c, rs, M, N, C, nsteps, tiles_m, gm)
+  hipLaunchKernelGGL((k_gemm_rb<FMT, CBF16, BM, BN, WM, WN, PD, KG>),                                           \
+                     dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits),                                     \
+                     dim3(64 * WM * WN * KG), 0, s, (const uint8_t *)packed, sc_off, a16,      \
+                     lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps, stag)
   // the depths whose LDS fits (activation buffers, the K groups' exchange,
   // the row scales); a deeper request falls back to the deepest that fits
   constexpr auto lds = [](int d) { return d * KG * BM * BK * 2 + (KG - 1) * WM * WN * 4096 + BM * 4; };
@@ -1188,7 +1275,7 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
 // tuning through GQ_GEMM_TILE.
 int pick_tile(int fmt, int M, int N, int K) {
   auto wgs = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const int nsteps = (int)(gq_kpad(fmt, K) / BK);
+  const int nsteps = (int)((fmt == GQ_FMT_F16 ? gq_f16w_kpad(K) : gq_kpad(fmt, K)) / BK);
   if (const char *e = getenv("GQ_GEMM_TILE")) {
     const int t = atoi(e);
     // K-group shapes need the K steps to divide among the groups
@@ -1231,17 +1318,48 @@ int launch_fmt(const void *packed, const _Float16 *a16, int lda, void *c, const 
   }
 }
 
-// Q6_K: the shapes pick_tile chooses by itself for whole chunks of 256 k (the
-// step count is then a multiple of 4)
+// Q6_K and fp16 weights: the shapes pick_tile chooses by itself for whole
+// chunks of 256 k (the step count is then a multiple of 4)
 template <int FMT, int CBF16>
 int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
                   hipStream_t s) {
   switch (pick_tile(FMT, M, N, K)) {
-  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 3);
+  // (fp16 weights hold 16 registers a step: depth 2 where the accumulators
+  // leave no room for more)
+  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 3);
   case 13: return launch_rb<FMT, CBF16, 128, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s);
   case 17: return launch_rb<FMT, CBF16, 128, 128, 1, 4, 2>(packed, a16, lda, c, rs, M, N, K, s);
-  default: return launch_rb<FMT, CBF16, 64, 128, 1, 4, 4>(packed, a16, lda, c, rs, M, N, K, s);
+  default:
+    return launch_rb<FMT, CBF16, 64, 128, 1, 4, 4>(packed, a16, lda, c, rs, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4);
   }
+}
+
+// Few workgroups (a short, narrow C over a long K): K in parts over workgroups,
+// each part's sums in fp32 in `part`, added by k_split_sum.  About one
+// workgroup per CU, at least 8 steps a part, and only from 32 steps on: fp16 weights,
+// 64 rows, unsplit / split: 4096 x 14336 174 / 47 us, 4096 x 4096 46 / 24, 300 x 14336
+// 130 / 28; 4096 x 1120 (20 steps) 18.6 / 20.3.
+struct SplitPlan {
+  int bm, splits;  // tile rows (64: 64 x 128 in four K groups; 128: 128 x 128 in two)
+};
+SplitPlan split_plan(int M, int N, int nsteps) {
+  const int bm = M > 64 ? 128 : 64;
+  const long wgs = (long)((M + bm - 1) / bm) * ((N + 127) / 128);
+  long want = nsteps < 32 ? 1 : 256 / wgs;
+  if (want > nsteps / 8) want = nsteps / 8;
+  return SplitPlan{bm, want > 1 ? split_parts(nsteps, (int)want) : 1};
+}
+template <int FMT>
+int launch_split(const void *packed, const _Float16 *a16, int lda, float *c, const float *rs, float *part, SplitPlan p,
+                 int M, int N, int K, hipStream_t s) {
+  if (p.bm == 128)
+    GQ_TRY((launch_rb<FMT, 0, 128, 128, 1, 4, 2>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
+  else
+    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 4>(packed, a16, lda, part, nullptr, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4,
+                                                p.splits)));
+  const size_t mn = (size_t)M * (size_t)N;
+  hipLaunchKernelGGL(k_split_sum, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
+  return gq_last_launch();
 }
 
 template <int FMT>
@@ -1304,14 +1422,42 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
 int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,
                          hipStream_t s) {
   const size_t row = gq_kpad(fmt, K) * 2;
-  GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32) && 256 * row <= kGqScratchMax / 2, GQ_ERR_UNSUPPORTED);
-  const size_t fit = (kGqScratchMax / 2 / row) & ~(size_t)255, mb = M < fit ? M : fit;
+  GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
+  const size_t fit = ((kGqScratchMax - (1 << 20)) / (row + 20)) & ~(size_t)255, mb = M < fit ? M : fit;
   const size_t bytes = gq_gemm_workspace_bytes(fmt, mb, K);
   GqScratch ws(bytes, s);
   GQ_CHECK(ws.ptr, GQ_ERR_WORKSPACE);
   for (size_t m0 = 0; m0 < M; m0 += mb)
     GQ_TRY(gemm_core(fmt, packed, a + m0 * K, GQ_DT_F32, c + m0 * N, GQ_DT_F32, M - m0 < mb ? M - m0 : mb, N, K,
                      ws.ptr, bytes, s));
+  return GQ_OK;
+}
+
+// gq_gemm_f16w's rows beyond the GEMV batches (K % 32 == 0, operands 16-byte
+// aligned): A to fp16 with row scales in a scratch buffer, then the register-B
+// kernel on the fp16 rows of W.  Status as gq_launch_matmul_q6k.
+int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_t N, size_t K, hipStream_t s) {
+  const size_t Kp = gq_f16w_kpad(K), row = Kp * 2;
+  // 32-bit weight offsets, with room for the columns read past a row's end
+  GQ_CHECK(N * K * 2 + row < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
+  const size_t fit = ((kGqScratchMax - (1 << 20)) / (row + 20)) & ~(size_t)255, mb = M < fit ? M : fit;
+  const size_t abytes = gq_align256(mb * row), rbytes = gq_align256((mb + 256) * 4);  // (row scales read by the tile)
+  const SplitPlan sp = split_plan((int)mb, (int)N, (int)(Kp / BK));
+  const size_t pbytes = sp.splits > 1 ? (size_t)sp.splits * M * N * 4 : 0;
+  const bool split = sp.splits > 1 && mb == M && abytes + rbytes + pbytes <= kGqScratchMax;
+  GqScratch ws(abytes + rbytes + (split ? pbytes : 0), s);
+  GQ_CHECK(ws.ptr, GQ_ERR_WORKSPACE);
+  float *rs = (float *)((uint8_t *)ws.ptr + abytes);
+  if (split) {
+    GQ_TRY(launch_a_to_f16(a, GQ_DT_F32, (_Float16 *)ws.ptr, rs, (int)M, (int)K, (int)Kp, 0, s));
+    return launch_split<GQ_FMT_F16>(w, (const _Float16 *)ws.ptr, (int)Kp, c, rs, (float *)((uint8_t *)rs + rbytes), sp,
+                                    (int)M, (int)N, (int)K, s);
+  }
+  for (size_t m0 = 0; m0 < M; m0 += mb) {
+    const int m = (int)(M - m0 < mb ? M - m0 : mb);
+    GQ_TRY(launch_a_to_f16(a + m0 * K, GQ_DT_F32, (_Float16 *)ws.ptr, rs, m, (int)K, (int)Kp, 0, s));
+    GQ_TRY((launch_fmt_kg<GQ_FMT_F16, 0>(w, (const _Float16 *)ws.ptr, (int)Kp, c + m0 * N, rs, m, (int)N, (int)K, s)));
+  }
   return GQ_OK;
 }
 

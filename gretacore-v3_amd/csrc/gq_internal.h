@@ -35,6 +35,8 @@ static inline int gq_check_shape(int fmt, size_t N, size_t K) {
 static inline size_t gq_align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // padded K of the T16 layout
 static inline size_t gq_kpad(int fmt, size_t K) { return gq_chunks(fmt, K) * gq_chunk_k(fmt); }
+// padded K of the tiled GEMM on fp16 weights (four 64-k steps: its K groups)
+static inline size_t gq_f16w_kpad(size_t K) { return (K + 255) & ~(size_t)255; }
 // GEMV workspace (batch > 4): int8 limbs [B][2][Kp] then a zero region of Kp
 // bytes, then per (batch row, 32-block) float4 (s, S, s / 254, 0).
 static inline size_t gq_xl_bytes(int fmt, size_t K, int B) {
@@ -67,13 +69,14 @@ int gq_launch_f16_to_f32(const void *in, size_t n, float *out, hipStream_t s);
 
 // Library-owned per-device workspace (grown on demand, never shrunk).
 int gq_default_workspace(size_t bytes, void **ptr);
-// Scratch memory of one call on stream s, ordered with the stream: from a pool
-// of the current device that keeps at most kGqScratchMax bytes between calls
-// (more goes back to the device as its work ends).  Each call has its own
-// block, so calls on other streams and threads do not meet.  ptr is NULL where
-// no block is to be had: more than kGqScratchMax asked for, no memory left, or
-// a stream under capture (an allocation would become part of the graph).
-constexpr size_t kGqScratchMax = (size_t)256 << 20;
+// Scratch memory of one call on stream s, for the kernels launched on s in this
+// object's lifetime.  The blocks are kept (at most four a device, of up to
+// kGqScratchMax bytes; one that is not asked for any more is freed) and pass
+// from call to call behind events, so calls on other streams and threads do
+// not meet.  ptr is NULL where no block is to be had: more than kGqScratchMax
+// asked for, no memory left, all four between acquisition and release, or a
+// stream under capture (the graph would keep the block's address).
+constexpr size_t kGqScratchMax = (size_t)128 << 20;
 struct GqScratch {
   void *ptr = nullptr;
   GqScratch(size_t bytes, hipStream_t s);
@@ -83,9 +86,12 @@ struct GqScratch {
 
 private:
   hipStream_t stream;
+  void *block = nullptr;
 };
 // Q6_K rows of gq_matmul through the tiled GEMM (gq_gemm.hip)
 int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,
                          hipStream_t s);
+// fp16-weight rows of gq_gemm_f16w through the tiled GEMM (gq_gemm.hip)
+int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_t N, size_t K, hipStream_t s);
 // Compute units of the current device (cached per device; 0 without a device).
 int gq_device_cus(void);

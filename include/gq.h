@@ -228,11 +228,13 @@ int gq_launch_gemm_mfma_int4_wt_fp32_acc32(void *stream, const void *a, const in
  * launch_gemm_mfma_mixed_f16f32 (gemm_kernels.hpp:30-44, gemm_kernels.hip:
  * 294-358, 387-523): C[M][N] = A[M][K] W^T, A fp32, W fp16 row-major N x K
  * (GGUF F16 tensors, e.g. a dequantized lm_head), C fp32.  Here on the fp16
- * matrix cores in batches of up to 16 rows of A (fp32 accumulation; A rounded
+ * matrix cores (fp32 accumulation; A rounded
  * to fp16 after a per-window power-of-two scaling) when K % 32 == 0 and d_w and
  * d_a are 16-byte aligned; any other K or alignment runs a plain fp32-accumulating
- * kernel (fp32 A times the fp16 weight, as the reference's VALU route).  Rows of
- * A beyond 16 take further launches, each streaming W again. */
+ * kernel (fp32 A times the fp16 weight, as the reference's VALU route).  More than
+ * 16 rows run on the tiled GEMM (A scaled by row), with scratch memory of the
+ * call's own; batches of 16 rows, each streaming W again, while the stream is
+ * being captured and where two or three of them over a small W are quicker. */
 int gq_gemm_f16w(const void *d_w, const float *d_a, float *d_c, size_t M, size_t N, size_t K, void *stream);
 /* The two reference launchers under their argument lists; lda must be K and
  * ldc N (what GretaCompute::gemm passes), ldb is ignored as in the reference. */

@@ -1,4 +1,4 @@
-"""Tiled-GEMM routes of Q6_K weights against float64 products of the
+"""Tiled-GEMM routes of Q6_K and fp16 weights against float64 products of the
 dequantized weights (the oracle's), at the edges of each tile shape."""
 import threading
 
@@ -93,3 +93,31 @@ def test_scratch_routes_on_streams(dev):
     for t in th:
         t.join()
     assert all(np.array_equal(x.cpu().numpy(), y.cpu().numpy()) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (4865, 5300, 96),     # 256 x 256 tiles; K past the last whole 64-k step
+    (700, 8300, 160),     # 128 x 256
+    (641, 4200, 1056),    # 128 x 128 in two K groups
+    (300, 4100, 32),      # 64 x 128 in four K groups, K within one step
+    (17, 33, 4128),       # K in parts, 64-row tiles, an odd count of outputs
+    (131, 300, 14304),    # K in parts of unequal length, 128-row tiles
+    (17, 100, 64), (40, 64, 512), (49, 64, 512),  # about the batch GEMVs' limits
+])
+def test_f16w_tiled(dev, m, n, k):
+    """Columns past K hold Inf in the next row's weights: they must not count."""
+    import gq
+    import torch
+    g = torch.Generator().manual_seed(m + k)
+    w = torch.randn(n + 1, k, generator=g).half()
+    w[n] = float("inf")  # (the row after the matrix)
+    w = w.to(dev)
+    a = torch.randn(m, k, generator=g).to(dev)
+    a[m // 2] *= 1e6     # a row beyond fp16's range
+    c = torch.full((m + 1, n), 7.0, device=dev)
+    gq.gemm_f16w(w[:n], a, n, k, c=c[:m])
+    ref = a.double() @ w[:n].double().t()
+    err = (c[:m].double() - ref).norm(dim=1) / ref.norm(dim=1)
+    # one row of n outputs: a little over the bound of a long row
+    assert float(err.max()) <= 2 * TOL and _rel(c[:m], ref) <= TOL
+    assert bool((c[m] == 7.0).all())
