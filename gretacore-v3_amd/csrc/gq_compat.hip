@@ -8,7 +8,8 @@
 // c[m*ldc + n].  Rows of a are lda apart.  M, N or K == 0 returns at once.
 //
 // Up to 32 rows (and with force_gemv) the GEMV in fp32, as the reference's
-// GEMV kernels; above, the reference's MFMA route on fp16 operands through
+// GEMV kernels -- on the VALU for small calls, on the matrix cores with fp32
+// precision (k_compat_mfma) for more; above, the reference's MFMA route on fp16 operands through
 // gq_gemm (compat_gemm_route).
 #include "gq_internal.h"
 
@@ -334,11 +335,416 @@ k_compat_gemv_lds(const TA *__restrict__ a, const uint8_t *__restrict__ b, float
   }
 }
 
+// ---- matrix-core form: 2..32 rows (any count with force_gemv) -----------------
+// A contraction of the integer codes with the fp32 (or fp16) activations that
+// loses nothing to the matrix cores' 16-bit operands: the codes are exact in
+// fp16, and an fp32 activation is split into two fp16 limbs, hi = fp16(x 2^s),
+// lo = fp16(x 2^s - hi) -- 22 bits and sign, s the power of two that brings the
+// largest magnitude of the row's window into [2^14, 2^15) (fp16 activations
+// are one limb, exact).  v_mfma_f32_16x16x32_f16 is one scale group of 32 for 16
+// weight rows and 16 activation rows; both limbs go to one fp32 accumulator,
+// which is scaled by the group's factor and added to the window's sum, that to
+// the total by 2^-s, compensated.  Odd groups hold -x and count with -s: the
+// MFMA's internal sum rounds downwards, a bias that would otherwise add up over
+// K (rel-L2 against float64 1.3e-7 at K = 4096, 1.9e-7 at 14336; alternating 9.1-
+// 9.8e-8, the fp32 VALU kernels 1.1-1.2e-7).  14336 x 4096, INT4 / INT8, 8 rows:
+// 43 / 49 -> 18 / 21 us; 32 rows 157 / 170 -> 32 / 34.
+//
+// Workgroup: TW row tiles of 16 x KS parts of K, one wave each.  The limbs of a
+// window (WIN k of every part) are made once per workgroup in LDS, double-
+// buffered; a wave's 16-byte weight loads (lane (g, r): row r, 16-byte piece g of 64)
+// go out two windows ahead.  A piece is one group's (INT4) or half a group's
+// (INT8) codes of one row, so lane swaps (permlane) turn four pieces into
+// B fragments of one group each; k order inside a group is free as long as the
+// limbs are stored alike.
+template <bool INT4>
+struct CmGroup {  // 128 k of 16 rows: four groups' codes and scales
+  gq_u4 q[INT4 ? 1 : 2];
+  float s;  // lane (g, r): the scale of group g of row r
+};
+
+GQ_DEV uint32_t cm_max_row(uint32_t v) {  // largest of each 16 lanes (DPP; 0 is max's identity)
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));
+}
+// lane groups (g0 g1 g2 g3) of a and b -> a: (a0 a1 b0 b1), b: (a2 a3 b2 b3)
+GQ_DEV void cm_swap32(uint32_t &a, uint32_t &b) {
+  const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = v[0];
+  b = v[1];
+}
+// -> a: (a0 b0 a2 b2), b: (a1 b1 a3 b3)
+GQ_DEV void cm_swap16(uint32_t &a, uint32_t &b) {
+  const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = v[0];
+  b = v[1];
+}
+
+template <bool INT4, typename TA, int MR, int WIN, int TW, int KS>
+__global__ void __launch_bounds__(64 * TW * KS)
+k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__restrict__ c,
+              const float *__restrict__ scales, const float *__restrict__ head_scales, int M, int N, int K, int lda,
+              int ldc, int head_dim, int NI) {
+  // K part blockIdx.z of gridDim.z: its windows, its own M x N of c
+  const int z0 = (K + WIN - 1) / WIN * (int)blockIdx.z / (int)gridDim.z;
+  const int nw = (K + WIN - 1) / WIN * ((int)blockIdx.z + 1) / (int)gridDim.z - z0;
+  c += (size_t)blockIdx.z * (size_t)M * (size_t)ldc;
+  constexpr int L = sizeof(TA) == 4 ? 2 : 1;  // limbs
+  constexpr int NG = WIN / 128;               // 128-k groups per window
+  constexpr int NB = WIN / 32;                // scale groups per window
+  constexpr int RUN = WIN / 8;                // runs of 8 per row and window
+  constexpr int NT = 64 * TW * KS;
+  constexpr int RPT = KS * MR * RUN / NT;     // runs per thread and window
+  constexpr int MT = MR > 16 ? MR / 16 : 1;   // 16-row tiles of activations
+  constexpr int LB = NB * 4 * MR * 16;        // LDS bytes of a limb of a part's window: [NB][4][MR][16]
+  static_assert(RPT >= 1 && RPT * NT == KS * MR * RUN && (RUN == 16 || RUN == 32), "runs divide evenly");
+  __shared__ __attribute__((aligned(16))) unsigned char xs[2][KS][L * LB];
+  __shared__ __attribute__((aligned(16))) float xsc[2][KS * MR];  // 2^-s per part and row
+  static_assert(sizeof(xs) >= (size_t)KS * TW * MT * 64 * 16, "the parts' sums reuse it");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tt = wave % TW, part = wave / TW;
+  const int g = lane >> 4, r = lane & 15;
+  const int m_base = (int)blockIdx.y * MR;
+  const int nb = K / 32;
+  const int w0 = z0 + nw * part / KS, w1 = z0 + nw * (part + 1) / KS;  // this wave's windows (<= NI)
+  const int n = ((int)blockIdx.x * TW + tt) * 16 + r;
+  const int nr = n < N ? n : N - 1;  // (rows past N are computed, never stored)
+  const uint8_t *wrow = b + (size_t)nr * K / (INT4 ? 2 : 1);
+  const float *srow = scales + (size_t)nr * nb;
+
+  // weights and scales of window w; past the row's end another group's are
+  // read instead, with scale 0 (their limbs are zeros too)
+  auto load_win = [&](int w, CmGroup<INT4> (&gr)[NG]) {
+    w = w < w1 ? w : w1 - 1;
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const int b0 = w * NB + 4 * j;
+      if constexpr (INT4) {
+        const int bi = b0 + g < nb ? b0 + g : nb - 1;
+        gr[j].q[0] = gq_ld16(wrow + 16 * (size_t)bi);
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int bi = b0 + 2 * h + (g >> 1) < nb ? b0 + 2 * h + (g >> 1) : nb - 1;
+          gr[j].q[h] = gq_ld16(wrow + 32 * (size_t)bi + 16 * (g & 1));
+        }
+      }
+      const float s = srow[b0 + g < nb ? b0 + g : nb - 1];
+      gr[j].s = b0 + g < nb ? s : 0.f;
+    }
+  };
+  // activations: run u of this thread = (part, row, run of the window)
+  float xv[RPT][8];
+  bool xin[RPT];
+  auto load_x = [&](int it) {
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      const int run = (int)threadIdx.x + u * NT;
+      const int kr = run % RUN, row = (run / RUN) % MR, p = run / (RUN * MR);
+      const int w = z0 + nw * p / KS + it;
+      const int k = w * WIN + 8 * kr;
+      xin[u] = m_base + row < M && w < z0 + nw * (p + 1) / KS && k < K;  // (K % 32 == 0: a run is whole)
+      const TA *src = a + (size_t)(xin[u] ? m_base + row : 0) * lda + (xin[u] ? k : 0);
+      if constexpr (L == 2) {
+        const gq_f4 v0 = *reinterpret_cast<const gq_f4 *>(src), v1 = *reinterpret_cast<const gq_f4 *>(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xv[u][e] = v0[e];
+          xv[u][4 + e] = v1[e];
+        }
+      } else {
+        const gq_half8 v = *reinterpret_cast<const gq_half8 *>(src);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xv[u][e] = (float)v[e];
+      }
+    }
+  };
+  auto store_x = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      const int run = (int)threadIdx.x + u * NT;
+      const int kr = run % RUN, row = (run / RUN) % MR, p = run / (RUN * MR);
+      // the window's largest magnitude (a NaN does not count: its limbs are
+      // NaN whatever the scale)
+      float af = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) af = fmaxf(af, fabsf(xv[u][e]));
+      uint32_t am = cm_max_row(xin[u] ? __float_as_uint(af) : 0u);
+      if constexpr (RUN == 32) {
+        const auto v = __builtin_amdgcn_permlane16_swap(am, am, false, false);
+        am = max(v[0], v[1]);
+      }
+      // 2^s and 2^-s, both normal floats
+      const uint32_t fe = (uint32_t)min(268 - (int)(am >> 23), 253);
+      const float f = __uint_as_float((fe << 23) | ((kr & 4) ? 0x80000000u : 0u)), f16 = f * 0.0625f;  // (odd groups: -x)
+      if (kr == 0) xsc[buf][p * MR + row] = __uint_as_float((254u - fe) << 23);
+      gq_half8 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        // INT4: the code order (gq_nib_halves over plain nibbles), its 16 x
+        // codes against a sixteenth of the activation.  Both limbs are one
+        // mixed-precision fma with one rounding (x f is exact).
+        const int k = INT4 ? (e >> 1) + 4 * (e & 1) : e;
+        const float fs = INT4 && (e & 2) ? f16 : f;
+        hi[e] = (_Float16)fmaf(xv[u][k], fs, -0.f);
+        if constexpr (L == 2) lo[e] = (_Float16)fmaf(xv[u][k], fs, -(float)hi[e]);
+      }
+      if constexpr (L == 2) {
+        // an Inf stays in hi alone: its residual would be NaN
+        if (__any((int)(am == 0x7F800000u))) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (__builtin_isinf((float)hi[e])) lo[e] = (_Float16)0.f;
+        }
+      }
+      const int blk = kr >> 2, unit = kr & 3;
+      const int gq = INT4 ? unit : ((unit & 1) << 1) | (unit >> 1);  // (the INT8 swap's order)
+      unsigned char *d = &xs[buf][p][((blk * 4 + gq) * MR + row) * 16];
+      gq_u4 hv = __builtin_bit_cast(gq_u4, hi);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) hv[e] = xin[u] ? hv[e] : 0u;
+      *reinterpret_cast<gq_u4 *>(d) = hv;
+      if constexpr (L == 2) {
+        gq_u4 lv = __builtin_bit_cast(gq_u4, lo);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lv[e] = xin[u] ? lv[e] : 0u;
+        *reinterpret_cast<gq_u4 *>(d + LB) = lv;
+      }
+    }
+  };
+
+  // (comp: what rounding took from the windows' sum so far)
+  gq_f4 acc[MT], comp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = comp[t] = gq_f4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t mg = gq_nib_magic();
+  auto consume = [&](int it, CmGroup<INT4> (&gr)[NG]) {
+    if (w0 + it >= w1) return;
+    const unsigned char *xb = &xs[it & 1][part][(g * MR + (MR == 8 ? (r & 7) : r)) * 16];
+    gq_f4 wa[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) wa[t] = gq_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      // scales of the four groups, each for every lane group
+      uint32_t sv[4];
+      sv[0] = sv[2] = __float_as_uint(gr[j].s);
+      cm_swap32(sv[0], sv[2]);
+      sv[1] = sv[0];
+      sv[3] = sv[2];
+      cm_swap16(sv[0], sv[1]);
+      cm_swap16(sv[2], sv[3]);
+      uint32_t q[4][2];
+      if constexpr (INT4) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e][0] = gr[j].q[0][e] ^ 0x88888888u;  // code + 8
+        cm_swap32(q[0][0], q[2][0]);
+        cm_swap32(q[1][0], q[3][0]);
+        cm_swap16(q[0][0], q[1][0]);
+        cm_swap16(q[2][0], q[3][0]);
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            q[2 * h][e] = gr[j].q[h][e] ^ 0x80808080u;  // code + 128
+            q[2 * h + 1][e] = gr[j].q[h][2 + e] ^ 0x80808080u;
+            cm_swap32(q[2 * h][e], q[2 * h + 1][e]);
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        gq_half2 p[4];
+        if constexpr (INT4) {
+          gq_nib_halves(q[i][0], mg, p);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            p[e] = p[e] + ((e & 1) ? gq_half2{(_Float16)-1152.f, (_Float16)-1152.f}
+                                   : gq_half2{(_Float16)-1032.f, (_Float16)-1032.f});
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            p[e] = gq_bits_h2(__builtin_amdgcn_perm(0x64646464u, q[i][e >> 1], (e & 1) ? 0x04030402u : 0x04010400u)) +
+                   gq_half2{(_Float16)-1152.f, (_Float16)-1152.f};
+        }
+        gq_half8 bf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bf[e] = p[e >> 1][e & 1];
+        const float s = __uint_as_float(sv[i]);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const unsigned char *x = xb + ((4 * j + i) * 4 * MR + 16 * t) * 16;
+          gq_f4 d = gq_f4{0.f, 0.f, 0.f, 0.f};
+          if constexpr (L == 2) d = gq_mfma16(*reinterpret_cast<const gq_half8 *>(x + LB), bf, d);
+          d = gq_mfma16(*reinterpret_cast<const gq_half8 *>(x), bf, d);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) wa[t][v] = fmaf((i & 1) ? -s : s, d[v], wa[t][v]);
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const gq_f4 us = *reinterpret_cast<const gq_f4 *>(&xsc[it & 1][part * MR + 16 * t + ((4 * g) & (MR - 1) & 15)]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float y = fmaf(wa[t][v], us[v], -comp[t][v]), z = acc[t][v] + y;
+        comp[t][v] = fabsf(z) < __builtin_inff() ? (z - acc[t][v]) - y : 0.f;  // (an Inf stays one)
+        acc[t][v] = z;
+      }
+    }
+  };
+
+  // the weights of the next two windows and the activations of the next one are
+  // requested before a window is consumed; three weight buffers rotate by
+  // unrolling (no load under a branch: surplus ones re-read the last window)
+  CmGroup<INT4> b0[NG], b1[NG], b2[NG];
+  load_x(0);
+  load_win(w0, b0);
+  load_win(w0 + 1, b1);
+  store_x(0);
+  __syncthreads();
+  auto window = [&](int it, CmGroup<INT4> (&cur)[NG], CmGroup<INT4> (&nxt)[NG]) {
+    load_x(it + 1);
+    load_win(w0 + it + 2, nxt);
+    consume(it, cur);
+    store_x((it + 1) & 1);
+    __syncthreads();
+  };
+  for (int it = 0; it < NI; it += 3) {
+    window(it, b0, b2);
+    if (it + 1 >= NI) break;
+    window(it + 1, b1, b0);
+    if (it + 2 >= NI) break;
+    window(it + 2, b2, b1);
+  }
+  // the parts' sums through LDS, added in part order
+  gq_f4 *red = reinterpret_cast<gq_f4 *>(&xs[0][0][0]);  // [KS][TW][MT][64]
+#pragma unroll
+  for (int t = 0; t < MT; ++t) red[((part * TW + tt) * MT + t) * 64 + lane] = acc[t];
+  __syncthreads();
+  if (part != 0 || n >= N) return;
+  const float h = (head_scales && head_dim > 0) ? head_scales[n / head_dim] : 1.0f;
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    gq_f4 sum = acc[t];
+#pragma unroll
+    for (int p = 1; p < KS; ++p) {
+      const gq_f4 v = red[((p * TW + tt) * MT + t) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] += v[e];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * t + 4 * g + v;  // D row (MR = 8: rows 8..15 repeat 0..7)
+      if (row < MR && m_base + row < M) c[(size_t)(m_base + row) * ldc + n] = sum[v] * h;
+    }
+  }
+}
+
+// c = h * (the K parts' sums [parts][M][N] added in part order, compensated)
+__global__ void __launch_bounds__(256) k_cm_sum(const float *__restrict__ part, const float *__restrict__ head_scales,
+                                                float *__restrict__ c, int M, int N, int ldc, int head_dim, int parts) {
+  const int n = (int)blockIdx.x * 256 + (int)threadIdx.x, m = (int)blockIdx.y;
+  if (n >= N) return;
+  const size_t mn = (size_t)M * N, i = (size_t)m * N + n;
+  float sum = part[i], comp = 0.f;
+  for (int p = 1; p < parts; ++p) {
+    const float y = part[p * mn + i] - comp, z = sum + y;
+    comp = fabsf(z) < __builtin_inff() ? (z - sum) - y : 0.f;
+    sum = z;
+  }
+  c[(size_t)m * ldc + n] = sum * ((head_scales && head_dim > 0) ? head_scales[n / head_dim] : 1.0f);
+}
+
+template <typename TA, bool INT4, int MR, int WIN, int TW, int KS>
+int launch_cm(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M, int N,
+              int K, int lda, int ldc, int hd, int kz = 1, float *part = nullptr) {
+  const int nw = (K + WIN - 1) / WIN, nz = (nw + kz - 1) / kz, NI = (nz + KS - 1) / KS;
+  const dim3 grid((unsigned)((gq_tiles(N) + TW - 1) / TW), (unsigned)((M + MR - 1) / MR), (unsigned)kz);
+  hipLaunchKernelGGL((k_compat_mfma<INT4, TA, MR, WIN, TW, KS>), grid, dim3(64 * TW * KS), 0, s, a, b,
+                     kz > 1 ? part : c, sc, kz > 1 ? nullptr : hs, M, N, K, lda, kz > 1 ? N : ldc, hd, NI);
+  if (kz > 1)
+    hipLaunchKernelGGL(k_cm_sum, dim3((unsigned)((N + 255) / 256), (unsigned)M), dim3(256), 0, s, part, hs, c, M, N,
+                       ldc, hd, kz);
+  return gq_last_launch();
+}
+// Whether the matrix-core form takes a shape: where the VALU kernels' time,
+// which grows with M N K, passes the matrix cores' start-up (int4, VALU / matrix
+// cores in us: 2 / 8 / 32 rows of 4096 x 4096 8.3 / 13.7 / 49.8 against 10.9 / 11.3 /
+// 18.6, of 1024 x 4096 8.3 / 8.3 / 13.1 against 11.2 / 11.1 / 17.6, of 4096 x 14336
+// 21.8 / 75 / 284 against 24.0 / 24.5 / 35.6, of 7000 x 1120 8.1 / 15.5 / 50 against
+// 8.3 / 8.3 / 14.4)
+bool cm_takes(int M, int N, int K) {
+  const double mnk = (double)M * N * K;
+  const double from = K <= 2048 ? 40e6 : K <= 4096 && N >= 4096 ? 120e6 : K <= 8192 ? 160e6 : 120e6;
+  return M >= 3 && mnk >= from;  // (two rows are one pass of the VALU kernels: 12.4 against 22.3 us, 20000 x 2048)
+}
+// Row tiles per workgroup and parts of K inside it (TW, KS) as the fp16 batch
+// GEMV's plan; few row tiles on a long K, or more than 16 rows, take K in parts
+// over workgroups as well (kz, sums in scratch): four row tiles then share the
+// activations' limbs, whose reads otherwise outweigh the weights (16 rows of
+// 4096 x 14336 43 -> 26 us, 32 rows of 4096 x 4096 31.6 -> 18.6; 8 rows of 4096 x
+// 4096 11.3 -> 17, so not there).
+template <typename TA, bool INT4, int MR, int WIN>
+int launch_cm_kz(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M, int N,
+                 int K, int lda, int ldc, int hd) {
+  const size_t tiles = gq_tiles(N);
+  const int nw = (K + WIN - 1) / WIN;
+  const long wgs = (long)((tiles + 3) / 4) * ((M + MR - 1) / MR);
+  const int kz = (int)(256 / wgs < nw / 8 ? 256 / wgs : nw / 8);
+  if (tiles >= 800 || kz <= 1 || (MR < 32 && K < 8192)) return GQ_ERR_UNSUPPORTED;
+  GqScratch ws((size_t)kz * M * N * 4, s);
+  if (!ws.ptr) return GQ_ERR_UNSUPPORTED;
+  return launch_cm<TA, INT4, MR, WIN, 4, 4>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd, kz, (float *)ws.ptr);
+}
+template <typename TA, bool INT4, int MR, int WIN>
+int launch_cm_plan(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M,
+                   int N, int K, int lda, int ldc, int hd) {
+  const int r = launch_cm_kz<TA, INT4, MR, WIN>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
+  if (r != GQ_ERR_UNSUPPORTED) return r;
+  const size_t tiles = gq_tiles(N), wgs = (tiles + 3) / 4 * ((M + MR - 1) / MR);
+  const int nw = (K + WIN - 1) / WIN;
+#define GQ_CM(TW, KS) return launch_cm<TA, INT4, MR, WIN, TW, KS>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd)
+  if constexpr (MR == 32) {
+    // (fewer row tiles: 16 rows at a time on smaller workgroups)
+    if (tiles < 400) return launch_cm_plan<TA, INT4, 16, WIN>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
+  }
+  if (MR == 32 || tiles >= 800) {
+    // a 16-wave workgroup fills a CU: beyond one each, 8 waves, two to a CU
+    // (8 rows, INT4: 20000 x 2048 22.5 -> 18.1 us, 28672 x 8192 63.8 -> 56.9)
+    if (nw >= 2 && wgs > 256) GQ_CM(4, 2);
+    if (nw >= 4) GQ_CM(4, 4);
+    GQ_CM(4, 1);
+  }
+  if constexpr (MR < 32) {
+    if (tiles >= 400) {
+      if (nw >= 8) GQ_CM(2, 8);
+      if (nw >= 4) GQ_CM(2, 4);
+      GQ_CM(2, 1);
+    }
+    if (nw >= 8) GQ_CM(1, 8);
+    if (nw >= 4) GQ_CM(1, 4);
+    GQ_CM(1, 1);
+  }
+  return GQ_ERR_INVALID_ARGS;
+#undef GQ_CM
+}
+
 template <typename TA, bool INT4>
 int launch_compat(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M,
                   int N, int K, int lda, int ldc, int gs, int srow, int hd) {
   const bool seg = K % 16 == 0 && (!sc || gs % 16 == 0) && lda % (sizeof(TA) == 4 ? 4 : 8) == 0 &&
                    (uintptr_t)a % 16 == 0 && (uintptr_t)b % 16 == 0;
+  // (K % 32 and groups of 32: the two scale indexings agree and a group is a
+  // row's own)
+  if (seg && sc && gs == 32 && K % 32 == 0 && cm_takes(M, N, K)) {
+    if (M <= 8) return launch_cm_plan<TA, INT4, 8, 256>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
+    if (M <= 16) return launch_cm_plan<TA, INT4, 16, 128>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
+    return launch_cm_plan<TA, INT4, 32, 128>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
+  }
   // activations staged in LDS per 16-row workgroup (K <= 16384), else read
   // per wave (4096 x 4096 M = 1 / 8: 5.9 / 14.2 us against 7.5 / 20)
   if (seg && K <= 16384) {

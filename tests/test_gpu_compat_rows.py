@@ -1,0 +1,104 @@
+"""The INT8 / INT4 GEMV band's matrix-core form against float64 products:
+ragged rows, columns and K, each plan, K in parts, both activation types."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+# fp32 throughout: input limbs 2^-23, sums of a few 2^-24 each
+TOL = 2e-7
+
+
+def _case(int4, m, n, k, seed, f16=False):
+    import torch
+    g = torch.Generator().manual_seed(seed)
+    lo, hi = (-8, 8) if int4 else (-128, 128)
+    q = torch.randint(lo, hi, (n, k), generator=g, dtype=torch.int8)
+    sc = 0.001 + torch.rand(n * k // 32, generator=g)
+    a = torch.randn(m, k, generator=g) * torch.exp(2 * torch.randn(m, 1, generator=g))
+    if f16:
+        a = a.half()
+    hs = 0.5 + torch.rand((n + 6) // 7, generator=g)
+    q, sc, a, hs = (t.cuda() for t in (q, sc, a, hs))
+    w = q.double().reshape(n, k // 32, 32) * sc.double().reshape(n, k // 32, 1)
+    ref = a.double() @ w.reshape(n, k).t()
+    if int4:
+        ref = ref * hs.double()[torch.arange(n, device="cuda") // 7]
+        u = (q & 15).view(torch.uint8)
+        q = u[:, 0::2] | (u[:, 1::2] << 4)
+    return a, q.contiguous(), sc, hs, ref
+
+
+def _run(int4, a, q, sc, hs, m, n, k, c=None, force=False):
+    import gq
+    if int4:
+        return gq.launch_int4_wt(a, q, sc, hs, m, n, k, head_dim=7, force_gemv=force, c=c)
+    return gq.launch_int8_wt(a, q, sc, m, n, k, c=c)
+
+
+def _rel(c, ref):
+    return float((c.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("int4", [True, False])
+@pytest.mark.parametrize("m,n,k", [
+    (2, 14337, 2080),   # four row tiles, the last of one row; K ends inside a window
+    (8, 7001, 800),     # two row tiles; fewer windows than K parts
+    (9, 4100, 1248), (16, 3000, 4128),   # one row tile
+    (3, 3001, 14304),   # K in parts over workgroups
+    (17, 4097, 4096), (32, 1500, 8224),  # 32 rows
+    (31, 14336, 96), (32, 6500, 992),    # K of a few groups
+])
+def test_rows_match_float64(dev, int4, m, n, k):
+    a, q, sc, hs, ref = _case(int4, m, n, k, m + k)
+    assert _rel(_run(int4, a, q, sc, hs, m, n, k), ref) <= TOL
+
+
+def test_fp16_activations_and_force_gemv(dev):
+    m, n, k = 70, 4100, 1056
+    a, q, sc, hs, ref = _case(True, m, n, k, 5, f16=True)
+    assert _rel(_run(True, a, q, sc, hs, m, n, k, force=True), ref) <= TOL
+
+
+@pytest.mark.parametrize("int4", [True, False])
+def test_wide_range_and_nonfinite_rows(dev, int4):
+    """Rows near fp32's ends stay exact to TOL; Inf and NaN stay in their row."""
+    import torch
+    m, n, k = 8, 4112, 4096
+    a, q, sc, hs, _ = _case(int4, m, n, k, 9)
+    a[0] *= 1e30
+    a[1] *= 1e-36
+    a[2, 300:] = 0.0
+    a[3, 77] = float("inf")
+    a[4, 4000] = float("nan")
+    a[5] = 0.0
+    w = (q if not int4 else torch.stack([q & 15, q >> 4], 2).reshape(n, k).to(torch.int16).add_(8).bitwise_and_(15).sub_(8))
+    w = (w.double().reshape(n, k // 32, 32) * sc.double().reshape(n, k // 32, 1)).reshape(n, k)
+    ref = a.double() @ w.t()
+    if int4:
+        ref = ref * hs.double()[torch.arange(n, device="cuda") // 7]
+    c = _run(int4, a, q, sc, hs, m, n, k)
+    for row in (0, 2, 6, 7):
+        assert _rel(c[row], ref[row]) <= TOL, row
+    assert _rel(c[1].double() * 2.0**60, ref[1] * 2.0**60) <= TOL
+    assert bool((c[5] == 0).all())
+    assert bool((torch.isnan(c[3]) == torch.isnan(ref[3])).all()) and bool((torch.isinf(c[3]) == torch.isinf(ref[3])).all())
+    assert bool((c[3][torch.isinf(c[3])] == ref[3][torch.isinf(c[3])].float()).all())
+    assert bool(torch.isnan(c[4]).all())
+
+
+def test_captured_without_scratch(dev):
+    import torch
+    m, n, k = 16, 2000, 14336
+    a, q, sc, hs, ref = _case(True, m, n, k, 11)
+    c = _run(True, a, q, sc, hs, m, n, k)
+    cg = torch.empty_like(c)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        _run(True, a, q, sc, hs, m, n, k, c=cg)
+    for _ in range(3):
+        cg.zero_()
+        g.replay()
+        _run(True, a, q, sc, hs, m, n, k, c=c)
+        torch.cuda.synchronize()
+        assert _rel(cg, ref) <= TOL and _rel(c, ref) <= TOL
+    assert np.isfinite(cg.cpu().numpy()).all()
