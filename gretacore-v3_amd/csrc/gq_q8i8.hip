@@ -5,12 +5,22 @@
 // products (oracle gqo_gemm_q8_i8).
 //
 // Both operands carry a scale per 32-block, so every block of every output
-// costs a conversion, a scale product and an fma after its MFMA (48 VALU
-// instructions per 32 x 32 x 32 MFMA): the route is VALU-bound, not
-// MFMA-bound.  The kernel keeps everything else off the VALU: operands come
-// straight from the T16 tiles and the row-major int8 activations as 16-byte
-// loads issued one block ahead, and the activation scales of a chunk (4
-// blocks) are staged once per workgroup in LDS, four rows per LDS read.
+// costs VALU work after its MFMA: the route is VALU-bound, not MFMA-bound.  Two
+// instructions per output remain (32 per 32 x 32 x 32 MFMA): the MFMA
+// accumulates onto the bits of 1.5 * 2^23, so its int32 result m + p (|p| < 2^20)
+// read as a float is 1.5 * 2^23 + p; fma(d_w, that, -1.5 * 2^23 d_w) is d_w p rounded
+// once (the constant is exact: d_w has 11 bits), and a second fma multiplies by
+// d_a and accumulates.  A conversion, the scale product and an fma (48 per
+// MFMA) took 120 us at 512 x 14336 x 4096 and 88 at 17 x 4096 x 4096, this 108 and
+// 61.  A tile with an infinite weight scale is walked again in the
+// three-instruction form.  The kernel keeps everything else off the VALU, and
+// every latency a step away: operands come straight from the T16 tiles and the
+// row-major int8 activations as 16-byte loads issued two blocks ahead, the
+// activation scales of a chunk (4 blocks) are staged once per workgroup in LDS
+// and read a tile ahead, four rows per LDS read, and a tile's MFMA is issued
+// before the previous tile's VALU work.
+#include <type_traits>
+
 #include "gq_internal.h"
 
 namespace {
@@ -50,7 +60,7 @@ GQ_DEV float q8i8_scale(uint32_t h16) {
 __global__ void __launch_bounds__(kThr, 2)
 k_gemm_q8_i8(const uint8_t *__restrict__ w, uint32_t sc_off, const int8_t *__restrict__ qa,
              const float *__restrict__ da, float *__restrict__ c, int M, int N, int K, int C, int tiles_m) {
-  __shared__ __attribute__((aligned(16))) float ds[2][4][kBM];  // [buffer][block of chunk][row]
+  __shared__ __attribute__((aligned(16))) float ds[4][4][kBM];  // [chunk & 3][block of chunk][row]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -88,13 +98,6 @@ k_gemm_q8_i8(const uint8_t *__restrict__ w, uint32_t sc_off, const int8_t *__res
   };
 
   gq_f16v acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
   // the activation scales of chunk cc (128 rows x 4 blocks): two entries per
   // thread, loaded unconditionally from clamped addresses (a load under a
   // branch would make the compiler wait for every load in flight), zero for
@@ -119,7 +122,7 @@ k_gemm_q8_i8(const uint8_t *__restrict__ w, uint32_t sc_off, const int8_t *__res
     }
   };
 
-  gq_i4 af[2][2], bf[2][2];  // [register stage][tile]
+  gq_i4 af[4][2], bf[4][2];  // [register stage: block & 3][tile]
   auto load_ops = [&](int blk, int st) {
     if (blk >= nb) blk = nb - 1;  // (the padding blocks of the last chunk)
     const uint32_t sa = 32u * (uint32_t)blk, sb = b_off(blk);
@@ -130,53 +133,106 @@ k_gemm_q8_i8(const uint8_t *__restrict__ w, uint32_t sc_off, const int8_t *__res
   };
 
   const int nch = (nb + 3) >> 2;
-  const gq_i16v zero = {};
-  {
-    float v0[2];
-    load_scales(0, v0);
-    store_scales(0, v0);
-  }
-  load_ops(0, 0);
-  for (int cc = 0; cc < nch; ++cc) {
-    const int buf = cc & 1;
-    __syncthreads();  // ds[buf] staged; ds[buf ^ 1] no longer read
-    float vn[2];
-    load_scales(cc + 1 < nch ? cc + 1 : cc, vn);
-    // the 4 block scales of this chunk for each column (block order 0, 2, 1, 3)
-    gq_u2 dwp[2];
+  constexpr int kMagic = 0x4B400000;  // 1.5 * 2^23
+  gq_i16v magic;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) dwp[j] = ld8(w, so[j], 128u * (uint32_t)cc);
+  for (int v = 0; v < 16; ++v) magic[v] = kMagic;
+  // All of K; true if a weight scale of this lane's columns is infinite, where
+  // the fma form gives Inf - Inf: the tile is then walked again in the
+  // three-instruction form (`finite` false).
+  auto walk = [&](auto finite) -> bool {
 #pragma unroll
-    for (int jb = 0; jb < 4; ++jb) {
-      const int st = jb & 1;
-      load_ops(4 * cc + jb + 1, st ^ 1);
-      float dw[2];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint32_t wd = dwp[j][jb & 1];
-        dw[j] = q8i8_scale((jb >> 1) ? (wd >> 16) : wd);
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    bool inf = false;
+    // the 4 block scales of a chunk for each column (block order 0, 2, 1, 3)
+    gq_u2 dwp[2], dwn[2];
+    auto load_dw = [&](int cc, gq_u2 (&d)[2]) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d[j] = ld8(w, so[j], 128u * (uint32_t)(cc < nch ? cc : nch - 1));
+    };
+    // rows 8 q + 4 hl + e (e = 0..3) of MFMA tile row i, block jb: four runs of four
+    auto read_da = [&](int buf, int jb, int i, float (&d)[16]) {
+      const float *dr = &ds[buf][jb][64 * wm + 32 * i + 4 * hl];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const gq_f4 t = *reinterpret_cast<const gq_f4 *>(dr + 8 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
       }
+    };
+    __syncthreads();  // (a second walk: the first one's reads have ended)
+    {
+      float v0[2];
+      load_scales(0, v0);
+      store_scales(0, v0);
+    }
+    load_dw(0, dwp);
+    load_ops(0, 0);
+    load_ops(1, 1);
+    // Everything a tile needs is one step ahead: its product is issued, and its
+    // activation scales are read from LDS, before the previous tile's VALU work
+    // (16 tiles per chunk: t = 4 block + 2 i + j); weight scales a chunk ahead
+    auto product = [&](int st, int i, int j) {
+      return __builtin_amdgcn_mfma_i32_32x32x32_i8(af[st][i], bf[st][j], magic, 0, 0, 0);
+    };
+    gq_i16v D = product(0, 0, 0);
+    __syncthreads();  // ds[0] staged
+    float dav[2][16];
+    read_da(0, 0, 0, dav[0]);
+    for (int cc = 0; cc < nch; ++cc) {
+      const int buf = cc & 3, nbuf = (cc + 1) & 3;
+      float vn[2];
+      load_scales(cc + 1 < nch ? cc + 1 : cc, vn);
+      load_dw(cc + 1, dwn);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        // rows 8 q + 4 hl + e (e = 0..3) of MFMA tile i: four runs of four
-        const float *dr = &ds[buf][jb][64 * wm + 32 * i + 4 * hl];
-        float dav[16];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const gq_f4 t = *reinterpret_cast<const gq_f4 *>(dr + 8 * q);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dav[4 * q + e] = t[e];
-        }
+      for (int jb = 0; jb < 4; ++jb) {
+        load_ops(4 * cc + jb + 2, (jb + 2) & 3);
+        float dw[2], dm[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const gq_i16v D = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[st][i], bf[st][j], zero, 0, 0, 0);
+          const uint32_t wd = dwp[j][jb & 1];
+          dw[j] = q8i8_scale((jb >> 1) ? (wd >> 16) : wd);
+          dm[j] = dw[j] * -12582912.0f;
+          inf |= __builtin_isinf(dw[j]);
+        }
+        // the next chunk's activation scales: stored (a buffer whose readers,
+        // two chunks back, have passed a barrier since) and made visible a
+        // block before their first use
+        if (jb == 2) {
+          store_scales(nbuf, vn);
+          __syncthreads();
+        }
 #pragma unroll
-          for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(dav[v] * dw[j], (float)D[v], acc[i][j][v]);
+        for (int i = 0; i < 2; ++i) {
+          if (i == 0) read_da(buf, jb, 1, dav[1]);
+          else if (jb < 3) read_da(buf, jb + 1, 0, dav[0]);
+          else read_da(nbuf, 0, 0, dav[0]);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int t = 2 * i + j + 1;  // (the last tile's successor: the next block's first)
+            const gq_i16v next = t < 4 ? product(jb, t >> 1, t & 1) : product((jb + 1) & 3, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              if constexpr (decltype(finite)::value)
+                acc[i][j][v] = fmaf(dav[i][v], fmaf(dw[j], __int_as_float(D[v]), dm[j]), acc[i][j][v]);
+              else
+                acc[i][j][v] = fmaf(dav[i][v] * dw[j], (float)(D[v] - kMagic), acc[i][j][v]);
+            }
+            D = next;
+          }
         }
       }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dwp[j] = dwn[j];
     }
-    store_scales(buf ^ 1, vn);
-  }
+    return inf;
+  };
+  if (__syncthreads_or((int)walk(std::true_type{}))) walk(std::false_type{});
 
 #pragma unroll
   for (int j = 0; j < 2; ++j) {

@@ -1,4 +1,4 @@
-"""Tiled-GEMM routes of Q6_K and fp16 weights against float64 products of the
+"""Tiled-GEMM routes of Q6_K and fp16 weights (and int8 x int8) against float64 products of the
 dequantized weights (the oracle's), at the edges of each tile shape."""
 import threading
 
@@ -121,3 +121,30 @@ def test_f16w_tiled(dev, m, n, k):
     # one row of n outputs: a little over the bound of a long row
     assert float(err.max()) <= 2 * TOL and _rel(c[:m], ref) <= TOL
     assert bool((c[m] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (130, 140, 96), (129, 257, 4128), (260, 100, 1056)])
+@pytest.mark.parametrize("inf", [False, True])
+def test_q8_i8_scales(dev, m, n, k, inf):
+    """Exact integer sums under fp32 scales; with infinite weight scales the
+    tile takes the form that keeps them infinite (NaN where the sum is 0)."""
+    import gq
+    import torch
+    w = O.gen_weights(O.Q8_0, n, k, seed=k).reshape(-1, 34)
+    if inf:
+        w[(n - 1) * (k // 32), 0:2] = (0x00, 0x7C)  # +Inf, the last row's first block
+        w[0, 0:2] = (0x00, 0xFC)                    # -Inf, row 0
+        w[0, 2:] = 0
+    qa, da = gq.quantize_act_q8(torch.randn(m, k, generator=torch.Generator().manual_seed(k)).to(dev))
+    packed = torch.from_numpy(gq.repack_host(O.Q8_0, w.ravel(), n, k)).to(dev)
+    c = gq.gemm_q8_i8(packed, qa, da, n).double().cpu().numpy()
+    q = w[:, 2:].view(np.int8).astype(np.float64).reshape(n, k // 32, 32)
+    d = w[:, :2].copy().view(np.float16).astype(np.float64).reshape(n, k // 32)
+    p = np.einsum("mbe,nbe->mnb", qa.cpu().numpy().astype(np.float64).reshape(m, k // 32, 32), q)
+    with np.errstate(invalid="ignore"):
+        ref = (p * d[None] * da.cpu().numpy().astype(np.float64)[:, None]).sum(2)
+    assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isinf(c), np.isinf(ref))
+    assert np.array_equal(c[np.isinf(c)], ref[np.isinf(ref)])
+    ok = np.isfinite(ref)
+    # two roundings per block and one per sum, K / 32 blocks: under 2e-6
+    assert np.linalg.norm(c[ok] - ref[ok]) <= 2e-6 * np.linalg.norm(ref[ok])
