@@ -59,6 +59,7 @@ void scratch_free(ScratchBlock &b) {  // its work has ended
 GqScratch::GqScratch(size_t bytes, hipStream_t s) : stream(s) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   int dev = 0;
+  if (bytes == 0) return;
   if (bytes > kGqScratchMax || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
       hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();  // (the caller takes a route without scratch)

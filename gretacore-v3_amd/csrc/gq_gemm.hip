@@ -1160,8 +1160,14 @@ int split_parts(int nsteps, int splits) {
 }
 
 // c[m][n] = rs[m] * (the sum of the K parts' [splits][M][N], in part order)
+template <int CBF16>
 __global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ part, const float *__restrict__ rs,
-                                                   float *__restrict__ c, size_t mn, int N, int splits) {
+                                                   void *__restrict__ c, size_t mn, int N, int splits) {
+  auto put = [&](size_t j, float v) {
+    if (rs) v *= rs[j / (size_t)N];
+    if constexpr (CBF16) reinterpret_cast<uint16_t *>(c)[j] = f32_to_bf16_rne(v);
+    else reinterpret_cast<float *>(c)[j] = v;
+  };
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= mn) return;
   if (i + 4 <= mn && (mn & 3) == 0) {
@@ -1171,17 +1177,15 @@ __global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ par
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] += t[e];
     }
+    // (c may start at any element)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] *= rs[(i + e) / (size_t)N];
-    // (c may start at any float)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c[i + e] = v[e];
+    for (int e = 0; e < 4; ++e) put(i + e, v[e]);
     return;
   }
   for (size_t j = i; j < i + 4 && j < mn; ++j) {
     float v = part[j];
     for (int p = 1; p < splits; ++p) v += part[(size_t)p * mn + j];
-    c[j] = v * rs[j / (size_t)N];
+    put(j, v);
   }
 }
 
@@ -1358,7 +1362,40 @@ int launch_split(const void *packed, const _Float16 *a16, int lda, float *c, con
     GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 4>(packed, a16, lda, part, nullptr, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4,
                                                 p.splits)));
   const size_t mn = (size_t)M * (size_t)N;
-  hipLaunchKernelGGL(k_split_sum, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
+  hipLaunchKernelGGL(k_split_sum<0>, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
+  return gq_last_launch();
+}
+
+// The T16 formats' K split (64 x 128 tiles in four K groups): a K past 8192 and
+// under half a workgroup per CU, each of which would walk it alone.  Fewer steps
+// or more workgroups gain nothing over pick_tile's shapes, up to 32 rows nothing
+// over the skinny kernel where it takes them (Q4_K, without / with: 64 x 4096 x 14336
+// 58 / 28 us, 128 x 4096 52 / 34, 200 x 300 x 8960 34 / 22; 17 x 4096 x 14336 22.7 /
+// 25.7, 200 x 4096 x 8192 34 / 36, 64 x 4096 x 4096 15 / 21; Q8_0 17 x 4096 x 14336
+// 47 / 27).  1: no split.
+int gemm_splits(int fmt, size_t M, size_t N, size_t K) {
+  const size_t nsteps = gq_kpad(fmt, K) / BK, wgs = ((M + 63) / 64) * ((N + 127) / 128);
+  int ct, nck;
+  if (nsteps <= 128 || nsteps % 4 || wgs >= 128 || M * nsteps * (2 * BK) >= ((size_t)1 << 32) || getenv("GQ_GEMM_TILE") ||
+      (M <= 32 && gq_gemm_skinny_plan(fmt, M, N, K, &ct, &nck) == GQ_OK))
+    return 1;
+  const size_t want = 256 / wgs < nsteps / 16 ? 256 / wgs : nsteps / 16;
+  return split_parts((int)nsteps, (int)want);
+}
+int launch_gemm_split(int fmt, const void *packed, const _Float16 *a16, int lda, void *c, int c_dtype, const float *rs,
+                      float *part, int splits, int M, int N, int K, hipStream_t s) {
+#define GQ_PARTS(F) launch_rb<F, 0, 64, 128, 1, 4, 4>(packed, a16, lda, part, nullptr, M, N, K, s, 4, splits)
+  if (fmt == GQ_FMT_Q4_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q4_0));
+  else if (fmt == GQ_FMT_Q8_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q8_0));
+  else if (gq_fmt_is_q6k(fmt)) GQ_TRY(GQ_PARTS(GQ_FMT_Q6_K));
+  else GQ_TRY(GQ_PARTS(GQ_FMT_Q4_K));
+#undef GQ_PARTS
+  const size_t mn = (size_t)M * (size_t)N;
+  const dim3 grid((unsigned)((mn + 1023) / 1024));
+  if (c_dtype == GQ_DT_BF16)
+    hipLaunchKernelGGL(k_split_sum<1>, grid, dim3(256), 0, s, part, rs, c, mn, N, splits);
+  else
+    hipLaunchKernelGGL(k_split_sum<0>, grid, dim3(256), 0, s, part, rs, c, mn, N, splits);
   return gq_last_launch();
 }
 
@@ -1396,12 +1433,11 @@ static bool gemm_converts_a(int fmt, size_t M, size_t N, size_t K, int a_dtype) 
 }
 
 static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
-                     size_t K, void *ws, size_t ws_bytes, hipStream_t s);
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed = false);
 
-extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M,
-                       size_t N, size_t K, void *ws, size_t ws_bytes, void *stream) {
+static int gemm_checked(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M,
+                        size_t N, size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed) {
   GQ_TRY(gq_check_shape(fmt, N, K));
-
   GQ_CHECK(M <= GQ_MAX_DIM, GQ_ERR_INVALID_ARGS);
   GQ_CHECK(a_dtype == GQ_DT_F32 || a_dtype == GQ_DT_F16 || a_dtype == GQ_DT_BF16, GQ_ERR_UNSUPPORTED);
   GQ_CHECK(c_dtype == GQ_DT_F32 || c_dtype == GQ_DT_BF16, GQ_ERR_UNSUPPORTED);
@@ -1412,7 +1448,12 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
   GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32), GQ_ERR_INVALID_ARGS);
   // Q6_K: K <= 4096 (gq_matmul takes any K)
   GQ_CHECK(!gq_fmt_is_q6k(fmt) || K <= 4096, GQ_ERR_UNSUPPORTED);
-  return gemm_core(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ws, ws_bytes, (hipStream_t)stream);
+  return gemm_core(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ws, ws_bytes, s, fixed);
+}
+
+extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M,
+                       size_t N, size_t K, void *ws, size_t ws_bytes, void *stream) {
+  return gemm_checked(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ws, ws_bytes, (hipStream_t)stream, false);
 }
 
 // gq_matmul's Q6_K rows beyond the GEMV batches, any K: blocks of rows whose
@@ -1461,8 +1502,34 @@ int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_
   return GQ_OK;
 }
 
+// fixed: ws holds all memory there is (the K parts' sums go behind the
+// conversion); otherwise the sums take a scratch block, and there is no split
+// without one.
 static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
-                     size_t K, void *ws, size_t ws_bytes, hipStream_t s) {
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed) {
+  const int splits = gemm_splits(fmt, M, N, K);
+  if (splits > 1) {
+    const size_t Kp = gq_kpad(fmt, K), conv = gq_gemm_workspace_bytes(fmt, M, K), pbytes = (size_t)splits * M * N * 4;
+    GqScratch sc(fixed ? 0 : pbytes, s);
+    float *part = fixed ? (conv + pbytes <= ws_bytes ? (float *)((uint8_t *)ws + conv) : nullptr) : (float *)sc.ptr;
+    if (part) {
+      const int q4 = fmt == GQ_FMT_Q4_0 || gq_fmt_is_q4k(fmt);
+      const _Float16 *a16 = (const _Float16 *)a;
+      const float *rs = nullptr;
+      if (a_dtype != GQ_DT_F16 || Kp != K || q4 || gq_fmt_is_q6k(fmt)) {
+        if (!ws) {
+          GQ_TRY(gq_default_workspace(conv, &ws));
+          ws_bytes = conv;
+        }
+        GQ_CHECK(ws_bytes >= conv, GQ_ERR_WORKSPACE);
+        float *rsw = (float *)((uint8_t *)ws + gq_align256(M * Kp * 2));
+        GQ_TRY(launch_a_to_f16(a, a_dtype, (_Float16 *)ws, rsw, (int)M, (int)K, (int)Kp, q4, s));
+        a16 = (const _Float16 *)ws;
+        rs = rsw;
+      }
+      return launch_gemm_split(fmt, packed, a16, (int)Kp, c, c_dtype, rs, part, splits, (int)M, (int)N, (int)K, s);
+    }
+  }
   // Few rows: the tiled GEMM gives N / 64 .. N / 128 workgroups, each walking
   // all of K (37-55 us at 4096 x 4096 or 14336 x 4096 for any M <= 256); the
   // skinny kernel takes the shapes gq_gemm_skinny_plan accepts (4096 x 4096:
@@ -1559,5 +1626,5 @@ extern "C" int gq_gemm_static(int fmt, const void *packed, const void *a, int a_
     }
     ptr = g_scratch_ptr[dev];
   }
-  return gq_gemm(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ptr, kGemmScratchBytes, stream);
+  return gemm_checked(fmt, packed, a, a_dtype, c, c_dtype, M, N, K, ptr, kGemmScratchBytes, (hipStream_t)stream, true);
 }

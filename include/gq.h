@@ -179,7 +179,9 @@ int gq_gemv_swiglu_plan(int fmt, size_t N, size_t K, int batch, int *ksplit, int
  * (M <= 256 where the grid stays within one workgroup per CU, or two for K
  * beyond 4096) run on a skinny kernel that splits K over the waves of a
  * workgroup; small tiled grids split K over 2 or 4 wave groups of a
- * workgroup. */
+ * workgroup, and few tiles on a K of 8192 or more over workgroups as well (the
+ * parts' fp32 sums in scratch memory of the call's own; not while the stream is
+ * being captured, where the sums round in another order). */
 size_t gq_gemm_workspace_bytes(int fmt, size_t M, size_t K);
 int gq_gemm(int fmt, const void *d_packed, const void *d_a, int a_dtype, void *d_c, int c_dtype, size_t M,
             size_t N, size_t K, void *d_workspace, size_t workspace_bytes, void *stream);

@@ -148,3 +148,47 @@ def test_q8_i8_scales(dev, m, n, k, inf):
     ok = np.isfinite(ref)
     # two roundings per block and one per sum, K / 32 blocks: under 2e-6
     assert np.linalg.norm(c[ok] - ref[ok]) <= 2e-6 * np.linalg.norm(ref[ok])
+
+
+@pytest.mark.parametrize("fmt", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("m,n,k,adt,odt", [
+    (33, 130, 8448, "float32", "float32"),
+    (64, 4096, 14336, "bfloat16", "bfloat16"),
+    (301, 333, 9216, "float32", "float32"),      # an odd count of outputs, parts of unequal length
+    (129, 1000, 16384, "float16", "float32"),
+])
+def test_gemm_k_parts(dev, fmt, m, n, k, adt, odt):
+    """K over workgroups: gq_gemm with a workspace, gq_gemm_static's own memory
+    (the same sums), and the unsplit form under capture."""
+    import ctypes
+
+    import gq
+    import torch
+    adt, odt = getattr(torch, adt), getattr(torch, odt)
+    w = O.gen_weights(fmt, n, k, seed=m)
+    packed = torch.from_numpy(gq.repack_host(fmt, w, n, k)).to(dev)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(adt).to(dev)
+    ref = _ref(fmt, w, a, n, k)
+    tol = TOL if odt == torch.float32 else 4e-3  # (one rounding to bf16: 2^-9)
+    if fmt == O.Q6_K:
+        c = gq.matmul(fmt, packed, a.float(), n, k)
+        assert _rel(c, ref) <= TOL
+        return
+    c = gq.gemm(fmt, packed, a, n, k, out_dtype=odt, workspace=gq.Workspace(dev))
+    assert _rel(c, ref) <= tol
+    cs = torch.empty_like(c)
+    dt = {torch.bfloat16: gq.DT_BF16, torch.float16: gq.DT_F16, torch.float32: gq.DT_F32}
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    st = gq.load().gq_gemm_static(fmt, p(packed), p(a), dt[adt], p(cs), dt[odt], m, n, k,
+                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0 and torch.equal(c, cs)
+    ws, cg = gq.Workspace(dev, gq.gemm_workspace_bytes(fmt, m, k)), torch.empty_like(c)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gq.gemm(fmt, packed, a, n, k, out_dtype=odt, c=cg, workspace=ws)
+    for _ in range(3):
+        cg.zero_()
+        g.replay()
+        gq.gemm(fmt, packed, a, n, k, out_dtype=odt, c=c, workspace=ws)
+        torch.cuda.synchronize()
+        assert _rel(cg, ref) <= tol and _rel(c, ref) <= tol
