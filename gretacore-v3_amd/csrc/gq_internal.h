@@ -48,6 +48,10 @@ static inline size_t gq_scl_bytes(int fmt, size_t K, int B) {
 
 // Zero-fills n floats with a kernel (no memset node, so it is safe to capture).
 int gq_fill_zero(float *p, size_t n, hipStream_t s);
+// INT8 / INT4 rows (K % 32 == 0, gs % 32 == 0) -> T16 Q8_0 / Q4_0, d = fp16(scale *
+// head factor); scales and head_scales may be NULL (1.0)
+int gq_launch_rows_to_t16(bool int4, const void *b, const float *scales, const float *head_scales, int N, int K, int gs,
+                          int head_dim, void *packed, hipStream_t s);
 int gq_launch_prep_x(int fmt, const float *x, void *ws, int B, int K, hipStream_t s);
 
 // fp16 batch GEMV (gq_gemv_h.hip)

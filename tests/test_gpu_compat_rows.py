@@ -102,3 +102,13 @@ def test_captured_without_scratch(dev):
         torch.cuda.synchronize()
         assert _rel(cg, ref) <= TOL and _rel(c, ref) <= TOL
     assert np.isfinite(cg.cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("int4", [True, False])
+@pytest.mark.parametrize("n,k", [(33, 32), (130, 1024), (100, 1056), (257, 544), (16, 2080)])
+def test_mfma_route_conversion(dev, int4, n, k):
+    """M > 32: rows converted to the tiled layout at the edges of a workgroup's
+    512 bytes of a row and of its 16 rows.  A and w s rounded to fp16 once each:
+    about 3.5e-4 (of the scale to fp16 as well)."""
+    a, q, sc, hs, ref = _case(int4, 40, n, k, n + k)
+    assert _rel(_run(int4, a, q, sc, hs, 40, n, k), ref) <= 1e-3
