@@ -708,12 +708,15 @@ GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const Q
 // 0 stores).  Grids with one workgroup per CU (M = 512) otherwise run one
 // wave per SIMD, each waiting out its loads' latency; KG groups put KG waves
 // on every SIMD with no partial sums leaving the CU.  nsteps % KG == 0.
-template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int PD = 2, int KG = 1>
+// SP: K in parts over workgroups (blockIdx.y); a template parameter, like the
+// staggered walk, because the extra scalar work per step costs the other grids
+// 2-3 % (1024 x 14336 x 4096).
+template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int PD = 2, int KG = 1, bool SP = false>
 __global__ void __launch_bounds__(64 * WM * WN * KG)
 __attribute__((amdgpu_waves_per_eu(WM * WN * KG / 4, WM * WN * KG / 4)))
 k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__restrict__ a16, int lda,
           void *__restrict__ c, const float *__restrict__ rs, int M, int N, int C, int nsteps, int tiles_m,
-          int gm, int sps, int stag) {
+          int gm, int sps) {
   constexpr int KS = BK / 16;
   constexpr int NW = WM * WN, TM = BM / WM / 32, NJ = BN / WN / 32;  // waves per group, MFMA tiles per wave
   static_assert(TM >= 1 && NJ >= 1 && BM % (8 * NW) == 0, "tile shape");
@@ -731,11 +734,12 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     constexpr int v = decltype(b)::value;
     return (v == 0 ? As_0 : v == 1 ? As_1 : v == 2 ? As_2 : As_3) + kg * (BM * BK);
   };
-  // this workgroup's K steps: part blockIdx.y of sps steps (all of them where
-  // the grid has one part), its output the part's own M x N
-  const int s0 = (int)blockIdx.y * sps;
-  const int nl = (nsteps - s0 < sps ? nsteps - s0 : sps) / KG;  // this group's steps
-  c = reinterpret_cast<uint8_t *>(c) + (size_t)blockIdx.y * (size_t)M * (size_t)N * (CBF16 ? 2u : 4u);
+  // this workgroup's K steps: part blockIdx.y of sps steps, its output the
+  // part's own M x N (all of K where there are no parts)
+  const int s0 = SP ? (int)blockIdx.y * sps : 0;
+  const int nl = (SP ? (nsteps - s0 < sps ? nsteps - s0 : sps) : nsteps) / KG;  // this group's steps
+  if constexpr (SP)
+    c = reinterpret_cast<uint8_t *>(c) + (size_t)blockIdx.y * (size_t)M * (size_t)N * (CBF16 ? 2u : 4u);
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
   using B2 = std::integral_constant<int, 2>;
@@ -799,11 +803,17 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   const int sw = a_swz(lane & 31);
 
   // the group's l-th step of K
-  const int off = stag ? (nt * stag) % nl : 0;  // (where this column tile's walk of K starts)
+  // fp16 rows at a power-of-two stride put every workgroup's step on the same
+  // few memory channels: each weight column tile starts its walk one step
+  // further on (17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
+  // formats, whose tiles are contiguous, gain nothing)
+  const int off = FMT == GQ_FMT_F16 ? nt % nl : 0;
   auto gstep = [&](int l) {
-    int i = l + off;
-    i = i < nl ? i : i - nl;
-    return s0 + i * KG + kg;
+    if constexpr (FMT == GQ_FMT_F16) {
+      l += off;
+      l = l < nl ? l : l - nl;
+    }
+    return s0 + l * KG + kg;
   };
   // the group's step l (buffer and register stage l % PD; `step` the K step);
   // steps past the end are skipped by every wave alike
@@ -1191,9 +1201,9 @@ __global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ par
 
 // pd_default: the pipeline depth of the shape (GQ_GEMM_PD=2|3|4 overrides it,
 // for tuning)
-// splits > 1: K in that many parts of whole KG steps (split_steps), c the
+// SP: K in `splits` parts of whole KG steps (split_steps), c the
 // parts' sums [splits][M][N] in fp32
-template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int KG = 1>
+template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int KG = 1, bool SP = false>
 int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
               hipStream_t s, int pd_default = 4, int splits = 1) {
   const int C = FMT == GQ_FMT_F16 ? K : (int)gq_chunks(FMT, K);
@@ -1201,12 +1211,7 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
   const int nsteps = (int)((FMT == GQ_FMT_F16 ? gq_f16w_kpad(K) : gq_kpad(FMT, K)) / BK);
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   if ((size_t)tiles_m * (size_t)tiles_n > 0x7FFFFFFFu) return GQ_ERR_INVALID_ARGS;  // (one grid dimension)
-  const int sps = splits > 1 ? split_steps(nsteps, splits) : nsteps;
-  // fp16 rows at a power-of-two stride put every workgroup's step on the same
-  // few memory channels: each weight column tile starts its K walk one step
-  // further on (17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
-  // formats, whose tiles are contiguous, gain nothing)
-  const int stag = FMT == GQ_FMT_F16 ? 1 : 0;
+  const int sps = SP ? split_steps(nsteps, splits) : nsteps;
   const char *e = getenv("GQ_GEMM_PD");
   const int pd = e ? atoi(e) : pd_default;
   // tile order in groups of 4 M tiles (GQ_GEMM_GM=n overrides, 0: plain
@@ -1215,10 +1220,10 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
   const char *eg = getenv("GQ_GEMM_GM");
   const int gm = eg ? atoi(eg) : 4;
 #define GQ_LAUNCH_RB(PD)                                                                                        \
-  hipLaunchKernelGGL((k_gemm_rb<FMT, CBF16, BM, BN, WM, WN, PD, KG>),                                           \
+  hipLaunchKernelGGL((k_gemm_rb<FMT, CBF16, BM, BN, WM, WN, PD, KG, SP>),                                           \
                      dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits),                                     \
                      dim3(64 * WM * WN * KG), 0, s, (const uint8_t *)packed, sc_off, a16,      \
-                     lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps, stag)
+                     lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps)
   // the depths whose LDS fits (activation buffers, the K groups' exchange,
   // the row scales); a deeper request falls back to the deepest that fits
   constexpr auto lds = [](int d) { return d * KG * BM * BK * 2 + (KG - 1) * WM * WN * 4096 + BM * 4; };
@@ -1357,9 +1362,9 @@ template <int FMT>
 int launch_split(const void *packed, const _Float16 *a16, int lda, float *c, const float *rs, float *part, SplitPlan p,
                  int M, int N, int K, hipStream_t s) {
   if (p.bm == 128)
-    GQ_TRY((launch_rb<FMT, 0, 128, 128, 1, 4, 2>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
+    GQ_TRY((launch_rb<FMT, 0, 128, 128, 1, 4, 2, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
   else
-    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 4>(packed, a16, lda, part, nullptr, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4,
+    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 4, true>(packed, a16, lda, part, nullptr, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4,
                                                 p.splits)));
   const size_t mn = (size_t)M * (size_t)N;
   hipLaunchKernelGGL(k_split_sum<0>, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
@@ -1384,7 +1389,7 @@ int gemm_splits(int fmt, size_t M, size_t N, size_t K) {
 }
 int launch_gemm_split(int fmt, const void *packed, const _Float16 *a16, int lda, void *c, int c_dtype, const float *rs,
                       float *part, int splits, int M, int N, int K, hipStream_t s) {
-#define GQ_PARTS(F) launch_rb<F, 0, 64, 128, 1, 4, 4>(packed, a16, lda, part, nullptr, M, N, K, s, 4, splits)
+#define GQ_PARTS(F) launch_rb<F, 0, 64, 128, 1, 4, 4, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, splits)
   if (fmt == GQ_FMT_Q4_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q4_0));
   else if (fmt == GQ_FMT_Q8_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q8_0));
   else if (gq_fmt_is_q6k(fmt)) GQ_TRY(GQ_PARTS(GQ_FMT_Q6_K));
