@@ -1417,6 +1417,12 @@ int launch_gemm(const void *packed, const _Float16 *a16, int lda, void *c, const
 
 }  // namespace
 
+int gq_launch_split_sum(const float *part, float *c, size_t n, int parts, hipStream_t s) {
+  hipLaunchKernelGGL(k_split_sum<0>, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, part, (const float *)nullptr, c,
+                     n, 1, parts);
+  return gq_last_launch();
+}
+
 extern "C" size_t gq_gemm_workspace_bytes(int fmt, size_t M, size_t K) {
   // activations are first written as fp16 [M][padded K (+ 8 for the skinny
   // kernel)] unless they are fp16 of the padded width already and in k order

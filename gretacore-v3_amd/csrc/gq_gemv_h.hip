@@ -402,7 +402,10 @@ k_gemv_h(const uint8_t *__restrict__ w, size_t sc_off, const float *__restrict__
   const int ntiles = (int)gq_tiles(N);
   const size_t tile = (size_t)blockIdx.x * TW + tt;
   const HSrc<FMT> src = hsrc<FMT>(w, sc_off, tile < (size_t)ntiles ? tile : (size_t)ntiles - 1, C, N, K, lane);
-  const int c0 = (C * part) / KS, c1 = (C * (part + 1)) / KS;  // this wave's chunks (c0 < c1: KS <= C)
+  // K part blockIdx.y over workgroups: Cz chunks from zc, its own nb x N of y
+  const int zc = C * (int)blockIdx.y / (int)gridDim.y, Cz = C * ((int)blockIdx.y + 1) / (int)gridDim.y - zc;
+  y += (size_t)blockIdx.y * (size_t)nb * (size_t)N;
+  const int c0 = zc + (Cz * part) / KS, c1 = zc + (Cz * (part + 1)) / KS;  // this wave's chunks (c0 < c1: KS <= Cz)
 
   // weights of window `it` (chunks past the part re-read its last chunk)
   auto load_win = [&](int it, HChunk<FMT> (&ch)[WC]) {
@@ -426,7 +429,7 @@ k_gemv_h(const uint8_t *__restrict__ w, size_t sc_off, const float *__restrict__
     const int run = (int)threadIdx.x + u * NT;
     const int kr = run & 31, b = (run >> 5) % MR, p = run / (32 * MR);
     xsrow[u] = p * MR + b;
-    const int pc0 = (C * p) / KS, pc1 = (C * (p + 1)) / KS;
+    const int pc0 = zc + (Cz * p) / KS, pc1 = zc + (Cz * (p + 1)) / KS;
     xsrc[u] = x + (size_t)(b < nb ? b : 0) * K;
     xk0[u] = pc0 * F::CK + 8 * kr;
     xk1[u] = b < nb ? min(pc1 * F::CK, K) : 0;  // K % 32 == 0: a run is wholly in or out
@@ -960,17 +963,17 @@ int gq_gemv_h_plan(int fmt, size_t N, size_t K, int nb, int *R_out, int *ks_out,
 
 namespace {
 template <int FMT, int TW, int MR>
-int launch_h_tw(const void *packed, const float *x, float *y, int N, int K, int nb, int ks, hipStream_t s) {
+int launch_h_tw(const void *packed, const float *x, float *y, int N, int K, int nb, int ks, hipStream_t s, int kz = 1) {
   const int C = (int)gq_chunks(FMT, K);
   const size_t wgs = (gq_tiles(N) + TW - 1) / TW;
   const size_t sc_off = gq_sc_plane_offset(FMT, N, K);
   const uint8_t *w = (const uint8_t *)packed;
   constexpr int WC = kWin / HFmt<FMT>::CK;
-  const int NI = ((C + ks - 1) / ks + WC - 1) / WC;
+  const int NI = (((C + kz - 1) / kz + ks - 1) / ks + WC - 1) / WC;
   // x runs must spread evenly over the threads (TW <= MR / 2)
 #define GQ_LAUNCH_H(KS)                                                                                               \
   if constexpr (2 * TW <= MR && !(FMT == GQ_FMT_F16 && TW * KS > 8)) {                                               \
-    hipLaunchKernelGGL((k_gemv_h<FMT, TW, KS, MR>), dim3((unsigned)wgs), dim3(64 * TW * KS), 0, s, w, sc_off, x, y, \
+    hipLaunchKernelGGL((k_gemv_h<FMT, TW, KS, MR>), dim3((unsigned)wgs, (unsigned)kz), dim3(64 * TW * KS), 0, s, w, sc_off, x, y, \
                        N, K, C, nb, NI);                                                                              \
   } else {                                                                                                            \
     return GQ_ERR_INVALID_ARGS;                                                                                       \
@@ -1014,9 +1017,35 @@ int launch_h1_nck(const void *packed, const float *x, float *y, int N, int K, in
 #undef GQ_LAUNCH_H1
 }
 
+// Batch 9..16, few row tiles on a long K: four row tiles per workgroup and K in
+// parts over workgroups, the parts' sums in scratch.  A workgroup stages 16 rows
+// of activations over its K range whatever its row tiles, so with one or two
+// tiles each that outweighs the weights (batch 16, without / with: Q4_K 4096 x
+// 14336 24.7 / 20.2 us, 1024 x 14336 23.9 / 15.9, 8192 x 8192 29.6 / 21.9, Q8_0 44.7 /
+// 30.2, Q6_K 42.4 / 27.1).  Batch 8, K = 8192 on 256 tiles and the larger formats on
+// 256 tiles gain nothing (Q4_K 4096 x 14336 batch 8 17.1 / 18.1; 4096 x 8192 batch 16
+// 15.7 / 15.9; Q6_K 4096 x 14336 26.6 / 27.2).  GQ_ERR_UNSUPPORTED there, and
+// without scratch.
+template <int FMT>
+int launch_h_kz(const void *packed, const float *x, float *y, int N, int K, int nb, hipStream_t s) {
+  const size_t tiles = gq_tiles(N);
+  const int C = (int)gq_chunks(FMT, K), win = C * HFmt<FMT>::CK / kWin, wgs = (int)((tiles + 3) / 4);
+  const int kz = 256 / wgs < win / 8 ? 256 / wgs : win / 8;
+  const bool pays = tiles >= 400 ? K >= 8192 : K > 8192 && (kNibOrder<FMT> || tiles <= 128);
+  if (nb <= 8 || kz <= 1 || !pays) return GQ_ERR_UNSUPPORTED;
+  GqScratch ws((size_t)kz * nb * N * 4, s);
+  if (!ws.ptr) return GQ_ERR_UNSUPPORTED;
+  GQ_TRY((launch_h_tw<FMT, 4, 16>(packed, x, (float *)ws.ptr, N, K, nb, 4, s, kz)));
+  return gq_launch_split_sum((const float *)ws.ptr, y, (size_t)nb * N, kz, s);
+}
+
 template <int FMT>
 int launch_h(const void *packed, const float *x, float *y, int N, int K, int nb, hipStream_t s) {
   int tw, ks, cpw;
+  if constexpr (FMT != GQ_FMT_F16) {
+    const int r = launch_h_kz<FMT>(packed, x, y, N, K, nb, s);
+    if (r != GQ_ERR_UNSUPPORTED) return r;
+  }
   if (gq_gemv_h1_plan(FMT, N, K, nb, &tw, &ks, &cpw) == GQ_OK) {
     if (nb <= 8) {
       if (tw == 1) return launch_h1_nck<FMT, 1, 16, 8>(packed, x, y, N, K, nb, cpw, s);

@@ -97,5 +97,7 @@ int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, 
                          hipStream_t s);
 // fp16-weight rows of gq_gemm_f16w through the tiled GEMM (gq_gemm.hip)
 int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_t N, size_t K, hipStream_t s);
+// c[i] = the sum over p of part[p][i], in part order (gq_gemm.hip)
+int gq_launch_split_sum(const float *part, float *c, size_t n, int parts, hipStream_t s);
 // Compute units of the current device (cached per device; 0 without a device).
 int gq_device_cus(void);

@@ -127,7 +127,10 @@ int gq_split_q8_0(const void *d_blocks, size_t n_blocks, int8_t *d_q, float *d_s
 size_t gq_gemv_workspace_bytes(int fmt, size_t K, int batch);
 /* x f32 [batch][K], y f32 [batch][N].  workspace may be NULL: the library then
  * uses a per-device buffer it owns (allocated on first use; not for use under
- * stream capture).  Concurrent calls that share a workspace race. */
+ * stream capture).  Concurrent calls that share a workspace race.  Batch 9..16
+ * on a K of 8192 or more may split K over workgroups, with scratch memory of the
+ * call's own (not while the stream is being captured; the sums then round in
+ * another order). */
 int gq_gemv(int fmt, const void *d_packed, const float *d_x, float *d_y, size_t N, size_t K, int batch,
             void *d_workspace, size_t workspace_bytes, void *stream);
 /* Launch plan of gq_gemv for a shape (no GPU needed): row tiles per

@@ -192,3 +192,28 @@ def test_gemm_k_parts(dev, fmt, m, n, k, adt, odt):
         gq.gemm(fmt, packed, a, n, k, out_dtype=odt, c=c, workspace=ws)
         torch.cuda.synchronize()
         assert _rel(cg, ref) <= tol and _rel(c, ref) <= tol
+
+
+@pytest.mark.parametrize("fmt", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("b,n,k", [(9, 1025, 8448), (16, 6500, 8192), (13, 2000, 14336)])
+def test_gemv_k_parts(dev, fmt, b, n, k):
+    """Batch 9..16 with K over workgroups, and the unsplit kernel under capture."""
+    import gq
+    import torch
+    w = O.gen_weights(fmt, n, k, seed=b)
+    packed = torch.from_numpy(gq.repack_host(fmt, w, n, k)).to(dev)
+    x = torch.randn(b, k, generator=torch.Generator().manual_seed(b)).to(dev)
+    x[b - 1] *= 1e6
+    ref = _ref(fmt, w, x, n, k)
+    y, yg = gq.gemv(fmt, packed, x, n, k), torch.empty(b, n, device=dev)
+    rel = lambda t: float(((t.double() - ref).norm(dim=1) / ref.norm(dim=1)).max())  # noqa: E731
+    assert rel(y) <= TOL
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gq.gemv(fmt, packed, x, n, k, y=yg)
+    for _ in range(3):
+        yg.zero_()
+        g.replay()
+        gq.gemv(fmt, packed, x, n, k, y=y)
+        torch.cuda.synchronize()
+        assert rel(yg) <= TOL and rel(y) <= TOL
