@@ -467,16 +467,18 @@ struct RStep<GQ_FMT_Q6_K, NJ> {
   uint32_t sc[NJ];     // the step's four int8 scales (one per 16 k)
   uint32_t d[NJ];      // the super-block's d (fp16 bits)
 };
-// fp16 weights, row-major N x K (no T16 layout): the fragments as they are, one
-// 16-byte load each.  A wave's load touches 32 rows, 32 bytes of each; the
-// step's four loads together take whole 128-byte lines.
+// fp16 weights, row-major N x K (no T16 layout): nothing to dequantize, so they
+// go through LDS as the activations do.  A load instruction then takes whole
+// 128-byte lines of 8 rows, where fragments loaded straight into registers touch 32
+// rows, 32 bytes of each; waves along M share the tile; and no registers are held
+// for steps in flight.  Registers / LDS, us: 64 x 4096 x 4096 25.2 / 21.3, 512 x 4096 x
+// 4096 45.4 / 40.4, 64 x 4096 x 14336 48.5 / 42.4, 128 x 32000 x 2048 50.7 / 47.1, 512 x
+// 32000 x 4096 209 / 203, 2048 x 4096 x 14336 319.5 / 320.5.
 template <int NJ>
-struct RStep<GQ_FMT_F16, NJ> {
-  gq_u4 q[NJ][4];  // MFMA k-step ks
-};
+struct RStep<GQ_FMT_F16, NJ> {};
 // loads of one column block and K step
 template <int FMT>
-constexpr int kRLoads = FMT == GQ_FMT_Q6_K ? 6 : FMT == GQ_FMT_F16 ? 4 : 3;
+constexpr int kRLoads = FMT == GQ_FMT_Q6_K ? 6 : FMT == GQ_FMT_F16 ? 0 : 3;
 
 // Buffer resource over the 4 GiB from p (raw: stride 0, the offset in
 // bytes).  The register-B kernel addresses its operands as a 32-bit per-lane
@@ -502,28 +504,9 @@ GQ_DEV uint32_t ld2_b(const void *base, uint32_t vo, uint32_t so) {
   return __builtin_amdgcn_raw_buffer_load_b16(gq_rsrc(base), vo, so, 0);
 }
 
-// (F16: so[0] is the matrix's size in bytes, K the row length.  The step's
-// halves of 32 k lie wholly inside the row or past it -- K % 32 == 0 -- and those
-// past it are read beyond the resource's range, which gives zeros.)
 template <int FMT, int NJ>
-GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_t (&so)[NJ], int K, int step,
+GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_t (&so)[NJ], int step,
                        RStep<FMT, NJ> &st) {
-  if constexpr (FMT == GQ_FMT_F16) {
-    const __amdgpu_buffer_rsrc_t r =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), (short)0, (int)so[0], 0x00020000);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint32_t vo = (int)BK * step + 32 * h < K ? qo[j] : so[0];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, 128u * (uint32_t)step + 64u * h + 16u * e, 0);
-          st.q[j][2 * h + e] = gq_u4{v[0], v[1], v[2], v[3]};
-        }
-      }
-    return;
-  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     if constexpr (FMT == GQ_FMT_F16) {
@@ -584,6 +567,36 @@ GQ_DEV void load_a_lds_b(const _Float16 *a, const uint32_t *ao, int step, int wa
   }
 }
 
+// fp16 weights: a step's BN rows x 64 k into LDS as the activation tile's.  Runs
+// of 8 past the row's end (K % 32 == 0) are read beyond the resource's range, which
+// writes zeros (no step of k past K leaves an earlier step's weights in the buffer).
+template <int BN, int NW>
+GQ_DEV void b_offsets(int K, int N, int n0, int wave, int lane, uint32_t (&bo)[BN / (8 * NW)]) {
+  constexpr int PER_WAVE = BN / (8 * NW);
+#pragma unroll
+  for (int i = 0; i < PER_WAVE; ++i) {
+    const int row0 = 8 * (wave * PER_WAVE + i);
+    const int c = (lane & 7) ^ a_swz(row0 + (lane >> 3));
+    int n = n0 + row0 + (lane >> 3);
+    if (n >= N) n = N - 1;  // clamped; those columns are never stored
+    bo[i] = 2u * ((uint32_t)n * (uint32_t)K + 8u * (uint32_t)c);
+  }
+}
+template <int BN, int NW>
+GQ_DEV void load_b_lds(const uint8_t *w, uint32_t wb, int K, const uint32_t *bo, int step, int wave, int lane,
+                       _Float16 *Bs) {
+  constexpr int PER_WAVE = BN / (8 * NW);
+  const __amdgpu_buffer_rsrc_t r =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(w), (short)0, (int)wb, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < PER_WAVE; ++i) {
+    const int row0 = 8 * (wave * PER_WAVE + i);
+    const int k = BK * step + 8 * ((lane & 7) ^ a_swz(row0 + (lane >> 3)));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)(Bs + row0 * BK), 16,
+                                             k < K ? bo[i] : wb, (uint32_t)step * (2u * BK), 0, 0);
+  }
+}
+
 // Q4_K: the fp16 factors of the sub-block 2 (step & 3) + h of column block j
 // (sc, -1024 sc, d, -dmin m), decoded once per K step.
 struct QKf {
@@ -641,7 +654,7 @@ GQ_DEV void q6k_factors(const RStep<GQ_FMT_Q6_K, NJ> &st, int kh, gq_half2 (&f)[
 template <int FMT, int NJ>
 GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const QKf *qk, const gq_half2 *q6,
                       uint32_t mg) {
-  if constexpr (FMT == GQ_FMT_F16) return __builtin_bit_cast(gq_half8, st.q[j][ks]);
+  if constexpr (FMT == GQ_FMT_F16) return gq_half8{};  // (read from LDS)
   else {
   const int h = ks >> 1;
   gq_half2 p[4];
@@ -729,10 +742,20 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   __shared__ __attribute__((aligned(16))) _Float16 As_1[KG * BM * BK];
   __shared__ __attribute__((aligned(16))) _Float16 As_2[PD >= 3 ? KG * BM * BK : 8];
   __shared__ __attribute__((aligned(16))) _Float16 As_3[PD >= 4 ? KG * BM * BK : 8];
+  // (fp16 weights: their tiles beside the activations')
+  constexpr bool LB = FMT == GQ_FMT_F16;
+  __shared__ __attribute__((aligned(16))) _Float16 Bs_0[LB ? KG * BN * BK : 8];
+  __shared__ __attribute__((aligned(16))) _Float16 Bs_1[LB ? KG * BN * BK : 8];
+  __shared__ __attribute__((aligned(16))) _Float16 Bs_2[LB && PD >= 3 ? KG * BN * BK : 8];
+  __shared__ __attribute__((aligned(16))) _Float16 Bs_3[LB && PD >= 4 ? KG * BN * BK : 8];
   const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) / NW);
   auto As_of = [&](auto b) -> _Float16 * {
     constexpr int v = decltype(b)::value;
     return (v == 0 ? As_0 : v == 1 ? As_1 : v == 2 ? As_2 : As_3) + kg * (BM * BK);
+  };
+  auto Bs_of = [&](auto b) -> _Float16 * {
+    constexpr int v = decltype(b)::value;
+    return (v == 0 ? Bs_0 : v == 1 ? Bs_1 : v == 2 ? Bs_2 : Bs_3) + kg * (BN * BK);
   };
   // this workgroup's K steps: part blockIdx.y of sps steps, its output the
   // part's own M x N (all of K where there are no parts)
@@ -744,7 +767,8 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   using B1 = std::integral_constant<int, 1>;
   using B2 = std::integral_constant<int, 2>;
   using B3 = std::integral_constant<int, 3>;
-  constexpr int NA = BM / (8 * NW);  // activation-tile loads per thread and K step
+  // activation-tile (fp16 weights: and weight-tile) loads per thread and K step
+  constexpr int NA = BM / (8 * NW) + (LB ? BN / (8 * NW) : 0);
   // loads a step may leave in flight at its end: the activation tiles of
   // steps s + 2 .. s + PD - 1 and the weights of steps s + 2 .. s + PD
   constexpr int pend = (PD - 2) * NA + (PD - 1) * kRLoads<FMT> * NJ;
@@ -768,10 +792,8 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     if (t >= ntiles) t = ntiles - 1;  // clamped; those columns are never stored
     const uint32_t tc = (uint32_t)t * (uint32_t)C;
     const uint32_t slot = 16u * (16u * (uint32_t)kh + (uint32_t)r);
-    if constexpr (FMT == GQ_FMT_F16) {  // (C: the row length, sc_off: the matrix's bytes)
-      const int n = n0 + (BN / WN) * wn + 32 * j + (lane & 31);
-      qo[j] = (uint32_t)(n < N ? n : N - 1) * (2u * (uint32_t)C) + 32u * (uint32_t)kh;
-      so[j] = sc_off;
+    if constexpr (LB) {
+      qo[j] = so[j] = 0;
     } else if constexpr (FMT == GQ_FMT_Q4_0) {
       qo[j] = (tc << 10) + slot;
       so[j] = sc_off + tc * 128u + 8u * r;
@@ -799,13 +821,17 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   const uint32_t mg = gq_nib_magic();
   uint32_t ao[BM / (8 * NW)];
   a_offsets<BM, NW>(lda, M, m0, wave, lane, ao);
+  // (fp16 weights: C is the row length, sc_off the matrix's bytes)
+  uint32_t bo[BN / (8 * NW)];
+  if constexpr (LB) b_offsets<BN, NW>(C, N, n0, wave, lane, bo);
+  const int brow = (BN / WN) * wn + (lane & 31);
   const int arow = (BM / WM) * wm + (lane & 31);
   const int sw = a_swz(lane & 31);
 
   // the group's l-th step of K
   // fp16 rows at a power-of-two stride put every workgroup's step on the same
   // few memory channels: each weight column tile starts its walk one step
-  // further on (17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
+  // further on (fragments loaded into registers, 17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
   // formats, whose tiles are contiguous, gain nothing)
   const int off = FMT == GQ_FMT_F16 ? nt % nl : 0;
   auto gstep = [&](int l) {
@@ -824,14 +850,20 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     const int s1 = gstep(l + PD - 1 < nl ? l + PD - 1 : nl - 1);
     const int s2 = gstep(l + PD < nl ? l + PD : nl - 1);
     load_a_lds_b<BM, NW>(a16, ao, s1, wave, As_of(NB{}));
+    if constexpr (LB) load_b_lds<BN, NW>(w, sc_off, C, bo, s1, wave, lane, Bs_of(NB{}));
     __builtin_amdgcn_sched_barrier(0);
     const _Float16 *As = As_of(buf_c) + arow * BK;
     RStep<FMT, NJ> &cur = wst[BUF];
-    gq_half8 af[2][TM];
+    gq_half8 af[2][TM], bl[2][NJ];
     auto read_a = [&](int ks, int fb) {
       const int ch = (4 * (ks >> 1) + 2 * kh + (ks & 1)) ^ sw;
 #pragma unroll
       for (int i = 0; i < TM; ++i) af[fb][i] = *reinterpret_cast<const gq_half8 *>(As + 32 * i * BK + 8 * ch);
+      if constexpr (LB) {
+        const _Float16 *Bs = Bs_of(buf_c) + brow * BK;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) bl[fb][j] = *reinterpret_cast<const gq_half8 *>(Bs + 32 * j * BK + 8 * ch);
+      }
     };
     read_a(0, 0);
     QKf qk[NJ][2];
@@ -843,13 +875,13 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
       if (ks + 1 < KS) read_a(ks + 1, (ks + 1) & 1);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const gq_half8 bf = rfrag<FMT, NJ>(cur, j, ks, step, qk[j], q6[j], mg);
+        const gq_half8 bf = LB ? bl[ks & 1][j] : rfrag<FMT, NJ>(cur, j, ks, step, qk[j], q6[j], mg);
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[i][j] = gq_mfma32(af[ks & 1][i], bf, acc[i][j]);
       }
     }
     // the register stage of this step is free: request step + PD into it
-    load_rstep<FMT, NJ>(w, qo, so, C, s2, cur);
+    if constexpr (!LB) load_rstep<FMT, NJ>(w, qo, so, s2, cur);
     // the activation tile and the weights of step + 1 must have landed
     __builtin_amdgcn_s_waitcnt(kWaitPend);
     __syncthreads();
@@ -861,7 +893,8 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     constexpr int i = decltype(b)::value;
     const int st = gstep(i < nl ? i : nl - 1);
     if constexpr (i < PD - 1) load_a_lds_b<BM, NW>(a16, ao, st, wave, As_of(b));
-    load_rstep<FMT, NJ>(w, qo, so, C, st, wst[i]);
+    if constexpr (LB && i < PD - 1) load_b_lds<BN, NW>(w, sc_off, C, bo, st, wave, lane, Bs_of(b));
+    if constexpr (!LB) load_rstep<FMT, NJ>(w, qo, so, st, wst[i]);
   };
   // the tile's row scales, requested before the operands (the oldest load,
   // so the wait below covers it) and kept in LDS for the epilogue, whose
@@ -1224,9 +1257,11 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
                      dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits),                                     \
                      dim3(64 * WM * WN * KG), 0, s, (const uint8_t *)packed, sc_off, a16,      \
                      lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps)
-  // the depths whose LDS fits (activation buffers, the K groups' exchange,
+  // the depths whose LDS fits (operand buffers, the K groups' exchange,
   // the row scales); a deeper request falls back to the deepest that fits
-  constexpr auto lds = [](int d) { return d * KG * BM * BK * 2 + (KG - 1) * WM * WN * 4096 + BM * 4; };
+  constexpr auto lds = [](int d) {
+    return d * KG * (BM + (FMT == GQ_FMT_F16 ? BN : 0)) * BK * 2 + (KG - 1) * WM * WN * 4096 + BM * 4;
+  };
   constexpr int kLds = 160 * 1024;
   if (KG > 1 && nsteps % KG) return GQ_ERR_INVALID_ARGS;
   if constexpr (lds(4) <= kLds) {
@@ -1333,23 +1368,23 @@ template <int FMT, int CBF16>
 int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
                   hipStream_t s) {
   switch (pick_tile(FMT, M, N, K)) {
-  // (fp16 weights hold 16 registers a step: depth 2 where the accumulators
-  // leave no room for more)
-  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 3);
+  // (fp16 weights: both tiles are in LDS, launch_rb takes the depth that fits, and
+  // the smallest tile runs two K groups, whose buffers leave room for depth 2)
+  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 3);
   case 13: return launch_rb<FMT, CBF16, 128, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s);
   case 17: return launch_rb<FMT, CBF16, 128, 128, 1, 4, 2>(packed, a16, lda, c, rs, M, N, K, s);
   default:
-    return launch_rb<FMT, CBF16, 64, 128, 1, 4, 4>(packed, a16, lda, c, rs, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4);
+    return launch_rb<FMT, CBF16, 64, 128, 1, 4, FMT == GQ_FMT_F16 ? 2 : 4>(packed, a16, lda, c, rs, M, N, K, s);
   }
 }
 
 // Few workgroups (a short, narrow C over a long K): K in parts over workgroups,
 // each part's sums in fp32 in `part`, added by k_split_sum.  About one
 // workgroup per CU, at least 8 steps a part, and only from 32 steps on: fp16 weights,
-// 64 rows, unsplit / split: 4096 x 14336 174 / 47 us, 4096 x 4096 46 / 24, 300 x 14336
+// 64 rows, unsplit / split (weights loaded into registers): 4096 x 14336 174 / 47 us, 4096 x 4096 46 / 24, 300 x 14336
 // 130 / 28; 4096 x 1120 (20 steps) 18.6 / 20.3.
 struct SplitPlan {
-  int bm, splits;  // tile rows (64: 64 x 128 in four K groups; 128: 128 x 128 in two)
+  int bm, splits;  // tile rows (64 x 128 or 128 x 128, in two K groups)
 };
 SplitPlan split_plan(int M, int N, int nsteps) {
   const int bm = M > 64 ? 128 : 64;
@@ -1364,8 +1399,7 @@ int launch_split(const void *packed, const _Float16 *a16, int lda, float *c, con
   if (p.bm == 128)
     GQ_TRY((launch_rb<FMT, 0, 128, 128, 1, 4, 2, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
   else
-    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 4, true>(packed, a16, lda, part, nullptr, M, N, K, s, FMT == GQ_FMT_F16 ? 2 : 4,
-                                                p.splits)));
+    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 2, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
   const size_t mn = (size_t)M * (size_t)N;
   hipLaunchKernelGGL(k_split_sum<0>, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
   return gq_last_launch();

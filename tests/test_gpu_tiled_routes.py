@@ -123,6 +123,23 @@ def test_f16w_tiled(dev, m, n, k):
     assert bool((c[m] == 7.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 4100, 352), (700, 8300, 352), (641, 4200, 352), (4865, 5300, 352)])
+def test_f16w_infinite_weight(dev, m, n, k):
+    """One infinite weight of a step whose buffer a step past K takes next: its
+    output is +-Inf, and NaN only if the buffer still held it against zeros."""
+    import gq
+    import torch
+    g = torch.Generator().manual_seed(n)
+    w = torch.randn(n, k, generator=g).half()
+    w[::2, 200] = float("inf")
+    w[1::2, 330] = float("inf")
+    w = w.to(dev)
+    a = torch.randn(m, k, generator=g).abs().add_(0.1).to(dev)
+    c = torch.empty(m, n, device=dev)
+    gq.gemm_f16w(w, a, n, k, c=c)
+    assert bool((c == float("inf")).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (130, 140, 96), (129, 257, 4128), (260, 100, 1056)])
 @pytest.mark.parametrize("inf", [False, True])
 def test_q8_i8_scales(dev, m, n, k, inf):
