@@ -568,8 +568,12 @@ GQ_DEV void load_a_lds_b(const _Float16 *a, const uint32_t *ao, int step, int wa
 }
 
 // fp16 weights: a step's BN rows x 64 k into LDS as the activation tile's.  Runs
-// of 8 past the row's end (K % 32 == 0) are read beyond the resource's range, which
-// writes zeros (no step of k past K leaves an earlier step's weights in the buffer).
+// of 8 past the row's end (K % 32 == 0) are given the resource's end as their
+// offset, and a load out of its range writes zeros (no step of k past K leaves an
+// earlier step's weights in the buffer).  The step is part of the per-lane offset:
+// in a matrix smaller than one padded row the step's columns alone lie past the
+// resource's end, and the range check must not depend on how it counts a scalar
+// offset.
 template <int BN, int NW>
 GQ_DEV void b_offsets(int K, int N, int n0, int wave, int lane, uint32_t (&bo)[BN / (8 * NW)]) {
   constexpr int PER_WAVE = BN / (8 * NW);
@@ -593,7 +597,7 @@ GQ_DEV void load_b_lds(const uint8_t *w, uint32_t wb, int K, const uint32_t *bo,
     const int row0 = 8 * (wave * PER_WAVE + i);
     const int k = BK * step + 8 * ((lane & 7) ^ a_swz(row0 + (lane >> 3)));
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)(Bs + row0 * BK), 16,
-                                             k < K ? bo[i] : wb, (uint32_t)step * (2u * BK), 0, 0);
+                                             k < K ? bo[i] + (uint32_t)step * (2u * BK) : wb, 0, 0, 0);
   }
 }
 

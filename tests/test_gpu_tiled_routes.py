@@ -123,6 +123,24 @@ def test_f16w_tiled(dev, m, n, k):
     assert bool((c[m] == 7.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(49, 1, 32), (64, 3, 64), (50, 7, 32), (70, 1, 288), (300, 2, 96)])
+def test_f16w_fewer_weights_than_a_padded_row(dev, m, n, k):
+    """Steps past K start beyond the matrix's end: they read zeros, not the Inf
+    that follows it.  A rounded once to fp16: 2^-11 of each product, 2^-10 bounds
+    it with the fp32 sums."""
+    import gq
+    import torch
+    g = torch.Generator().manual_seed(m + k)
+    w = torch.randn(n * k + 4096, generator=g).half()
+    w[n * k:] = float("inf")
+    w = w.to(dev)
+    wm = w[:n * k].view(n, k)
+    a = torch.randn(m, k, generator=g).to(dev)
+    c = gq.gemm_f16w(wm, a, n, k).double()
+    ref = a.double() @ wm.double().t()
+    assert bool(((c - ref).abs() <= 2.0**-10 * (a.double().abs() @ wm.double().abs().t())).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 4100, 352), (700, 8300, 352), (641, 4200, 352), (4865, 5300, 352)])
 def test_f16w_infinite_weight(dev, m, n, k):
     """One infinite weight of a step whose buffer a step past K takes next: its
