@@ -335,40 +335,44 @@ k_compat_gemv_lds(const TA *__restrict__ a, const uint8_t *__restrict__ b, float
   }
 }
 
-// ---- matrix-core form: 2..32 rows (any count with force_gemv) -----------------
-// A contraction of the integer codes with the fp32 (or fp16) activations that
-// loses nothing to the matrix cores' 16-bit operands: the codes are exact in
-// fp16, and an fp32 activation is split into two fp16 limbs, hi = fp16(x 2^s),
-// lo = fp16(x 2^s - hi) -- 22 bits and sign, s the power of two that brings the
-// largest magnitude of the row's window into [2^14, 2^15) (fp16 activations
-// are one limb, exact).  v_mfma_f32_16x16x32_f16 is one scale group of 32 for 16
-// weight rows and 16 activation rows; both limbs go to one fp32 accumulator,
-// which is scaled by the group's factor and added to the window's sum, that to
-// the total by 2^-s, compensated.  Odd groups hold -x and count with -s: the
-// MFMA's internal sum rounds downwards, a bias that would otherwise add up over
-// K (rel-L2 against float64 1.3e-7 at K = 4096, 1.9e-7 at 14336; alternating 9.1-
-// 9.8e-8, the fp32 VALU kernels 1.1-1.2e-7).  14336 x 4096, INT4 / INT8, 8 rows:
-// 43 / 49 -> 18 / 21 us; 32 rows 157 / 170 -> 32 / 34.
+// ---- matrix-core form: 3..32 rows (any count with force_gemv) -----------------
+// The codes against the activations with nothing of either lost on the way to the
+// products; fp32 sums.
+//  - fp32 activations: three bf16 limbs, x = hi + mid + lo, each the top 8 bits of what
+//    is left: 24 bits at any exponent (the codes are exact in bf16).  The MFMA takes
+//    subnormal inputs as zeros, so a row's window below 2^-60 goes in times 2^66; entries
+//    under 2^-110 beside one above 2^-63 keep their first 8 or 16 bits.
+//    (Two fp16 limbs under one power of two per 256 k kept 22 bits of a window's
+//    largest entries and fewer of the rest: with an entry 1e7 times the others, whose
+//    code was 0, 9e-5 off.  v_mfma_f32_16x16x4_f32 instead, 1/16 of the rate: 8 rows
+//    of 14336 x 4096, INT4, 29 us; v_mfma_f32_4x4x1 with its 16 blocks 24.5.)
+//  - fp16 activations: as they are (the codes are exact in fp16).
+// v_mfma_f32_16x16x32 is one scale group of 32 for 16 weight rows and 16 activation
+// rows; the limbs go to one fp32 accumulator, lowest first, which is scaled by the
+// group's factor and added to the window's sum, that to the total, compensated.
+// Up to 8 rows two MFMAs do: A rows 0..7 hold hi and 8..15 mid, then lo / 2 both
+// times, and the two halves of D are added at the end.  Odd groups count the
+// codes negated and with -s: the MFMA's internal sum rounds downwards, a bias that
+// would otherwise add up over K.
 //
-// Workgroup: TW row tiles of 16 x KS parts of K, one wave each.  The limbs of a
-// window (WIN k of every part) are made once per workgroup in LDS, double-
-// buffered; a wave's 16-byte weight loads (lane (g, r): row r, 16-byte piece g of 64)
-// go out two windows ahead.  A piece is one group's (INT4) or half a group's
-// (INT8) codes of one row, so lane swaps (permlane) turn four pieces into
+// What bounds it is VALU work: a code's way to bf16 (v_cvt_off_f32_i4 or a byte's
+// conversion, and half a packing) and the limbs' making.  14336 x 4096, INT4 / INT8,
+// VALU kernels -> this: 8 rows 44 / 51 -> 19.1 / 25.4 us, 32 rows 155 / 172 -> 31 / 36;
+// rel-L2 against float64 8.9e-8 at 8 rows (VALU kernels 1.1-1.2e-7).
+//
+// Workgroup: TW row tiles of 16 x KS parts of K, one wave each.  The operands of
+// a window (WIN k of every part) are made once per workgroup in LDS, double-
+// buffered where that fits; a wave's 16-byte weight loads (lane (g, r): row r, 16-byte
+// piece g of 64) go out two windows ahead.  A piece is one group's (INT4) or half a
+// group's (INT8) codes of one row, so lane swaps (permlane) turn four pieces into
 // B fragments of one group each; k order inside a group is free as long as the
-// limbs are stored alike.
+// activations are stored alike.
 template <bool INT4>
 struct CmGroup {  // 128 k of 16 rows: four groups' codes and scales
   gq_u4 q[INT4 ? 1 : 2];
   float s;  // lane (g, r): the scale of group g of row r
 };
 
-GQ_DEV uint32_t cm_max_row(uint32_t v) {  // largest of each 16 lanes (DPP; 0 is max's identity)
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));
-  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));
-}
 // lane groups (g0 g1 g2 g3) of a and b -> a: (a0 a1 b0 b1), b: (a2 a3 b2 b3)
 GQ_DEV void cm_swap32(uint32_t &a, uint32_t &b) {
   const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
@@ -382,8 +386,18 @@ GQ_DEV void cm_swap16(uint32_t &a, uint32_t &b) {
   b = v[1];
 }
 
+typedef __bf16 cm_bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 cm_bf2 __attribute__((ext_vector_type(2)));
+
+GQ_DEV uint32_t cm_max_row(uint32_t v) {  // largest of each 16 lanes (DPP; 0 is max's identity)
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));
+}
+
 template <bool INT4, typename TA, int MR, int WIN, int TW, int KS>
-__global__ void __launch_bounds__(64 * TW * KS)
+__global__ void __launch_bounds__(64 * TW * KS, MR == 32 && KS == 2 ? 4 : 1)
 k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__restrict__ c,
               const float *__restrict__ scales, const float *__restrict__ head_scales, int M, int N, int K, int lda,
               int ldc, int head_dim, int NI) {
@@ -391,17 +405,21 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
   const int z0 = (K + WIN - 1) / WIN * (int)blockIdx.z / (int)gridDim.z;
   const int nw = (K + WIN - 1) / WIN * ((int)blockIdx.z + 1) / (int)gridDim.z - z0;
   c += (size_t)blockIdx.z * (size_t)M * (size_t)ldc;
-  constexpr int L = sizeof(TA) == 4 ? 2 : 1;  // limbs
+  constexpr bool F32 = sizeof(TA) == 4;
+  static_assert(F32 || INT4, "fp16 activations: INT4 only");
+  constexpr int U = F32 ? 3 : 1;              // limbs
   constexpr int NG = WIN / 128;               // 128-k groups per window
   constexpr int NB = WIN / 32;                // scale groups per window
   constexpr int RUN = WIN / 8;                // runs of 8 per row and window
   constexpr int NT = 64 * TW * KS;
   constexpr int RPT = KS * MR * RUN / NT;     // runs per thread and window
   constexpr int MT = MR > 16 ? MR / 16 : 1;   // 16-row tiles of activations
-  constexpr int LB = NB * 4 * MR * 16;        // LDS bytes of a limb of a part's window: [NB][4][MR][16]
+  constexpr int WB = NB * U * 4 * MR * 16;    // LDS bytes of a part's window: [NB][U][4][MR][16]
   static_assert(RPT >= 1 && RPT * NT == KS * MR * RUN && (RUN == 16 || RUN == 32), "runs divide evenly");
-  __shared__ __attribute__((aligned(16))) unsigned char xs[2][KS][L * LB];
-  __shared__ __attribute__((aligned(16))) float xsc[2][KS * MR];  // 2^-s per part and row
+  // buffers: two where they leave room for the workgroups a CU should hold (16 waves)
+  constexpr int XB = 2 * KS * WB <= (TW * KS > 8 ? 160 : 80) * 1024 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) unsigned char xs[XB][KS][WB];
+  __shared__ __attribute__((aligned(16))) float xsc[XB][KS * MR];  // what a part's row of the window counts for
   static_assert(sizeof(xs) >= (size_t)KS * TW * MT * 64 * 16, "the parts' sums reuse it");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -416,7 +434,7 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
   const float *srow = scales + (size_t)nr * nb;
 
   // weights and scales of window w; past the row's end another group's are
-  // read instead, with scale 0 (their limbs are zeros too)
+  // read instead, with scale 0 (their activations are zeros too)
   auto load_win = [&](int w, CmGroup<INT4> (&gr)[NG]) {
     w = w < w1 ? w : w1 - 1;
 #pragma unroll
@@ -437,8 +455,8 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
     }
   };
   // activations: run u of this thread = (part, row, run of the window)
-  float xv[RPT][8];
-  bool xin[RPT];
+  constexpr int XU = F32 ? 2 : 1;  // 16-byte loads of a run
+  gq_u4 xv[RPT][XU];
   auto load_x = [&](int it) {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
@@ -446,72 +464,86 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
       const int kr = run % RUN, row = (run / RUN) % MR, p = run / (RUN * MR);
       const int w = z0 + nw * p / KS + it;
       const int k = w * WIN + 8 * kr;
-      xin[u] = m_base + row < M && w < z0 + nw * (p + 1) / KS && k < K;  // (K % 32 == 0: a run is whole)
-      const TA *src = a + (size_t)(xin[u] ? m_base + row : 0) * lda + (xin[u] ? k : 0);
-      if constexpr (L == 2) {
-        const gq_f4 v0 = *reinterpret_cast<const gq_f4 *>(src), v1 = *reinterpret_cast<const gq_f4 *>(src + 4);
+      const bool in = m_base + row < M && w < z0 + nw * (p + 1) / KS && k < K;  // (K % 32 == 0: a run is whole)
+      const gq_u4 *src = reinterpret_cast<const gq_u4 *>(a + (size_t)(in ? m_base + row : 0) * lda + (in ? k : 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          xv[u][e] = v0[e];
-          xv[u][4 + e] = v1[e];
-        }
-      } else {
-        const gq_half8 v = *reinterpret_cast<const gq_half8 *>(src);
+      for (int i = 0; i < XU; ++i) {
+        const gq_u4 v = src[i];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xv[u][e] = (float)v[e];
+        for (int e = 0; e < 4; ++e) xv[u][i][e] = in ? v[e] : 0u;
       }
     }
   };
+  // A limb's units of a group: [4 lane groups][rows][16].  The row's place is
+  // exclusive-or'ed with the unit's, so the runs that consecutive lanes store lie in
+  // different banks.  Limbs (offsets from the group's): MR = 8: 16 rows hi and
+  // mid, 8 rows lo / 2; else one after the other
+  constexpr int GB = U * 4 * MR * 16;                  // bytes of a group
+  constexpr int R0 = F32 && MR == 8 ? 16 : MR;         // rows of the first unit
+  constexpr int MID = MR == 8 ? 8 * 16 : 4 * MR * 16;  // hi -> mid
   auto store_x = [&](int buf) {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
       const int run = (int)threadIdx.x + u * NT;
       const int kr = run % RUN, row = (run / RUN) % MR, p = run / (RUN * MR);
-      // the window's largest magnitude (a NaN does not count: its limbs are
-      // NaN whatever the scale)
-      float af = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) af = fmaxf(af, fabsf(xv[u][e]));
-      uint32_t am = cm_max_row(xin[u] ? __float_as_uint(af) : 0u);
-      if constexpr (RUN == 32) {
-        const auto v = __builtin_amdgcn_permlane16_swap(am, am, false, false);
-        am = max(v[0], v[1]);
-      }
-      // 2^s and 2^-s, both normal floats
-      const uint32_t fe = (uint32_t)min(268 - (int)(am >> 23), 253);
-      const float f = __uint_as_float((fe << 23) | ((kr & 4) ? 0x80000000u : 0u)), f16 = f * 0.0625f;  // (odd groups: -x)
-      if (kr == 0) xsc[buf][p * MR + row] = __uint_as_float((254u - fe) << 23);
-      gq_half8 hi, lo;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        // INT4: the code order (gq_nib_halves over plain nibbles), its 16 x
-        // codes against a sixteenth of the activation.  Both limbs are one
-        // mixed-precision fma with one rounding (x f is exact).
-        const int k = INT4 ? (e >> 1) + 4 * (e & 1) : e;
-        const float fs = INT4 && (e & 2) ? f16 : f;
-        hi[e] = (_Float16)fmaf(xv[u][k], fs, -0.f);
-        if constexpr (L == 2) lo[e] = (_Float16)fmaf(xv[u][k], fs, -(float)hi[e]);
-      }
-      if constexpr (L == 2) {
-        // an Inf stays in hi alone: its residual would be NaN
-        if (__any((int)(am == 0x7F800000u))) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (__builtin_isinf((float)hi[e])) lo[e] = (_Float16)0.f;
-        }
-      }
       const int blk = kr >> 2, unit = kr & 3;
       const int gq = INT4 ? unit : ((unit & 1) << 1) | (unit >> 1);  // (the INT8 swap's order)
-      unsigned char *d = &xs[buf][p][((blk * 4 + gq) * MR + row) * 16];
-      gq_u4 hv = __builtin_bit_cast(gq_u4, hi);
+      const int rx = row ^ (gq | (blk & 1) << 2);
+      unsigned char *d = &xs[XB == 2 ? buf : 0][p][blk * GB + (gq * R0 + rx) * 16];
+      if constexpr (F32) {
+        float x[8], m[8], l[8], t = 0.f, us = 1.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) hv[e] = xin[u] ? hv[e] : 0u;
-      *reinterpret_cast<gq_u4 *>(d) = hv;
-      if constexpr (L == 2) {
-        gq_u4 lv = __builtin_bit_cast(gq_u4, lo);
+        for (int e = 0; e < 8; ++e) {
+          x[e] = __uint_as_float(xv[u][e >> 2][e & 3]);
+          t += fabsf(x[e]);
+        }
+        const bool odd = t != 0.f && !(t >= 0x1p-60f && t < __builtin_inff());  // small or not finite
+        const bool any = __any(odd);
+        if (any) {
+          float mx = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) lv[e] = xin[u] ? lv[e] : 0u;
-        *reinterpret_cast<gq_u4 *>(d + LB) = lv;
+          for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[e]));
+          uint32_t wm = cm_max_row(__float_as_uint(mx));  // (the window's RUN lanes are consecutive)
+          if constexpr (RUN == 32) {
+            const auto v = __builtin_amdgcn_permlane16_swap(wm, wm, false, false);
+            wm = max(v[0], v[1]);
+          }
+          const bool up = __uint_as_float(wm) < 0x1p-60f;
+          us = up ? 0x1p-66f : 1.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            x[e] *= up ? 0x1p66f : 1.f;
+            if (x[e] != x[e]) x[e] = __uint_as_float(0x7FC00000u);
+          }
+        }
+        if (kr == 0) xsc[XB == 2 ? buf : 0][p * MR + row] = us * (INT4 ? 16.f : 1.f);  // (INT4 codes: by sixteenths)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m[e] = x[e] - __uint_as_float(__float_as_uint(x[e]) & 0xFFFF0000u);
+        if (any) {  // (an Inf or NaN is its first limb alone)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) m[e] = fabsf(x[e]) < __builtin_inff() ? m[e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          l[e] = m[e] - __uint_as_float(__float_as_uint(m[e]) & 0xFFFF0000u);
+          if constexpr (MR == 8) l[e] *= 0.5f;
+        }
+        auto put = [&](unsigned char *to, const float (&v)[8]) {
+          gq_u4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)  // (the upper halves of two)
+            o[e] = __builtin_amdgcn_perm(__float_as_uint(v[2 * e + 1]), __float_as_uint(v[2 * e]), 0x07060302u);
+          *reinterpret_cast<gq_u4 *>(to) = o;
+        };
+        put(d, x);
+        put(d + MID, m);
+        put(MR == 8 ? &xs[XB == 2 ? buf : 0][p][blk * GB + (4 * 16 + gq * 8 + rx) * 16] : d + 2 * MID, l);
+      } else {
+        // (the order of gq_nib_halves over plain nibbles: k 0 4 1 5 2 6 3 7)
+        const uint32_t x0 = xv[u][0][0], x1 = xv[u][0][1], x2 = xv[u][0][2], x3 = xv[u][0][3];
+        *reinterpret_cast<gq_u4 *>(d) =
+            gq_u4{__builtin_amdgcn_perm(x2, x0, 0x05040100u), __builtin_amdgcn_perm(x2, x0, 0x07060302u),
+                  __builtin_amdgcn_perm(x3, x1, 0x05040100u), __builtin_amdgcn_perm(x3, x1, 0x07060302u)};
       }
     }
   };
@@ -521,9 +553,14 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = comp[t] = gq_f4{0.f, 0.f, 0.f, 0.f};
   const uint32_t mg = gq_nib_magic();
+  // the lane's A row in an even and an odd group's units
+  const int r8 = MR == 8 ? (r & 7) : r;
+  const int ra = F32 ? r : r8;  // (the first unit's row)
+  const int xo[2] = {(g * R0 + (ra ^ g)) * 16, (g * R0 + (ra ^ (g | 4))) * 16};
+  const int xl[2] = {(64 + g * 8 + (r8 ^ g)) * 16, (64 + g * 8 + (r8 ^ (g | 4))) * 16};  // (MR = 8: lo / 2)
   auto consume = [&](int it, CmGroup<INT4> (&gr)[NG]) {
     if (w0 + it >= w1) return;
-    const unsigned char *xb = &xs[it & 1][part][(g * MR + (MR == 8 ? (r & 7) : r)) * 16];
+    const unsigned char *xb = xs[XB == 2 ? it & 1 : 0][part];
     gq_f4 wa[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) wa[t] = gq_f4{0.f, 0.f, 0.f, 0.f};
@@ -537,10 +574,11 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
       sv[3] = sv[2];
       cm_swap16(sv[0], sv[1]);
       cm_swap16(sv[2], sv[3]);
-      uint32_t q[4][2];
+      // lane group g: codes 8 g .. 8 g + 7 of each group (INT8: in the swap's order)
+      uint32_t q[4][INT4 ? 1 : 2];
       if constexpr (INT4) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[e][0] = gr[j].q[0][e] ^ 0x88888888u;  // code + 8
+        for (int e = 0; e < 4; ++e) q[e][0] = gr[j].q[0][e];
         cm_swap32(q[0][0], q[2][0]);
         cm_swap32(q[1][0], q[3][0]);
         cm_swap16(q[0][0], q[1][0]);
@@ -550,44 +588,65 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
         for (int h = 0; h < 2; ++h)
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
-            q[2 * h][e] = gr[j].q[h][e] ^ 0x80808080u;  // code + 128
-            q[2 * h + 1][e] = gr[j].q[h][2 + e] ^ 0x80808080u;
+            q[2 * h][e] = gr[j].q[h][e];
+            q[2 * h + 1][e] = gr[j].q[h][2 + e];
             cm_swap32(q[2 * h][e], q[2 * h + 1][e]);
           }
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        gq_half2 p[4];
-        if constexpr (INT4) {
-          gq_nib_halves(q[i][0], mg, p);
+        const unsigned char *xg = xb + (4 * j + i) * GB + xo[i & 1];
+        const float s = (i & 1) ? -__uint_as_float(sv[i]) : __uint_as_float(sv[i]);
+        gq_f4 d[MT];
+        if constexpr (F32) {
+          cm_bf8 bf;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            p[e] = p[e] + ((e & 1) ? gq_half2{(_Float16)-1152.f, (_Float16)-1152.f}
-                                   : gq_half2{(_Float16)-1032.f, (_Float16)-1032.f});
+          for (int e = 0; e < 8; ++e) {
+            float f;
+            if constexpr (INT4) f = __builtin_amdgcn_cvt_off_f32_i4((int)(q[i][0] >> (4 * e)));  // code / 16
+            else f = (float)(int8_t)(q[i][e >> 2] >> (8 * (e & 3)));
+            bf[e] = (__bf16)((i & 1) ? -f : f);
+          }
+          auto rd = [&](const unsigned char *at) { return *reinterpret_cast<const cm_bf8 *>(at); };
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            const gq_f4 z = gq_f4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (MR == 8) {
+              d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rd(xb + (4 * j + i) * GB + xl[i & 1]), bf, z, 0, 0, 0);
+            } else {
+              d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rd(xg + 2 * MID + 256 * t), bf, z, 0, 0, 0);
+              d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rd(xg + MID + 256 * t), bf, d[t], 0, 0, 0);
+            }
+            d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rd(xg + 256 * t), bf, d[t], 0, 0, 0);
+          }
         } else {
+          gq_half2 p[4];
+          // (1024 + u, 1024 + 16 u) -> u - 8, u = code + 8
+          gq_nib_halves(q[i][0] ^ 0x88888888u, mg, p);
+          const gq_half2 b1 = {(_Float16)-1032.f, (_Float16)-1032.f}, b16 = {(_Float16)-72.f, (_Float16)-72.f};
+          const gq_half2 k16 = {(_Float16)0.0625f, (_Float16)0.0625f};
+          gq_half8 bf;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            p[e] = gq_bits_h2(__builtin_amdgcn_perm(0x64646464u, q[i][e >> 1], (e & 1) ? 0x04030402u : 0x04010400u)) +
-                   gq_half2{(_Float16)-1152.f, (_Float16)-1152.f};
+          for (int e = 0; e < 4; ++e) {
+            const gq_half2 v = (e & 1) ? __builtin_elementwise_fma(p[e], k16, b16) : p[e] + b1;
+            bf[2 * e] = (i & 1) ? -v[0] : v[0];
+            bf[2 * e + 1] = (i & 1) ? -v[1] : v[1];
+          }
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            d[t] = gq_mfma16(*reinterpret_cast<const gq_half8 *>(xg + 256 * t), bf, gq_f4{0.f, 0.f, 0.f, 0.f});
         }
-        gq_half8 bf;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) bf[e] = p[e >> 1][e & 1];
-        const float s = __uint_as_float(sv[i]);
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          const unsigned char *x = xb + ((4 * j + i) * 4 * MR + 16 * t) * 16;
-          gq_f4 d = gq_f4{0.f, 0.f, 0.f, 0.f};
-          if constexpr (L == 2) d = gq_mfma16(*reinterpret_cast<const gq_half8 *>(x + LB), bf, d);
-          d = gq_mfma16(*reinterpret_cast<const gq_half8 *>(x), bf, d);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) wa[t][v] = fmaf((i & 1) ? -s : s, d[v], wa[t][v]);
-        }
+          for (int v = 0; v < 4; ++v) wa[t][v] = fmaf(s, d[t][v], wa[t][v]);
       }
     }
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      const gq_f4 us = *reinterpret_cast<const gq_f4 *>(&xsc[it & 1][part * MR + 16 * t + ((4 * g) & (MR - 1) & 15)]);
+      gq_f4 us = gq_f4{1.f, 1.f, 1.f, 1.f};
+      if constexpr (F32)
+        us = *reinterpret_cast<const gq_f4 *>(&xsc[XB == 2 ? it & 1 : 0][part * MR + 16 * t + ((4 * g) & (MR - 1) & 15)]);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const float y = fmaf(wa[t][v], us[v], -comp[t][v]), z = acc[t][v] + y;
@@ -610,6 +669,7 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
     load_x(it + 1);
     load_win(w0 + it + 2, nxt);
     consume(it, cur);
+    if constexpr (XB == 1) __syncthreads();  // (every wave has read the window)
     store_x((it + 1) & 1);
     __syncthreads();
   };
@@ -619,6 +679,10 @@ k_compat_mfma(const TA *__restrict__ a, const uint8_t *__restrict__ b, float *__
     window(it + 1, b1, b0);
     if (it + 2 >= NI) break;
     window(it + 2, b2, b1);
+  }
+  if constexpr (F32 && MR == 8) {  // (D rows 8..15, lane groups 2 and 3: the mid limbs' of rows 0..7)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[0][v] += __shfl_xor(acc[0][v], 32, 64);
   }
   // the parts' sums through LDS, added in part order
   gq_f4 *red = reinterpret_cast<gq_f4 *>(&xs[0][0][0]);  // [KS][TW][MT][64]
@@ -673,21 +737,25 @@ int launch_cm(hipStream_t s, const TA *a, const uint8_t *b, float *c, const floa
 }
 // Whether the matrix-core form takes a shape: where the VALU kernels' time,
 // which grows with M N K, passes the matrix cores' start-up (int4, VALU / matrix
-// cores in us: 2 / 8 / 32 rows of 4096 x 4096 8.3 / 13.7 / 49.8 against 10.9 / 11.3 /
-// 18.6, of 1024 x 4096 8.3 / 8.3 / 13.1 against 11.2 / 11.1 / 17.6, of 4096 x 14336
-// 21.8 / 75 / 284 against 24.0 / 24.5 / 35.6, of 7000 x 1120 8.1 / 15.5 / 50 against
-// 8.3 / 8.3 / 14.4)
+// cores in us: 3 / 5 / 8 / 32 rows of 4096 x 4096 8.4 / 12.6 / 13.2 / 44.7 against 10.7 /
+// 10.8 / 10.9 / 18.0, 8 / 32 rows of 1024 x 4096 7.0 / 13.0 against 10.5 / 16.8, 3 rows of
+// 14336 x 4096 25.1 against 18.5; K <= 2048: 4 / 8 rows of 4096 x 2048 5.5 / 9.2 against 7.9 /
+// 8.1, of 7000 x 1120 8.5 / 15.7 against 8.2 / 8.3; K <= 8192: 8 / 16 / 32 rows of 1024 x
+// 6144 7.3 / 12.3 / 22.0 against 13.5 / 17.8 / 18.0, 4 / 5 rows of 4096 x 8192 17.5 / 23.8
+// against 18.0; longer: 4 / 8 / 16 rows of 1024 x 14336 10.4 / 18.5 / 33.9 against 18.1 / 18.3 /
+// 17.4.  The start-up grows with K: from 1024 x 6144 on a workgroup or two per CU
+// walk several windows; past K = 8192 K goes over workgroups and it stops growing)
 bool cm_takes(int M, int N, int K) {
   const double mnk = (double)M * N * K;
   const double from = K <= 2048 ? 40e6 : K <= 4096 && N >= 4096 ? 120e6 : K <= 8192 ? 160e6 : 120e6;
-  return M >= 3 && mnk >= from;  // (two rows are one pass of the VALU kernels: 12.4 against 22.3 us, 20000 x 2048)
+  return M >= 3 && mnk >= from;  // (two rows are one pass of the VALU kernels: 11.0 against 12.4 us, 14336 x 2048)
 }
 // Row tiles per workgroup and parts of K inside it (TW, KS) as the fp16 batch
 // GEMV's plan; few row tiles on a long K, or more than 16 rows, take K in parts
 // over workgroups as well (kz, sums in scratch): four row tiles then share the
-// activations' limbs, whose reads otherwise outweigh the weights (16 rows of
-// 4096 x 14336 43 -> 26 us, 32 rows of 4096 x 4096 31.6 -> 18.6; 8 rows of 4096 x
-// 4096 11.3 -> 17, so not there).
+// activations' limbs, whose making and reads otherwise outweigh the weights
+// (int4, without / with: 16 rows of 4096 x 14336 38.3 / 26.9 us, 32 rows of 4096 x 4096
+// 25.7 / 18.4, of 4096 x 14336 73.9 / 35.3; 8 rows of 4096 x 8192 18.3 / 19.1).
 template <typename TA, bool INT4, int MR, int WIN>
 int launch_cm_kz(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M, int N,
                  int K, int lda, int ldc, int hd) {
@@ -714,7 +782,7 @@ int launch_cm_plan(hipStream_t s, const TA *a, const uint8_t *b, float *c, const
   }
   if (MR == 32 || tiles >= 800) {
     // a 16-wave workgroup fills a CU: beyond one each, 8 waves, two to a CU
-    // (8 rows, INT4: 20000 x 2048 22.5 -> 18.1 us, 28672 x 8192 63.8 -> 56.9)
+    // (int4: 8 rows of 20000 x 2048 23.1 -> 19.2 us, of 28672 x 8192 63.5 -> 55.0; 32 rows 36.2 -> 29.5, 113 -> 102)
     if (nw >= 2 && wgs > 256) GQ_CM(4, 2);
     if (nw >= 4) GQ_CM(4, 4);
     GQ_CM(4, 1);

@@ -86,6 +86,61 @@ def test_wide_range_and_nonfinite_rows(dev, int4):
     assert bool(torch.isnan(c[4]).all())
 
 
+@pytest.mark.parametrize("int4,f16", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(8, 4112, 4096), (13, 4112, 4128), (32, 2000, 8224), (8, 13000, 1056)])
+def test_outlier_under_a_zero_code(dev, int4, f16, m, n, k):
+    """One entry of each row far above the others, in a column whose codes are 0:
+    the others count in full.  (fp16 activations: the others mostly subnormal.)"""
+    import torch
+    a, q, sc, hs, _ = _case(int4, m, n, k, m + n, f16=f16)
+    w = torch.stack([q & 15, q >> 4], 2).reshape(n, k).to(torch.int16).add_(8).bitwise_and_(15).sub_(8) if int4 else q.clone()
+    col = torch.arange(m, device="cuda") * 37 % k
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(n)).cuda()
+    if f16:
+        a = (a * 2.0**-16).half()   # mostly subnormal
+        big = torch.full((m,), 60000.0, device="cuda")
+    else:
+        big = 10.0 ** (4 + torch.arange(m, device="cuda") % 9).float()
+    a[torch.arange(m, device="cuda"), col] = big.to(a.dtype)
+    w[:, col] = 0
+    if int4:
+        u = (w & 15).to(torch.uint8)
+        q = (u[:, 0::2] | (u[:, 1::2] << 4)).contiguous()
+    else:
+        q = w.contiguous()
+    wd = (w.double().reshape(n, k // 32, 32) * sc.double().reshape(n, k // 32, 1)).reshape(n, k)
+    ref = a.double() @ wd.t()
+    if int4:
+        ref = ref * hs.double()[torch.arange(n, device="cuda") // 7]
+    c = _run(int4, a, q, sc, hs, m, n, k)
+    err = (c.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= TOL, err
+
+
+@pytest.mark.parametrize("int4", [True, False])
+@pytest.mark.parametrize("m,n,k", [(8, 4112, 4096), (16, 4112, 4096), (32, 4112, 4096)])
+def test_tiny_windows(dev, int4, m, n, k):
+    """Windows of a row down to fp32's smallest normal values beside windows of
+    zeros and of each other's sizes: every row's sum as its largest window's."""
+    import torch
+    a, q, sc, hs, _ = _case(int4, m, n, k, 31)
+    w = torch.stack([q & 15, q >> 4], 2).reshape(n, k).to(torch.int16).add_(8).bitwise_and_(15).sub_(8) if int4 else q
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(n)).cuda()
+    for row in range(m):
+        a[row] *= 2.0 ** -(8 * row % 124)
+        a[row, 256 * (row % 8):256 * (row % 8) + 256] *= 2.0**-40
+        a[row, 3000:3000 + 20 * row] = 0.0
+    a[a.abs() < 2.0**-126] = 0.0
+    wd = (w.double().reshape(n, k // 32, 32) * sc.double().reshape(n, k // 32, 1)).reshape(n, k)
+    ref = a.double() @ wd.t()
+    if int4:
+        ref = ref * hs.double()[torch.arange(n, device="cuda") // 7]
+    c = _run(int4, a, q, sc, hs, m, n, k).double()
+    up = 2.0**60
+    err = ((c - ref) * up).norm(dim=1) / (ref * up).norm(dim=1)
+    assert float(err.max()) <= TOL, err
+
+
 def test_captured_without_scratch(dev):
     import torch
     m, n, k = 16, 2000, 14336
