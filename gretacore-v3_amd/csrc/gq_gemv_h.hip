@@ -382,7 +382,9 @@ constexpr int kWin = 256;
 // (g, r).  The KS parts' partial sums are reduced in LDS at the end.  MR
 // activation rows are staged, as in k_gemv_h1 (MR = 8 up to batch 8: A rows
 // 8..15 re-read rows 0..7, their D rows are never stored).
-template <int FMT, int TW, int KS, int MR>
+// SP: K in parts over workgroups too (blockIdx.y); a template parameter, since its
+// scalar work cost the other launches 0.1-0.3 us each.
+template <int FMT, int TW, int KS, int MR, bool SP = false>
 __global__ void __launch_bounds__(64 * TW * KS)
 k_gemv_h(const uint8_t *__restrict__ w, size_t sc_off, const float *__restrict__ x, float *__restrict__ y, int N,
          int K, int C, int nb, int NI) {
@@ -402,9 +404,10 @@ k_gemv_h(const uint8_t *__restrict__ w, size_t sc_off, const float *__restrict__
   const int ntiles = (int)gq_tiles(N);
   const size_t tile = (size_t)blockIdx.x * TW + tt;
   const HSrc<FMT> src = hsrc<FMT>(w, sc_off, tile < (size_t)ntiles ? tile : (size_t)ntiles - 1, C, N, K, lane);
-  // K part blockIdx.y over workgroups: Cz chunks from zc, its own nb x N of y
-  const int zc = C * (int)blockIdx.y / (int)gridDim.y, Cz = C * ((int)blockIdx.y + 1) / (int)gridDim.y - zc;
-  y += (size_t)blockIdx.y * (size_t)nb * (size_t)N;
+  // this workgroup's Cz chunks from zc; a part writes its own nb x N of y
+  const int zc = SP ? C * (int)blockIdx.y / (int)gridDim.y : 0;
+  const int Cz = SP ? C * ((int)blockIdx.y + 1) / (int)gridDim.y - zc : C;
+  if constexpr (SP) y += (size_t)blockIdx.y * (size_t)nb * (size_t)N;
   const int c0 = zc + (Cz * part) / KS, c1 = zc + (Cz * (part + 1)) / KS;  // this wave's chunks (c0 < c1: KS <= Cz)
 
   // weights of window `it` (chunks past the part re-read its last chunk)
@@ -963,17 +966,17 @@ int gq_gemv_h_plan(int fmt, size_t N, size_t K, int nb, int *R_out, int *ks_out,
 
 namespace {
 template <int FMT, int TW, int MR>
-int launch_h_tw(const void *packed, const float *x, float *y, int N, int K, int nb, int ks, hipStream_t s, int kz = 1) {
+int launch_h_tw(const void *packed, const float *x, float *y, int N, int K, int nb, int ks, hipStream_t s) {
   const int C = (int)gq_chunks(FMT, K);
   const size_t wgs = (gq_tiles(N) + TW - 1) / TW;
   const size_t sc_off = gq_sc_plane_offset(FMT, N, K);
   const uint8_t *w = (const uint8_t *)packed;
   constexpr int WC = kWin / HFmt<FMT>::CK;
-  const int NI = (((C + kz - 1) / kz + ks - 1) / ks + WC - 1) / WC;
+  const int NI = ((C + ks - 1) / ks + WC - 1) / WC;
   // x runs must spread evenly over the threads (TW <= MR / 2)
 #define GQ_LAUNCH_H(KS)                                                                                               \
   if constexpr (2 * TW <= MR && !(FMT == GQ_FMT_F16 && TW * KS > 8)) {                                               \
-    hipLaunchKernelGGL((k_gemv_h<FMT, TW, KS, MR>), dim3((unsigned)wgs, (unsigned)kz), dim3(64 * TW * KS), 0, s, w, sc_off, x, y, \
+    hipLaunchKernelGGL((k_gemv_h<FMT, TW, KS, MR>), dim3((unsigned)wgs), dim3(64 * TW * KS), 0, s, w, sc_off, x, y, \
                        N, K, C, nb, NI);                                                                              \
   } else {                                                                                                            \
     return GQ_ERR_INVALID_ARGS;                                                                                       \
@@ -1035,7 +1038,11 @@ int launch_h_kz(const void *packed, const float *x, float *y, int N, int K, int 
   if (nb <= 8 || kz <= 1 || !pays) return GQ_ERR_UNSUPPORTED;
   GqScratch ws((size_t)kz * nb * N * 4, s);
   if (!ws.ptr) return GQ_ERR_UNSUPPORTED;
-  GQ_TRY((launch_h_tw<FMT, 4, 16>(packed, x, (float *)ws.ptr, N, K, nb, 4, s, kz)));
+  constexpr int WC = kWin / HFmt<FMT>::CK;
+  const int NI = (((C + kz - 1) / kz + 3) / 4 + WC - 1) / WC;
+  hipLaunchKernelGGL((k_gemv_h<FMT, 4, 4, 16, true>), dim3((unsigned)wgs, (unsigned)kz), dim3(64 * 16), 0, s,
+                     (const uint8_t *)packed, gq_sc_plane_offset(FMT, N, K), x, (float *)ws.ptr, N, K, C, nb, NI);
+  GQ_TRY(gq_last_launch());
   return gq_launch_split_sum((const float *)ws.ptr, y, (size_t)nb * N, kz, s);
 }
 
