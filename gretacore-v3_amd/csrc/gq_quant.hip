@@ -160,8 +160,10 @@ k_dequant_t16(int fmt, const uint8_t *__restrict__ w, float *__restrict__ out, i
 // records' order, so loads and stores are both coalesced and no code is touched
 // byte by byte.  14336 x 4096 Q4_K: 110 us with one thread per block (144-byte
 // strides, byte loads) -> 12.4 us; Q6_K 982 -> 16.8 us; 128256 x 4096 Q6_K 12.8 ms -> 150 us
-// (5.7 TB/s read and written).  Positions outside the tensor (rows
-// past N, blocks past K) become zeros in LDS, so no memset is needed.
+// (5.7 TB/s read and written).  A row's last, partial span goes the same way
+// up to its last whole 16 bytes (by byte pairs alone, 128256 x 256 took 23.7 us
+// in Q4_0 and 35 in Q8_0, one thread per block 8.1 and 20.7).  Positions outside
+// the tensor (rows past N, blocks past K) become zeros in LDS, so no memset is needed.
 // ---------------------------------------------------------------------------
 template <int FMT>
 struct RpFmt;  // per row and chunk: GGUF bytes; 16-byte pieces of the code record and of the scale record
@@ -251,19 +253,19 @@ GQ_DEV uint32_t rp_hi(const uint8_t *p, int o, int j, int eh, int ggml) {
   return h;
 }
 
-template <int FMT>
-__global__ void __launch_bounds__(256)
+template <int FMT, int kSpan = RpFmt<FMT>::kSpan, int NT = 256>
+__global__ void __launch_bounds__(NT)
 k_repack(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t sc_off, int N, size_t row_bytes, int C,
          int row0, int ggml) {
   using F = RpFmt<FMT>;
-  constexpr int SEG = F::kBytes * F::kSpan;        // a multiple of 8
+  constexpr int SEG = F::kBytes * kSpan;        // a multiple of 8
   constexpr int UPR = (SEG + 15) / 16;             // 16-byte loads per row
   constexpr int PITCH = (UPR * 4 + 2) * 4 + 4;     // an odd count of dwords: the 16 rows on different banks
   static_assert((PITCH / 4) % 2 == 1 && PITCH >= UPR * 16 + 4, "LDS pitch");
-  constexpr int LD = (16 * UPR + 255) / 256;
+  constexpr int LD = (16 * UPR + NT - 1) / NT;
   __shared__ __attribute__((aligned(16))) uint8_t seg[16 * PITCH];
-  const int nsp = (C + F::kSpan - 1) / F::kSpan;
-  const int t = (int)(blockIdx.x / (unsigned)nsp), c0 = (int)(blockIdx.x % (unsigned)nsp) * F::kSpan;  // tile of the slice
+  const int nsp = (C + kSpan - 1) / kSpan;
+  const int t = (int)(blockIdx.x / (unsigned)nsp), c0 = (int)(blockIdx.x % (unsigned)nsp) * kSpan;  // tile of the slice
   const int tid = threadIdx.x;
   const int nrows = min(16, N - (row0 + 16 * t));  // rows inside the tensor (>= 1)
   const size_t sb = (size_t)c0 * F::kBytes;
@@ -275,12 +277,12 @@ k_repack(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t sc_o
     gq_u4 v[LD];
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int i = tid + 256 * q, row = min(i / UPR, nrows - 1), o = min(16 * (i % UPR), SEG - 16);
+      const int i = tid + NT * q, row = min(i / UPR, nrows - 1), o = min(16 * (i % UPR), SEG - 16);
       v[q] = reinterpret_cast<const RpLoad16 *>(base + (size_t)row * row_bytes + o)->v;
     }
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int i = tid + 256 * q, row = i / UPR, o = min(16 * (i % UPR), SEG - 16);
+      const int i = tid + NT * q, row = i / UPR, o = min(16 * (i % UPR), SEG - 16);
       if (row < 16) {
         uint32_t *d = reinterpret_cast<uint32_t *>(seg + row * PITCH + o);
 #pragma unroll
@@ -288,22 +290,39 @@ k_repack(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t sc_o
       }
     }
   } else {
-    // the row's end: byte pairs, zeros past it
-    for (int i = tid; i < 16 * (SEG / 2); i += 256) {
-      const int row = i / (SEG / 2), o = 2 * (i % (SEG / 2));
-      uint32_t v = 0;
+    // the row's end (a short row's only segment): whole pieces of 16, then byte
+    // pairs, zeros past the row up to the last chunk's end
+    const int full = (int)left >> 4, end = min(kSpan, C - c0) * F::kBytes;
+    gq_u4 v[LD];
+#pragma unroll
+    for (int q = 0; q < LD; ++q) {
+      const int i = tid + NT * q, row = min(i / UPR, nrows - 1), u = min(i % UPR, full - 1);
+      if (full > 0) v[q] = reinterpret_cast<const RpLoad16 *>(base + (size_t)row * row_bytes + 16 * u)->v;
+    }
+#pragma unroll
+    for (int q = 0; q < LD; ++q) {
+      const int i = tid + NT * q, row = i / UPR, u = i % UPR;
+      if (row < 16 && u < full) {
+        uint32_t *d = reinterpret_cast<uint32_t *>(seg + row * PITCH + 16 * u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[e] = row < nrows ? v[q][e] : 0u;
+      }
+    }
+    for (int i = tid >> 4; i < (end >> 1) - 8 * full; i += NT / 16) {
+      const int row = tid & 15, o = 16 * full + 2 * i;
+      uint32_t x = 0;
       if (row < nrows && (size_t)o + 2 <= left) {
         const uint8_t *p = base + (size_t)row * row_bytes + o;
-        v = (uint32_t)p[0] | ((uint32_t)p[1] << 8);
+        x = (uint32_t)p[0] | ((uint32_t)p[1] << 8);
       }
-      *reinterpret_cast<uint16_t *>(seg + row * PITCH + o) = (uint16_t)v;
+      *reinterpret_cast<uint16_t *>(seg + row * PITCH + o) = (uint16_t)x;
     }
   }
   __syncthreads();
-  const int nc = min(F::kSpan, C - c0);
+  const int nc = min(kSpan, C - c0);
   const size_t tc = (size_t)(row0 / 16 + t) * (size_t)C + (size_t)c0;
   gq_u4 *qs = reinterpret_cast<gq_u4 *>(dst + tc * (16 * F::kQs));
-  for (int i = tid; i < nc * F::kQs; i += 256) {
+  for (int i = tid; i < nc * F::kQs; i += NT) {
     const int c = i / F::kQs, pc = i % F::kQs, l = pc & 63, part = pc >> 6;
     const int r = l & 15, g = l >> 4, eh = g & 1, jh = g >> 1;
     const uint8_t *p = seg + r * PITCH;
@@ -324,7 +343,7 @@ k_repack(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t sc_o
     qs[i] = v;
   }
   gq_u4 *sc = reinterpret_cast<gq_u4 *>(dst + sc_off + tc * (16 * F::kSc));
-  for (int i = tid; i < nc * F::kSc; i += 256) {
+  for (int i = tid; i < nc * F::kSc; i += NT) {
     const int c = i / F::kSc, pc = i % F::kSc;
     const int o = c * F::kBytes;
     gq_u4 v;
@@ -440,6 +459,15 @@ template <int FMT>
 void launch_repack(const uint8_t *src, uint8_t *dst, size_t N, size_t K, size_t row0, size_t tiles, int ggml,
                    hipStream_t s) {
   const size_t C = gq_chunks(FMT, K), nsp = (C + RpFmt<FMT>::kSpan - 1) / RpFmt<FMT>::kSpan;
+  // one or two chunks a row leave a workgroup little: one wave takes them
+  // (128256 x 256, Q4_0 10.4 -> 6.9 us, Q8_0 13.4 -> 12.8)
+  if constexpr (FMT == GQ_FMT_Q4_0 || FMT == GQ_FMT_Q8_0) {
+    if (C <= 2) {
+      hipLaunchKernelGGL((k_repack<FMT, 2, 64>), dim3((unsigned)tiles), dim3(64), 0, s, src, dst,
+                         gq_sc_plane_offset(FMT, N, K), (int)N, gq_layout_gguf_bytes(FMT, 1, K), (int)C, (int)row0, ggml);
+      return;
+    }
+  }
   hipLaunchKernelGGL(k_repack<FMT>, dim3((unsigned)(tiles * nsp)), dim3(256), 0, s, src, dst,
                      gq_sc_plane_offset(FMT, N, K), (int)N, gq_layout_gguf_bytes(FMT, 1, K), (int)C, (int)row0, ggml);
 }

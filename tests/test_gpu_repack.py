@@ -23,3 +23,21 @@ def test_repack_spans(dev, fmt, n, spans):
             src[shift:] = torch.from_numpy(w).to(dev)
             got = gq.repack(fmt, src[shift:], n, k).cpu().numpy()
             assert np.array_equal(got, host), (k, shift)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("n", [1, 16, 35])
+def test_repack_short_and_partial_rows(dev, fmt, n):
+    """Rows of one or two chunks, and last spans of every length in blocks."""
+    import gq
+    import torch
+    step = 32 if fmt in (O.Q4_0, O.Q8_0) else 256
+    for k in range(step, 36 * step if step == 32 else 9 * step, step):
+        w = O.gen_weights(fmt, n, k, seed=n + k)
+        host = gq.repack_host(fmt, w, n, k)
+        shift = (k // step) % 3
+        # bytes after the rows that must not be taken in
+        src = torch.full((w.size + shift + 64,), 0xA5, dtype=torch.uint8, device=dev)
+        src[shift:shift + w.size] = torch.from_numpy(w).to(dev)
+        got = gq.repack(fmt, src[shift:shift + w.size], n, k).cpu().numpy()
+        assert np.array_equal(got, host), (k, shift)
