@@ -1209,11 +1209,24 @@ int gq_gemm_skinny_plan(int fmt, size_t M, size_t N, size_t K, int *ct_out, int 
   // is (4096 x 4096 at 64 / 128 rows: 15.6 / 17.5 vs 20-23 us)
   // (GQ_GEMM_SKINNY=2: up to two per CU, for tuning)
   const size_t lim = (nckp >= 16 || (e && e[0] == '2')) ? 2 * cus : cus;
-  // Q6_K stays here for up to 40 rows, whose one row block reads the weights
-  // once either way (17 x 14336 x 4096: 22.5 us against 28.4 tiled; 48 rows: 29.3
-  // against 29.2), and where the tiled kernel's 32-bit activation offsets end
-  const bool q6_any = q6 && (M <= 40 || M * gq_kpad(fmt, K) * 2 >= ((size_t)1 << 32));
-  if (!q6_any && wgs > lim) return GQ_ERR_UNSUPPORTED;
+  // Q6_K, whose tiled kernel takes about 9 us + 5.2 us per 1024 k for few
+  // workgroups, stays here longer (skinny / tiled, us):
+  //  - up to 40 rows, whose one row block reads the weights once either way (17 x
+  //    14336 x 4096: 22.5 / 28.4), and where the tiled kernel's 32-bit activation
+  //    offsets end;
+  //  - while its work, in 16-row blocks, is one round (130 x 1400 x 3072 / 4096: 16.6 /
+  //    24.8, 16.0 / 29.9);
+  //  - in two rounds where its 8 waves' chunks are mostly full: K near 2048 or 4096 (41 x
+  //    14336 17.3 / 19.3, 28.0 / 33.6; 300 x 1024 15.2 / 20.3, 25.9 / 31.2), or from 1024
+  //    on single row tiles (300 x 1024 x 1024 12.3 / 14.9).  300 x 1024 x 256 / 3072 12.0 /
+  //    10.9, 26.7 / 25.9, 300 x 1900 x 1024 15.5 / 15.0, 1500 x 200 x 2048 23.9 / 22.7: not.
+  auto q6_stays = [&] {
+    const size_t gy16 = (M + 15) / 16;
+    if (M <= 40 || M * gq_kpad(fmt, K) * 2 >= ((size_t)1 << 32)) return true;
+    if (C >= 2 && ct == 1 && tiles * gy16 <= 4 * cus) return true;
+    return wgs <= 2 * cus && gy <= 12 && (nckp == 1 ? C >= 8 || (C >= 4 && ct == 1) : C >= 14);
+  };
+  if (wgs > lim && !(q6 && q6_stays())) return GQ_ERR_UNSUPPORTED;
   *ct_out = ct;
   *nck_out = nckp;
   return GQ_OK;

@@ -43,6 +43,22 @@ def test_q6k_tiled_gemm(dev, fmt, m, n, k):
     assert torch.equal(cb, c.bfloat16())
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (130, 1400, 3072), (130, 1400, 256),    # one round of 16-row blocks; one chunk
+    (41, 8200, 2048), (64, 8200, 4096),     # two rounds, full chunks
+    (300, 832, 1024), (300, 1024, 3072),    # single row tiles; chunks three quarters full
+    (1000, 300, 4096), (40, 20000, 256),    # more than 12 row blocks; up to 40 rows
+])
+def test_q6k_gemm_skinny_or_tiled(dev, m, n, k):
+    """Both sides of the limits between the skinny and the tiled kernel."""
+    import gq
+    import torch
+    w = O.gen_weights(O.Q6_K, n, k, seed=n)
+    packed = torch.from_numpy(gq.repack_host(O.Q6_K, w, n, k)).to(dev)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dev)
+    assert _rel(gq.gemm(O.Q6_K, packed, a, n, k), _ref(O.Q6_K, w, a, n, k)) <= TOL
+
+
 @pytest.mark.parametrize("m,n,k", [(49, 33, 4352), (33, 8192, 4352), (130, 8200, 4608), (300, 100, 14336)])
 def test_q6k_matmul_long_k(dev, m, n, k):
     """K > 4096: the tiled kernel on scratch memory, the 16-row GEMVs under
