@@ -755,7 +755,8 @@ bool cm_takes(int M, int N, int K) {
 // over workgroups as well (kz, sums in scratch): four row tiles then share the
 // activations' limbs, whose making and reads otherwise outweigh the weights
 // (int4, without / with: 16 rows of 4096 x 14336 38.3 / 26.9 us, 32 rows of 4096 x 4096
-// 25.7 / 18.4, of 4096 x 14336 73.9 / 35.3; 8 rows of 4096 x 8192 18.3 / 19.1).
+// 25.7 / 18.4, of 4096 x 14336 73.9 / 35.3; 8 rows of 4096 x 8192 18.3 / 19.1; 32 rows of
+// 1024 x 2048, two parts, 8.5 / 16.3: the second launch is not worth two).
 template <typename TA, bool INT4, int MR, int WIN>
 int launch_cm_kz(hipStream_t s, const TA *a, const uint8_t *b, float *c, const float *sc, const float *hs, int M, int N,
                  int K, int lda, int ldc, int hd) {
@@ -763,7 +764,7 @@ int launch_cm_kz(hipStream_t s, const TA *a, const uint8_t *b, float *c, const f
   const int nw = (K + WIN - 1) / WIN;
   const long wgs = (long)((tiles + 3) / 4) * ((M + MR - 1) / MR);
   const int kz = (int)(256 / wgs < nw / 8 ? 256 / wgs : nw / 8);
-  if (tiles >= 800 || kz <= 1 || (MR < 32 && K < 8192)) return GQ_ERR_UNSUPPORTED;
+  if (tiles >= 800 || kz <= (K < 4096 ? 2 : 1) || (MR < 32 && K < 8192)) return GQ_ERR_UNSUPPORTED;
   GqScratch ws((size_t)kz * M * N * 4, s);
   if (!ws.ptr) return GQ_ERR_UNSUPPORTED;
   return launch_cm<TA, INT4, MR, WIN, 4, 4>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd, kz, (float *)ws.ptr);
