@@ -357,7 +357,7 @@ k_compat_gemv_lds(const TA *__restrict__ a, const uint8_t *__restrict__ b, float
 //
 // What bounds it is VALU work: a code's way to bf16 (v_cvt_off_f32_i4 or a byte's
 // conversion, and half a packing) and the limbs' making.  14336 x 4096, INT4 / INT8,
-// VALU kernels -> this: 8 rows 44 / 51 -> 19.1 / 25.4 us, 32 rows 155 / 172 -> 31 / 36;
+// VALU kernels -> this: 8 rows 44 / 51 -> 19.1 / 23.6 us, 32 rows 155 / 172 -> 31 / 36;
 // rel-L2 against float64 8.9e-8 at 8 rows (VALU kernels 1.1-1.2e-7).
 //
 // Workgroup: TW row tiles of 16 x KS parts of K, one wave each.  The operands of
@@ -781,16 +781,27 @@ int launch_cm_plan(hipStream_t s, const TA *a, const uint8_t *b, float *c, const
     // (fewer row tiles: 16 rows at a time on smaller workgroups)
     if (tiles < 400) return launch_cm_plan<TA, INT4, 16, WIN>(s, a, b, c, sc, hs, M, N, K, lda, ldc, hd);
   }
-  if (MR == 32 || tiles >= 800) {
-    // a 16-wave workgroup fills a CU: beyond one each, 8 waves, two to a CU
-    // (int4: 8 rows of 20000 x 2048 23.1 -> 19.2 us, of 28672 x 8192 63.5 -> 55.0; 32 rows 36.2 -> 29.5, 113 -> 102)
-    if (nw >= 2 && wgs > 256) GQ_CM(4, 2);
+  // (a 16-wave workgroup fills a CU: two row tiles each past 512 would run in two
+  // rounds; 9000 x 4096, two / four tiles: 4 / 8 / 16 rows int4 26.0 / 26.6 / 30.3 -> 18.0 / 19.0 /
+  // 21.3 us, int8 38.5 / 38.7 / 33.5 -> 22.3 / 22.7 / 25.0)
+  if (MR == 32 || tiles > 512) {
+    // 8 waves, two workgroups to a CU, beyond one 16-wave workgroup each (int4: 8 rows
+    // of 20000 x 2048 23.1 -> 19.2 us, of 28672 x 8192 63.5 -> 55.0; 32 rows 36.2 -> 29.5, 113 ->
+    // 102) and, up to 8 rows, on a K whose walk is short (8 rows of 14336 x 1024 / 2048 / 4096 /
+    // 6144 / 14336, 16 / 8 waves: int4 8.9 / 8.0, 12.9 / 11.9, 19.1 / 19.1, 27.0 / 27.6, 53 / 56; int8
+    // 12.2 / 10.2, 16.6 / 14.3, 25.3 / 23.6, 35.0 / 33.7, 69.9 / 69.6)
+    const bool short_walk = MR == 8 && K <= (INT4 ? 2048 : 6144);
+    if (nw >= 2 && (wgs > 256 || short_walk)) GQ_CM(4, 2);
     if (nw >= 4) GQ_CM(4, 4);
     GQ_CM(4, 1);
   }
   if constexpr (MR < 32) {
     if (tiles >= 400) {
-      if (nw >= 8) GQ_CM(2, 8);
+      // (up to 8 rows the 16 waves' budget of 128 registers spills: 6400 x 4096, 16 / 8
+      // waves, int4 14.3 / 13.7, int8 20.8 / 16.0; 16 rows 16.3 / 17.7)
+      if constexpr (MR == 16) {
+        if (nw >= 8) GQ_CM(2, 8);
+      }
       if (nw >= 4) GQ_CM(2, 4);
       GQ_CM(2, 1);
     }

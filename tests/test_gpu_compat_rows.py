@@ -39,18 +39,37 @@ def _rel(c, ref):
     return float((c.double() - ref).norm() / ref.norm())
 
 
+# Shapes of every launch of the matrix-core form (row tiles of 16 x parts of K a
+# workgroup; activation rows): ragged last tiles, K that ends inside a window
+SHAPES = [
+    (2, 14337, 2080),   # (two rows: the VALU kernels)
+    (8, 14337, 2080), (8, 16500, 544),  # 4 x 2, 8 rows: a short K; more workgroups than CUs
+    (8, 8300, 6272),    # 4 x 4, 8 rows, the last workgroup of three tiles
+    (8, 20001, 256),    # 4 x 1, one window
+    (8, 7001, 800), (8, 7001, 736),     # 2 x 4; 2 x 1: fewer windows than K parts
+    (8, 4100, 4096), (8, 6001, 1056),   # 1 x 8, 1 x 4
+    (3, 3001, 14304),   # 8 rows, K in parts over workgroups
+    (12, 16500, 544), (9, 14337, 2080), (16, 14337, 352),  # 16 rows, four row tiles: 4 x 2, 4 x 4, 4 x 1
+    (16, 7001, 1056), (16, 7001, 800), (16, 7001, 384),    # two row tiles: 2 x 8, 2 x 4, 2 x 1
+    (9, 4100, 1248), (16, 3000, 4128), (16, 6001, 800), (32, 6001, 352),  # one row tile: 1 x 8 twice, 1 x 4, 1 x 1
+    (16, 3000, 14304),  # 16 rows, K in parts over workgroups
+    (17, 16500, 544), (31, 14336, 96), (32, 6500, 992),    # 32 rows: 4 x 2, 4 x 1, 4 x 4
+    (17, 4097, 4096), (32, 1500, 8224),  # 32 rows, K in parts over workgroups
+    (32, 1024, 2048),   # ... not in two
+]
+
+
 @pytest.mark.parametrize("int4", [True, False])
-@pytest.mark.parametrize("m,n,k", [
-    (2, 14337, 2080),   # four row tiles, the last of one row; K ends inside a window
-    (8, 7001, 800),     # two row tiles; fewer windows than K parts
-    (9, 4100, 1248), (16, 3000, 4128),   # one row tile
-    (3, 3001, 14304),   # K in parts over workgroups
-    (17, 4097, 4096), (32, 1500, 8224),  # 32 rows
-    (31, 14336, 96), (32, 6500, 992),    # K of a few groups
-])
+@pytest.mark.parametrize("m,n,k", SHAPES)
 def test_rows_match_float64(dev, int4, m, n, k):
     a, q, sc, hs, ref = _case(int4, m, n, k, m + k)
     assert _rel(_run(int4, a, q, sc, hs, m, n, k), ref) <= TOL
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES[1::2])
+def test_rows_of_fp16_activations(dev, m, n, k):
+    a, q, sc, hs, ref = _case(True, m, n, k, m + k, f16=True)
+    assert _rel(_run(True, a, q, sc, hs, m, n, k), ref) <= TOL
 
 
 def test_fp16_activations_and_force_gemv(dev):
