@@ -21,21 +21,24 @@ std::vector<DeviceWorkspace> g_ws;
 std::vector<int> g_cus;
 
 // Scratch blocks of a device.  A block is one call's from its acquisition to
-// the event recorded behind that call's last kernel; a later call waits for
-// the event on its own stream.  (hipMallocAsync / hipFreeAsync do the same but
-// cost 18 us a call.)
+// the event recorded behind that call's last kernel; it passes to a later call on
+// the same stream, or on another one once that event has come to pass.  (No kept
+// block: an allocation of the call's own by hipMallocAsync / hipFreeAsync, 18 us of
+// host time a call where a kept block costs 4.)
 struct ScratchBlock {
   void *ptr = nullptr;
   size_t bytes = 0;
   hipEvent_t done = nullptr;
   hipStream_t last = nullptr;
-  bool busy = false;      // between acquisition and release
+  bool busy = false;      // one thread's: between acquisition and release
   uint64_t used = 0;      // acquisition count at the last use
 };
-constexpr int kScratchBlocks = 4;          // of at most kGqScratchMax bytes each
-constexpr uint64_t kScratchIdle = 4096;    // acquisitions an idle block is kept for
+constexpr int kScratchBlocks = 8;
+constexpr size_t kScratchHeld = 4 * kGqScratchMax;  // bytes kept a device
+constexpr uint64_t kScratchIdle = 4096;             // acquisitions an idle block is kept for
 struct ScratchDevice {
   ScratchBlock block[kScratchBlocks];
+  size_t held = 0;  // bytes of the blocks, and of those being allocated
   uint64_t count = 0;
 };
 std::mutex g_scratch_mutex;
@@ -48,14 +51,11 @@ struct RelaxedCapture {
   RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
-
-void scratch_free(ScratchBlock &b) {  // its work has ended
-  (void)hipFree(b.ptr);
-  b.ptr = nullptr;
-  b.bytes = 0;
-}
 }  // namespace
 
+// The lock is held for the choice alone: no allocation, no release and no wait
+// under it, and none of them waits for the device (memory is freed in the
+// stream's order).
 GqScratch::GqScratch(size_t bytes, hipStream_t s) : stream(s) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   int dev = 0;
@@ -66,66 +66,102 @@ GqScratch::GqScratch(size_t bytes, hipStream_t s) : stream(s) {
     return;
   }
   RelaxedCapture relaxed;
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  if ((size_t)dev >= g_scratch.size()) g_scratch.resize(dev + 1, nullptr);
-  if (!g_scratch[dev]) g_scratch[dev] = new ScratchDevice;
-  ScratchDevice &d = *g_scratch[dev];
-  ++d.count;
-  auto ended = [](const ScratchBlock &b) { return hipEventQuery(b.done) == hipSuccess; };
-  // the block this stream used last (its work is in order already), else one
-  // whose work has ended, else an empty place, else any that is large enough
-  ScratchBlock *best = nullptr;
-  int rank = 0;
-  for (ScratchBlock &b : d.block) {
-    if (b.busy) continue;
-    int r = 1;  // (a smaller block: replaced)
-    if (!b.ptr) r = 3;
-    else if (d.count - b.used > kScratchIdle && ended(b)) {
-      scratch_free(b);
-      r = 3;
-    } else if (b.bytes >= bytes) r = b.last == s ? 5 : ended(b) ? 4 : 2;
-    if (r > rank) {
-      rank = r;
-      best = &b;
+  const size_t want = (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+  ScratchDevice *d = nullptr;
+  ScratchBlock *own = nullptr, *idle = nullptr;  // this call's block; one to be given back
+  void *old = nullptr;                           // what own held, if that is to be replaced
+  size_t old_bytes = 0;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    if ((size_t)dev >= g_scratch.size()) g_scratch.resize(dev + 1, nullptr);
+    if (!g_scratch[dev]) g_scratch[dev] = new ScratchDevice;
+    d = g_scratch[dev];
+    ++d->count;
+    auto free_for = [&](const ScratchBlock &b, bool query) {  // (same stream: in order already)
+      return b.ptr && !b.busy && (query ? hipEventQuery(b.done) == hipSuccess : b.last == s);
+    };
+    // the smallest block that is large enough, this stream's before another's
+    for (int query = 0; query < 2 && !own; ++query)
+      for (ScratchBlock &b : d->block)
+        if (b.bytes >= bytes && (!own || b.bytes < own->bytes) && free_for(b, query)) own = &b;
+    if (!own) {  // a new one in an empty place or in the place of a smaller one
+      for (ScratchBlock &b : d->block)
+        if (!own && !b.busy && !b.ptr && d->held + want <= kScratchHeld) own = &b;
+      for (int query = 0; query < 2 && !own; ++query)
+        for (ScratchBlock &b : d->block)
+          if (!own && d->held - b.bytes + want <= kScratchHeld && free_for(b, query)) own = &b;
+      if (own) {
+        d->held += want - own->bytes;
+        old = own->ptr;
+        old_bytes = own->bytes;
+        own->ptr = nullptr;
+        own->bytes = want;
+      }
     }
+    if (own) {
+      own->busy = true;
+      own->used = d->count;
+    }
+    for (ScratchBlock &b : d->block)
+      if (!idle && b.ptr && !b.busy && d->count - b.used > kScratchIdle && free_for(b, true)) {
+        idle = &b;
+        b.busy = true;
+      }
+    (void)hipGetLastError();  // (queries of running work)
   }
-  if (!best) return;
-  if (best->ptr && best->bytes < bytes) {
-    if (hipEventSynchronize(best->done) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    scratch_free(*best);
+  auto put_back = [&](ScratchBlock *b, void *mem, size_t n) {  // (mem NULL: an empty place)
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    d->held -= b->bytes - n;
+    b->ptr = mem;
+    b->bytes = n;
+    b->busy = false;
+  };
+  if (idle) {
+    if (hipFreeAsync(idle->ptr, s) != hipSuccess) (void)hipGetLastError();  // (its work has ended)
+    put_back(idle, nullptr, 0);
   }
-  if (!best->ptr) {
-    const size_t want = (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
-    if ((!best->done && hipEventCreateWithFlags(&best->done, hipEventDisableTiming) != hipSuccess) ||
-        hipMalloc(&best->ptr, want) != hipSuccess) {
-      best->ptr = nullptr;
+  if (!own) {  // every block in use, or too much held: memory of this call's own
+    if (hipMallocAsync(&ptr, want, s) != hipSuccess) {
       (void)hipGetLastError();
-      return;
+      ptr = nullptr;
     }
-    best->bytes = want;
-  } else if (hipStreamWaitEvent(s, best->done, 0) != hipSuccess) {
-    // (also on the stream that used it last: a stream made anew may have an
-    // old one's handle)
-    (void)hipGetLastError();
     return;
   }
-  (void)hipGetLastError();  // (a query of running work)
-  best->busy = true;
-  best->last = s;
-  best->used = d.count;
-  block = best;
-  ptr = best->ptr;
+  // (the event also on the stream that used the block last: a stream made anew
+  // may have an old one's handle)
+  void *mem = own->ptr;
+  hipError_t e = hipSuccess;
+  if (mem || old) e = hipStreamWaitEvent(s, own->done, 0);
+  if (e == hipSuccess && old && (e = hipFreeAsync(old, s)) == hipSuccess) old = nullptr;
+  if (e == hipSuccess && !mem && !own->done) e = hipEventCreateWithFlags(&own->done, hipEventDisableTiming);
+  if (e == hipSuccess && !mem && (e = hipMallocAsync(&mem, own->bytes, s)) != hipSuccess) mem = nullptr;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    put_back(own, mem ? mem : old, mem ? own->bytes : old ? old_bytes : 0);
+    return;
+  }
+  own->ptr = mem;
+  own->last = s;
+  device = d;
+  block = own;
+  ptr = own->ptr;
 }
 GqScratch::~GqScratch() {
-  if (!block) return;
+  if (!ptr) return;
+  ScratchBlock *b = (ScratchBlock *)block;
+  const bool kept = b && hipEventRecord(b->done, stream) == hipSuccess;
+  if (!kept) {  // given back in the stream's order
+    RelaxedCapture relaxed;
+    if (hipFreeAsync(ptr, stream) != hipSuccess) (void)hipGetLastError();
+    if (!b) return;
+  }
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  ScratchBlock &b = *(ScratchBlock *)block;
-  // without the event the block stays out of use
-  if (hipEventRecord(b.done, stream) == hipSuccess) b.busy = false;
-  else (void)hipGetLastError();
+  if (!kept) {
+    ((ScratchDevice *)device)->held -= b->bytes;
+    b->ptr = nullptr;
+    b->bytes = 0;
+  }
+  b->busy = false;
 }
 
 int gq_hip_status(hipError_t e) {

@@ -74,12 +74,14 @@ int gq_launch_f16_to_f32(const void *in, size_t n, float *out, hipStream_t s);
 // Library-owned per-device workspace (grown on demand, never shrunk).
 int gq_default_workspace(size_t bytes, void **ptr);
 // Scratch memory of one call on stream s, for the kernels launched on s in this
-// object's lifetime.  The blocks are kept (at most four a device, of up to
-// kGqScratchMax bytes; one that is not asked for any more is freed) and pass
-// from call to call behind events, so calls on other streams and threads do
-// not meet.  ptr is NULL where no block is to be had: more than kGqScratchMax
-// asked for, no memory left, all four between acquisition and release, or a
-// stream under capture (the graph would keep the block's address).
+// object's lifetime.  Blocks are kept (at most eight a device, of 4 kGqScratchMax bytes
+// together; one that is not asked for any more is freed) and pass from call to
+// call on one stream, or to another's once the last call's work has ended; a
+// call that finds none has memory allocated in its stream's order.  So no call
+// waits for another stream or thread, on the host or on the device, and which
+// kernels it runs does not depend on them.  ptr is NULL where there is none: more
+// than kGqScratchMax asked for, no memory left, or a stream under capture (the
+// graph would keep the block's address).
 constexpr size_t kGqScratchMax = (size_t)128 << 20;
 struct GqScratch {
   void *ptr = nullptr;
@@ -90,7 +92,7 @@ struct GqScratch {
 
 private:
   hipStream_t stream;
-  void *block = nullptr;
+  void *device = nullptr, *block = nullptr;  // (of the kept blocks; none: memory of this call's own)
 };
 // Q6_K rows of gq_matmul through the tiled GEMM (gq_gemm.hip)
 int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,

@@ -111,6 +111,63 @@ def test_scratch_routes_on_streams(dev):
     assert all(np.array_equal(x.cpu().numpy(), y.cpu().numpy()) for x, y in zip(got, want))
 
 
+@pytest.mark.parametrize("m,n,k", [(100, 500, 5120), (64, 1000, 14336)])  # (the second splits K: two blocks a call)
+def test_scratch_routes_of_many_threads(dev, m, n, k):
+    """Twelve threads on streams of their own: more than blocks are kept.  Each call
+    runs the kernels it runs alone, bit for bit."""
+    import gq
+    import torch
+    w = O.gen_weights(O.Q6_K, n, k, seed=1)
+    packed = torch.from_numpy(gq.repack_host(O.Q6_K, w, n, k)).to(dev)
+    a = [torch.randn(m, k, generator=torch.Generator().manual_seed(i)).to(dev) for i in range(12)]
+    want = [gq.matmul(O.Q6_K, packed, x, n, k) for x in a]
+    got = [[torch.zeros(m, n, device=dev) for _ in range(20)] for _ in a]
+    torch.cuda.synchronize()
+    go = threading.Barrier(len(a))
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            go.wait()
+            for c in got[i]:
+                gq.matmul(O.Q6_K, packed, a[i], n, k, c=c)
+        s.synchronize()
+
+    th = [threading.Thread(target=work, args=(i,)) for i in range(len(a))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    bad = sum(not torch.equal(c, y) for x, y in zip(got, want) for c in x)
+    assert bad == 0, bad
+
+
+def test_scratch_of_many_streams_and_sizes(dev):
+    """One thread, ten streams with work pending on each, sizes that grow and
+    shrink: blocks are replaced and handed on in every state."""
+    import gq
+    import torch
+    k = 4096
+    w = torch.randn(700, k, generator=torch.Generator().manual_seed(2)).half().to(dev)
+    a = torch.randn(900, k, generator=torch.Generator().manual_seed(3)).to(dev)
+    sizes = [(17, 700), (900, 100), (64, 300), (300, 700), (40, 64), (600, 512)]
+    want = {(m, n): gq.gemm_f16w(w[:n], a[:m], n, k) for m, n in sizes}
+    big = torch.randn(2048, 2048, device=dev)
+    streams = [torch.cuda.Stream() for _ in range(10)]
+    torch.cuda.synchronize()
+    got = []
+    for turn in range(12):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                if turn % 3 == 0:
+                    big @ big
+                m, n = sizes[(turn * 7 + i) % len(sizes)]
+                c = torch.zeros(m, n, device=dev)
+                got.append(((m, n), gq.gemm_f16w(w[:n], a[:m], n, k, c=c)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(c, want[mn]) for mn, c in got)
+
+
 @pytest.mark.parametrize("m,n,k", [
     (4865, 5300, 96),     # 256 x 256 tiles; K past the last whole 64-k step
     (700, 8300, 160),     # 128 x 256
