@@ -670,6 +670,11 @@ extern "C" int gq_gemv_plan(int fmt, size_t N, size_t K, int batch, int *R_out, 
   return GQ_OK;
 }
 
+extern "C" int gq_gemv_k_parts(int fmt, size_t N, size_t K, int batch) {
+  if (gq_check_shape(fmt, N, K) != GQ_OK || N == 0 || K == 0 || batch < 1 || batch > GQ_MAX_BATCH) return 1;
+  return gq_gemv_on_h(fmt, N, K, batch) ? gq_gemv_h_parts(fmt, N, K, batch) : 1;
+}
+
 namespace {
 
 template <int FMT, int NBC, int MT, bool PREP>

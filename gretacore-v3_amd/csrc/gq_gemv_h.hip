@@ -964,6 +964,28 @@ int gq_gemv_h_plan(int fmt, size_t N, size_t K, int nb, int *R_out, int *ks_out,
   return GQ_OK;
 }
 
+// K parts over workgroups at batch 9..16 (1: none): few row tiles on a long K take
+// kGemvHPartsTw of them per workgroup and kGemvHPartsKs waves each.  A workgroup
+// stages 16 rows of activations over its K range whatever its row tiles, so with one
+// or two tiles each that outweighs the weights (batch 16, without / with: Q4_K 4096 x
+// 14336 24.7 / 20.2 us, 1024 x 14336 23.9 / 15.9, 8192 x 8192 29.6 / 21.9, Q8_0 44.7 /
+// 30.2, Q6_K 42.4 / 27.1).  Batch 8, K = 8192 on 256 tiles and the larger formats on
+// 256 tiles gain nothing (Q4_K 4096 x 14336 batch 8 17.1 / 18.1; 4096 x 8192 batch 16
+// 15.7 / 15.9; Q6_K 4096 x 14336 26.6 / 27.2).  At least 8 windows a part.  A plan forced
+// through the environment is not split.
+int gq_gemv_h_parts(int fmt, size_t N, size_t K, int nb) {
+  const int f = gq_fmt_is_q4k(fmt) ? GQ_FMT_Q4_K : gq_fmt_is_q6k(fmt) ? GQ_FMT_Q6_K : fmt;
+  if (f == GQ_FMT_F16 || nb <= 8 || K < 8192) return 1;
+  const size_t tiles = gq_tiles(N);
+  const int ck = f == GQ_FMT_Q4_K || f == GQ_FMT_Q6_K ? 256 : 128, win = (int)gq_chunks(f, K) * ck / kWin;
+  const int wgs = (int)((tiles + kGemvHPartsTw - 1) / kGemvHPartsTw);
+  const bool nib = f == GQ_FMT_Q4_0 || f == GQ_FMT_Q4_K;
+  if (tiles < 400 && (K == 8192 || !(nib || tiles <= 128))) return 1;
+  const int kz = 256 / wgs < win / 8 ? 256 / wgs : win / 8;
+  if (kz <= 1 || getenv("GQ_GEMV_H1") || getenv("GQ_GEMV_H_R") || getenv("GQ_GEMV_H_KSPLIT")) return 1;
+  return kz;
+}
+
 namespace {
 template <int FMT, int TW, int MR>
 int launch_h_tw(const void *packed, const float *x, float *y, int N, int K, int nb, int ks, hipStream_t s) {
@@ -1020,28 +1042,19 @@ int launch_h1_nck(const void *packed, const float *x, float *y, int N, int K, in
 #undef GQ_LAUNCH_H1
 }
 
-// Batch 9..16, few row tiles on a long K: four row tiles per workgroup and K in
-// parts over workgroups, the parts' sums in scratch.  A workgroup stages 16 rows
-// of activations over its K range whatever its row tiles, so with one or two
-// tiles each that outweighs the weights (batch 16, without / with: Q4_K 4096 x
-// 14336 24.7 / 20.2 us, 1024 x 14336 23.9 / 15.9, 8192 x 8192 29.6 / 21.9, Q8_0 44.7 /
-// 30.2, Q6_K 42.4 / 27.1).  Batch 8, K = 8192 on 256 tiles and the larger formats on
-// 256 tiles gain nothing (Q4_K 4096 x 14336 batch 8 17.1 / 18.1; 4096 x 8192 batch 16
-// 15.7 / 15.9; Q6_K 4096 x 14336 26.6 / 27.2).  GQ_ERR_UNSUPPORTED there, and
-// without scratch.
+// Batch 9..16 with K in parts over workgroups (gq_gemv_h_parts), the parts' sums in
+// scratch.  GQ_ERR_UNSUPPORTED for one part, and without scratch.
 template <int FMT>
 int launch_h_kz(const void *packed, const float *x, float *y, int N, int K, int nb, hipStream_t s) {
-  const size_t tiles = gq_tiles(N);
-  const int C = (int)gq_chunks(FMT, K), win = C * HFmt<FMT>::CK / kWin, wgs = (int)((tiles + 3) / 4);
-  const int kz = 256 / wgs < win / 8 ? 256 / wgs : win / 8;
-  const bool pays = tiles >= 400 ? K >= 8192 : K > 8192 && (kNibOrder<FMT> || tiles <= 128);
-  if (nb <= 8 || kz <= 1 || !pays) return GQ_ERR_UNSUPPORTED;
+  const int kz = gq_gemv_h_parts(FMT, N, K, nb);
+  if (kz <= 1) return GQ_ERR_UNSUPPORTED;
   GqScratch ws((size_t)kz * nb * N * 4, s);
   if (!ws.ptr) return GQ_ERR_UNSUPPORTED;
-  constexpr int WC = kWin / HFmt<FMT>::CK;
-  const int NI = (((C + kz - 1) / kz + 3) / 4 + WC - 1) / WC;
-  hipLaunchKernelGGL((k_gemv_h<FMT, 4, 4, 16, true>), dim3((unsigned)wgs, (unsigned)kz), dim3(64 * 16), 0, s,
-                     (const uint8_t *)packed, gq_sc_plane_offset(FMT, N, K), x, (float *)ws.ptr, N, K, C, nb, NI);
+  constexpr int TW = kGemvHPartsTw, KS = kGemvHPartsKs, WC = kWin / HFmt<FMT>::CK;
+  const int C = (int)gq_chunks(FMT, K), NI = (((C + kz - 1) / kz + KS - 1) / KS + WC - 1) / WC;
+  hipLaunchKernelGGL((k_gemv_h<FMT, TW, KS, 16, true>), dim3((unsigned)((gq_tiles(N) + TW - 1) / TW), (unsigned)kz),
+                     dim3(64 * TW * KS), 0, s, (const uint8_t *)packed, gq_sc_plane_offset(FMT, N, K), x, (float *)ws.ptr,
+                     N, K, C, nb, NI);
   GQ_TRY(gq_last_launch());
   return gq_launch_split_sum((const float *)ws.ptr, y, (size_t)nb * N, kz, s);
 }

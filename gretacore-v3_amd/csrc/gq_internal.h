@@ -58,6 +58,10 @@ int gq_launch_prep_x(int fmt, const float *x, void *ws, int B, int K, hipStream_
 int gq_gemv_h_min(void);
 int gq_gemv_h_plan(int fmt, size_t N, size_t K, int nb, int *R_out, int *ks_out, int *cpw_out);
 int gq_gemv_h1_plan(int fmt, size_t N, size_t K, int nb, int *R_out, int *ks_out, int *cpw_out);
+// K parts over workgroups (1: the plans above), with the row tiles and waves a
+// workgroup then takes
+constexpr int kGemvHPartsTw = 4, kGemvHPartsKs = 4;
+int gq_gemv_h_parts(int fmt, size_t N, size_t K, int nb);
 int gq_launch_gemv_h(int fmt, const void *packed, const float *x, float *y, int N, int K, int nb, hipStream_t s);
 
 // skinny GEMM for M <= 256 (gq_gemv_h.hip); A fp16 in the B fragments' order

@@ -46,6 +46,7 @@ _SIGS = {
     "gq_gemv": (ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, _c_size, _c_size, ctypes.c_int, _vp, _c_size, _vp]),
     "gq_gemv_plan": (ctypes.c_int, [ctypes.c_int, _c_size, _c_size, ctypes.c_int, ctypes.POINTER(ctypes.c_int),
                                      ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
+    "gq_gemv_k_parts": (ctypes.c_int, [ctypes.c_int, _c_size, _c_size, ctypes.c_int]),
     "gq_gemv_prep": (ctypes.c_int, [ctypes.c_int, _vp, _c_size, ctypes.c_int, _vp, _c_size, _vp]),
     "gq_gemv_prepped": (ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, _c_size, _c_size, ctypes.c_int, _vp]),
     "gq_gemm_workspace_bytes": (_c_size, [ctypes.c_int, _c_size, _c_size]),
@@ -198,7 +199,6 @@ def _require_device(*tensors):
             raise GQError("device tensor expected (libgq has no CPU path)")
 
 
-
 # ---- sizes / host repack (no GPU needed) ----------------------------------
 def gguf_bytes(fmt: int, n: int, k: int) -> int:
     return load().gq_gguf_bytes(fmt, n, k)
@@ -281,6 +281,11 @@ def gemv_plan(fmt: int, n: int, k: int, batch: int):
     r, ks, cpw = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     check(load().gq_gemv_plan(fmt, n, k, batch, ctypes.byref(r), ctypes.byref(ks), ctypes.byref(cpw)), "gq_gemv_plan")
     return r.value, ks.value, cpw.value
+
+
+def gemv_k_parts(fmt: int, n: int, k: int, batch: int) -> int:
+    """Parts of K over workgroups of an uncaptured gemv (1: none)."""
+    return load().gq_gemv_k_parts(fmt, n, k, batch)
 
 
 def gemv_workspace_bytes(fmt: int, k: int, batch: int) -> int:

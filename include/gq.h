@@ -135,9 +135,14 @@ int gq_gemv(int fmt, const void *d_packed, const float *d_x, float *d_y, size_t 
             void *d_workspace, size_t workspace_bytes, void *stream);
 /* Launch plan of gq_gemv for a shape (no GPU needed): row tiles per
  * workgroup, waves per workgroup (K split) and the most K chunks one wave
- * streams.  Environment overrides for tuning: GQ_GEMV_R, GQ_GEMV_KSPLIT. */
+ * streams.  Environment overrides for tuning: GQ_GEMV_R, GQ_GEMV_KSPLIT.  Where
+ * gq_gemv_k_parts is more than 1 this is the launch without parts, as under
+ * capture. */
 int gq_gemv_plan(int fmt, size_t N, size_t K, int batch, int *row_tiles_per_wg, int *ksplit,
                  int *chunks_per_wave);
+/* Parts of K over workgroups of an uncaptured gq_gemv (1: none); each workgroup then
+ * takes 4 row tiles with 4 waves each.  No GPU needed. */
+int gq_gemv_k_parts(int fmt, size_t N, size_t K, int batch);
 /* Split form: prepare x once (gq_gemv_prep) and run several GEMVs that share
  * it (q/k/v, gate/up) with gq_gemv_prepped. */
 int gq_gemv_prep(int fmt, const float *d_x, size_t K, int batch, void *d_workspace, size_t workspace_bytes,

@@ -23,12 +23,15 @@ SB = {gq.FMT_Q4_0: 128, gq.FMT_Q8_0: 128, gq.FMT_Q4_K: 256, gq.FMT_Q4_K_GGML: 25
 KWIN = 256  # k per activation staging window of the fp16 batch kernel
 
 
-def emulate_h(fmt, n, k, batch):
+def emulate_h(fmt, n, k, batch, parts=1):
     """Replays k_gemv_h's window, chunk and address arithmetic on the host:
     workgroup = TW row tiles x KS parts of K, weights prefetched two windows
     ahead (clamped to the part's last chunk), MR (8 up to batch 8, else 16)
-    activation rows staged per window in runs of 8."""
+    activation rows staged per window in runs of 8.  parts > 1: K in parts over
+    workgroups too, 4 x 4 each."""
     TW, KS, cpw = gq.gemv_plan(fmt, n, k, batch)
+    if parts > 1:
+        emulate_h_parts(fmt, n, k, batch, parts)
     mr = 8 if batch <= 8 else 16
     assert TW in (1, 2, 4) and KS in (1, 2, 4, 8) and TW * KS <= 16
     assert 2 * TW <= mr  # x runs spread evenly over the threads
@@ -64,6 +67,57 @@ def emulate_h(fmt, n, k, batch):
         m, g, j = o >> 6, (o & 63) >> 4, (o & 15) >> 3
         dst = p * WB + (((m * 2 + j) * 4 + g) * mr + b) * 16
         assert 0 <= dst and dst + 16 <= KS * WB
+
+
+def emulate_h_parts(fmt, n, k, batch, kz):
+    """The same for K in kz parts over workgroups: every chunk of K in exactly one
+    wave of one part, none empty, windows of the launch enough for the longest."""
+    TW, KS, mr = 4, 4, 16
+    C = -(-k // CK[fmt])
+    tiles = -(-n // 16)
+    wc = KWIN // CK[fmt]
+    assert 9 <= batch <= 16 and 1 < kz and -(-tiles // TW) * kz <= 256
+    NI = -(-(-(-(-(-C // kz)) // KS)) // wc)
+    assert 2 * KS * KWIN * 2 * mr <= 160 * 1024
+    seen = []
+    for z in range(kz):
+        zc = C * z // kz
+        cz = C * (z + 1) // kz - zc
+        assert cz >= KS and cz * CK[fmt] >= 8 * KWIN - CK[fmt]
+        for part in range(KS):
+            c0, c1 = zc + cz * part // KS, zc + cz * (part + 1) // KS
+            assert c0 < c1 <= C and -(-(c1 - c0) // wc) <= NI
+            seen += range(c0, c1)
+            for it in range(max(NI, 2) + 2):
+                for j in range(wc):
+                    ci = min(c0 + it * wc + j, c1 - 1)
+                    t = tiles - 1
+                    assert (t * C + ci + 1) * QB[fmt] <= tiles * C * QB[fmt]
+            for it in range(NI):
+                for kr in range(32):
+                    kk = c0 * CK[fmt] + 8 * kr + it * KWIN
+                    if kk < min(c1 * CK[fmt], k):
+                        assert kk + 8 <= k
+    assert seen == list(range(C))
+
+
+@pytest.mark.parametrize("fmt", [gq.FMT_Q4_0, gq.FMT_Q8_0, gq.FMT_Q4_K, gq.FMT_Q6_K])
+def test_gemv_k_parts_in_bounds(fmt, monkeypatch):
+    split = 0
+    for n in (16, 17, 500, 1024, 2047, 2064, 4096, 6384, 6400, 8192, 8208, 12000, 14336):
+        for k in (4096, 8192, 8448, 10240, 11008, 14336, 16384, 28672, 65536) + ((8224, 14368) if CK[fmt] == 128 else ()):
+            for batch in (8, 9, 16):
+                kz = gq.gemv_k_parts(fmt, n, k, batch)
+                assert kz >= 1 and (kz == 1 or batch > 8 and k >= 8192)
+                if kz > 1:
+                    split += 1
+                    emulate_h(fmt, n, k, batch, kz)
+    assert split > 50
+    assert gq.gemv_k_parts(fmt, 2048, 14336, 16) > 1
+    for name in ("GQ_GEMV_H_R", "GQ_GEMV_H_KSPLIT", "GQ_GEMV_H1"):  # a forced plan is the plan that runs
+        with monkeypatch.context() as m:
+            m.setenv(name, "1")
+            assert gq.gemv_k_parts(fmt, 2048, 14336, 16) == 1
 
 
 def h1_plan(fmt, n, k, batch):
