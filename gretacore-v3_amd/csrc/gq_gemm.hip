@@ -733,7 +733,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KG)
 __attribute__((amdgpu_waves_per_eu(WM * WN * KG / 4, WM * WN * KG / 4)))
 k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__restrict__ a16, int lda,
           void *__restrict__ c, const float *__restrict__ rs, int M, int N, int C, int nsteps, int tiles_m,
-          int gm, int sps) {
+          int gm, int sps, const uint8_t *__restrict__ wsh) {
   constexpr int KS = BK / 16;
   constexpr int NW = WM * WN, TM = BM / WM / 32, NJ = BN / WN / 32;  // waves per group, MFMA tiles per wave
   static_assert(TM >= 1 && NJ >= 1 && BM % (8 * NW) == 0, "tile shape");
@@ -845,12 +845,44 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     }
     return s0 + l * KG + kg;
   };
+  // Windows of 256 k under shifts of their own (k_a_to_f16's WIN): the sums are
+  // brought from window `from`'s scale to window `to`'s (-1: the row's), in
+  // workgroups with such a row.
+  constexpr bool WINF = FMT == GQ_FMT_Q6_K || FMT == GQ_FMT_F16;
+  auto rescale = [&](int from, int to) __attribute__((always_inline)) {
+    // [window][row]: four rows' shifts are one load (rows from M on: any value)
+    const uint32_t ld = (uint32_t)(M + 3) & ~3u;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(wsh), (short)0, (int)(ld * (uint32_t)(nsteps >> 2)), 0x00020000);
+    const uint32_t vo = (uint32_t)(m0 + (BM / WM) * wm + 4 * (lane >> 5));
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t o = vo + (uint32_t)(32 * i + 8 * q);
+        const uint32_t a = from < 0 ? 0u : __builtin_amdgcn_raw_buffer_load_b32(r, o, (uint32_t)from * ld, 0);
+        const uint32_t b = to < 0 ? 0u : __builtin_amdgcn_raw_buffer_load_b32(r, o, (uint32_t)to * ld, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int d = (int)((b >> (8 * e)) & 255u) - (int)((a >> (8 * e)) & 255u);
+          const float f = __uint_as_float((uint32_t)(127 + d) << 23);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) acc[i][j][4 * q + e] *= f;
+        }
+        if (TM > 4 || q == 3) __builtin_amdgcn_sched_barrier(0);  // (few loads at a time: registers)
+      }
+    }
+  };
   // the group's step l (buffer and register stage l % PD; `step` the K step);
   // steps past the end are skipped by every wave alike
-  auto run_step = [&](int l, auto buf_c) {
+  auto run_step = [&](int l, auto buf_c, auto wide_c) {
     constexpr int BUF = decltype(buf_c)::value;
     using NB = std::integral_constant<int, (BUF + PD - 1) % PD>;  // buffer of l + PD - 1
     const int step = gstep(l);
+    if constexpr (decltype(wide_c)::value) {
+      const int from = l > 0 ? gstep(l - 1) >> 2 : -1;
+      if (from != step >> 2) rescale(from, step >> 2);
+    }
     const int s1 = gstep(l + PD - 1 < nl ? l + PD - 1 : nl - 1);
     const int s2 = gstep(l + PD < nl ? l + PD : nl - 1);
     load_a_lds_b<BM, NW>(a16, ao, s1, wave, As_of(NB{}));
@@ -912,13 +944,29 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   __builtin_amdgcn_s_waitcnt(kWaitPend);
   if (tid < BM / 4) *reinterpret_cast<gq_f4 *>(rs_s + 4 * tid) = rs4;
   __syncthreads();
-  for (int l = 0; l < nl; l += PD) {
-    run_step(l, B0{});
-    if (l + 1 < nl) run_step(l + 1, B1{});
-    if constexpr (PD >= 3)
-      if (l + 2 < nl) run_step(l + 2, B2{});
-    if constexpr (PD >= 4)
-      if (l + 3 < nl) run_step(l + 3, B3{});
+  auto walk = [&](auto wide_c) {
+    for (int l = 0; l < nl; l += PD) {
+      run_step(l, B0{}, wide_c);
+      if (l + 1 < nl) run_step(l + 1, B1{}, wide_c);
+      if constexpr (PD >= 3)
+        if (l + 2 < nl) run_step(l + 2, B2{}, wide_c);
+      if constexpr (PD >= 4)
+        if (l + 3 < nl) run_step(l + 3, B3{}, wide_c);
+    }
+    if constexpr (decltype(wide_c)::value) rescale(gstep(nl - 1) >> 2, -1);
+  };
+  if constexpr (WINF) {
+    // a walk of its own (with the rescaling under a branch in the one walk, 1-3 %
+    // slower without such rows): 100 x 32000 x 4096 fp16 62 us without such rows, as
+    // with one scale per row, 81 with them; 512 x 4096 x 14336 Q6_K 98 and 145.  The
+    // scales behind row M are not set
+    bool neg = false;
+#pragma unroll
+    for (int i = 0; i < BM; i += 64) neg = neg || (m0 + i + lane < M && rs_s[i + lane] < 0.f);
+    if (__any(neg)) walk(std::true_type{});
+    else walk(std::false_type{});
+  } else {
+    walk(std::false_type{});
   }
   if constexpr (KG > 1) {
     // the groups' sums, one MFMA tile at a time: groups 1 .. KG - 1 write
@@ -968,7 +1016,7 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
     for (int q = 0; q < 4; ++q) {
       const gq_f4 t = *reinterpret_cast<const gq_f4 *>(rs_s + (mb - m0) + 8 * q);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) rsv[4 * q + e] = t[e];
+      for (int e = 0; e < 4; ++e) rsv[4 * q + e] = !WINF ? t[e] : SP ? 1.f : fabsf(t[e]);  // (parts: k_split_sum's)
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
@@ -1057,15 +1105,53 @@ GQ_DEV gq_half8 conv8(const float (&v)[8], float f, int q4perm) {
   return h;
 }
 
-template <int DT, int RUNS>
+// Magnitude as it counts for a scale.  WIN: of finite values only, so that those
+// beside an Inf or NaN don't overflow.
+template <bool WIN>
+GQ_DEV float scale_mag(float x) {
+  const float m = fabsf(x);
+  return !WIN || m < __builtin_inff() ? m : 0.f;
+}
+// The largest of a window of 256 k: 32 lanes, a run of 8 each (n runs at a time, so
+// that their exchanges overlap)
+template <int NR>
+GQ_DEV void win_max(float (&m)[NR], int n) {
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1)
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (r < n) m[r] = fmaxf(m[r], __shfl_xor(m[r], o, 64));
+}
+// s = 14 - floor(log2(amax)) from the exponent field (0 for a zero row, Inf / NaN;
+// clamped so 2^s and 2^-s stay normal floats)
+template <bool WIN>
+GQ_DEV int row_shift(float amax) {
+  const uint32_t eb = (__float_as_uint(amax) >> 23) & 0xFFu;
+  const int sh = (!WIN && eb == 0u) || eb == 0xFFu ? 0 : 14 - ((int)eb - 127);
+  return sh < -100 ? -100 : sh > 100 ? 100 : sh;
+}
+// WIN: a window of 256 k whose largest magnitude is more than 2^20 below the row's is scaled
+// up by 2^t more, t to wsh[window][row] (rows padded to 4), and such a row's rs is negative; the GEMM
+// undoes t around the window.  In any other window an entry down to 2^-9 of its
+// largest keeps all 11 bits, so rows without an outlier of that size run as before.
+// (Q6_K with K > 4096 and fp16 weights, whose few-row kernel scales by window.)
+GQ_DEV int win_shift(float amax, float wmax, int sh) {
+  const int t = (int)(__float_as_uint(amax) >> 23) - (int)(__float_as_uint(wmax) >> 23);
+  const int top = 100 - sh < 64 ? 100 - sh : 64;
+  return wmax == 0.f || t <= 20 ? 0 : t < top ? t : top;
+}
+GQ_DEV float pow2f(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
+
+template <int DT, int RUNS, bool WIN>
 __global__ void __launch_bounds__(kConvThreads) k_a_to_f16(const void *__restrict__ a, _Float16 *__restrict__ o,
-                                                           float *__restrict__ rs, int K, int ldo, int q4perm) {
-  __shared__ float wmax[kConvThreads / 64];
+                                                           float *__restrict__ rs, int K, int ldo, int q4perm,
+                                                           uint8_t *__restrict__ wsh) {
+  __shared__ float wmax[kConvThreads / 64], wmin[WIN ? kConvThreads / 64 : 1];
   const size_t m = blockIdx.x;
   const int tid = threadIdx.x;
   constexpr int SPAN = 8 * kConvThreads * kConvRuns;  // elements held in registers
   // K % 8 == 0 (host-checked), so a run of 8 is all inside or all past K
-  float v[kConvRuns][8];
+  float v[kConvRuns][8], wm[kConvRuns] = {};
   float amax = 0.f;
 #pragma unroll
   for (int r = 0; r < kConvRuns; ++r) {
@@ -1078,38 +1164,69 @@ __global__ void __launch_bounds__(kConvThreads) k_a_to_f16(const void *__restric
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       v[r][e] = (r < RUNS && k0 < K) ? v[r][e] : 0.f;
-      amax = fmaxf(amax, fabsf(v[r][e]));
+      wm[r] = fmaxf(wm[r], scale_mag<WIN>(v[r][e]));
     }
   }
-  for (int k0 = SPAN + 8 * tid; k0 < K; k0 += 8 * kConvThreads) {  // (rows longer than SPAN)
-    float u[8];
-    load8_t<DT>(a, m * K + k0, u);
+  if constexpr (WIN) win_max(wm, RUNS);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(u[e]));
+  for (int r = 0; r < kConvRuns; ++r) amax = fmaxf(amax, wm[r]);
+  float amin = __builtin_inff();  // WIN: the smallest maximum of a window, zeros apart
+#pragma unroll
+  for (int r = 0; r < kConvRuns; ++r) amin = wm[r] > 0.f ? fminf(amin, wm[r]) : amin;
+  // (rows longer than SPAN; WIN: ldo is whole windows, a window's lanes together)
+  for (int k0 = SPAN + 8 * tid; k0 < (WIN ? ldo : K); k0 += 8 * kConvThreads) {
+    float u[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, um[1] = {0.f};
+    if (!WIN || k0 < K) load8_t<DT>(a, m * K + k0, u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) um[0] = fmaxf(um[0], scale_mag<WIN>(u[e]));
+    if constexpr (WIN) win_max(um, 1);
+    amax = fmaxf(amax, um[0]);
+    amin = um[0] > 0.f ? fminf(amin, um[0]) : amin;
   }
 #pragma unroll
-  for (int o2 = 32; o2 > 0; o2 >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o2, 64));
-  if ((tid & 63) == 0) wmax[tid >> 6] = amax;
+  for (int o2 = 32; o2 > (WIN ? 16 : 0); o2 >>= 1) {  // (WIN: the same in 32 lanes already)
+    amax = fmaxf(amax, __shfl_xor(amax, o2, 64));
+    if constexpr (WIN) amin = fminf(amin, __shfl_xor(amin, o2, 64));
+  }
+  if ((tid & 63) == 0) {
+    wmax[tid >> 6] = amax;
+    if constexpr (WIN) wmin[tid >> 6] = amin;
+  }
   __syncthreads();
   amax = wmax[0];
 #pragma unroll
   for (int w = 1; w < kConvThreads / 64; ++w) amax = fmaxf(amax, wmax[w]);
-  // s = 14 - floor(log2(amax)) from the exponent field (0 for a zero row,
-  // Inf / NaN; clamped so 2^s and 2^-s stay normal floats)
-  const uint32_t eb = (__float_as_uint(amax) >> 23) & 0xFFu;
-  int sh = (eb == 0u || eb == 0xFFu) ? 0 : 14 - ((int)eb - 127);
-  sh = sh < -100 ? -100 : sh > 100 ? 100 : sh;
-  const float f = __uint_as_float((uint32_t)(127 + sh) << 23);
-  if (tid == 0) rs[m] = __uint_as_float((uint32_t)(127 - sh) << 23);
+  if constexpr (WIN) {
+#pragma unroll
+    for (int w = 0; w < kConvThreads / 64; ++w) amin = fminf(amin, wmin[w]);
+  }
+  const int sh = row_shift<WIN>(amax);
+  const float f = pow2f(sh);
+  if (tid == 0) rs[m] = WIN && win_shift(amax, amin, sh) > 0 ? -pow2f(-sh) : pow2f(-sh);
+  auto put = [&](const float(&x)[8], int k0, float wmax) {  // (wmax: of the run's window)
+    float fw = f;
+    if constexpr (WIN) {
+      const int t = win_shift(amax, wmax, sh);
+      fw = pow2f(sh + t);
+      if ((tid & 31) == 0) wsh[(size_t)(k0 >> 8) * ((gridDim.x + 3) & ~3u) + m] = (uint8_t)t;
+    }
+    *reinterpret_cast<gq_half8 *>(o + m * ldo + k0) = conv8(x, fw, q4perm);
+  };
 #pragma unroll
   for (int r = 0; r < kConvRuns; ++r) {
     const int k0 = 8 * (tid + kConvThreads * r);
-    if (k0 < ldo) *reinterpret_cast<gq_half8 *>(o + m * ldo + k0) = conv8(v[r], f, q4perm);
+    if (k0 < ldo) put(v[r], k0, wm[r]);
   }
   for (int k0 = SPAN + 8 * tid; k0 < ldo; k0 += 8 * kConvThreads) {
     float u[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (k0 < K) load8_t<DT>(a, m * K + k0, u);
-    *reinterpret_cast<gq_half8 *>(o + m * ldo + k0) = conv8(u, f, q4perm);
+    float um[1] = {0.f};
+    if constexpr (WIN) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) um[0] = fmaxf(um[0], scale_mag<WIN>(u[e]));
+      win_max(um, 1);
+    }
+    put(u, k0, um[0]);
   }
 }
 
@@ -1117,13 +1234,14 @@ __global__ void __launch_bounds__(kConvThreads) k_a_to_f16(const void *__restric
 // workgroup), the row held in registers (R runs of 8 per lane) and its
 // largest magnitude reduced within the wave -- no LDS, no barrier.  The same
 // scaling and rounding as k_a_to_f16.
-template <int R, int DT>
+template <int R, int DT, bool WIN>
 __global__ void __launch_bounds__(256) k_a_to_f16_w(const void *__restrict__ a, _Float16 *__restrict__ o,
-                                                    float *__restrict__ rs, int M, int K, int ldo, int q4perm) {
+                                                    float *__restrict__ rs, int M, int K, int ldo, int q4perm,
+                                                    uint8_t *__restrict__ wsh) {
   const int lane = threadIdx.x & 63;
   const size_t m = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= (size_t)M) return;
-  float v[R][8];
+  float v[R][8], wm[R] = {};
   float amax = 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -1136,20 +1254,34 @@ __global__ void __launch_bounds__(256) k_a_to_f16_w(const void *__restrict__ a, 
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       v[r][e] = k0 < K ? v[r][e] : 0.f;
-      amax = fmaxf(amax, fabsf(v[r][e]));
+      wm[r] = fmaxf(wm[r], scale_mag<WIN>(v[r][e]));
     }
   }
+  if constexpr (WIN) win_max(wm, R);
 #pragma unroll
-  for (int o2 = 32; o2 > 0; o2 >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o2, 64));
-  const uint32_t eb = (__float_as_uint(amax) >> 23) & 0xFFu;
-  int sh = (eb == 0u || eb == 0xFFu) ? 0 : 14 - ((int)eb - 127);
-  sh = sh < -100 ? -100 : sh > 100 ? 100 : sh;
-  const float f = __uint_as_float((uint32_t)(127 + sh) << 23);
-  if (lane == 0) rs[m] = __uint_as_float((uint32_t)(127 - sh) << 23);
+  for (int r = 0; r < R; ++r) amax = fmaxf(amax, wm[r]);
+  float amin = __builtin_inff();
+#pragma unroll
+  for (int r = 0; r < R; ++r) amin = wm[r] > 0.f ? fminf(amin, wm[r]) : amin;
+#pragma unroll
+  for (int o2 = 32; o2 > (WIN ? 16 : 0); o2 >>= 1) {
+    amax = fmaxf(amax, __shfl_xor(amax, o2, 64));
+    if constexpr (WIN) amin = fminf(amin, __shfl_xor(amin, o2, 64));
+  }
+  const int sh = row_shift<WIN>(amax);
+  const float f = pow2f(sh);
+  if (lane == 0) rs[m] = WIN && win_shift(amax, amin, sh) > 0 ? -pow2f(-sh) : pow2f(-sh);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int k0 = 8 * (lane + 64 * r);
-    if (k0 < ldo) *reinterpret_cast<gq_half8 *>(o + m * ldo + k0) = conv8(v[r], f, q4perm);
+    if (k0 >= ldo) continue;
+    float fw = f;
+    if constexpr (WIN) {
+      const int t = win_shift(amax, wm[r], sh);
+      fw = pow2f(sh + t);
+      if ((lane & 31) == 0) wsh[(size_t)(k0 >> 8) * (((unsigned)M + 3) & ~3u) + m] = (uint8_t)t;
+    }
+    *reinterpret_cast<gq_half8 *>(o + m * ldo + k0) = conv8(v[r], fw, q4perm);
   }
 }
 
@@ -1157,32 +1289,37 @@ __global__ void __launch_bounds__(256) k_a_to_f16_w(const void *__restrict__ a, 
 // of up to 8192 padded columns (2048 x 4096 bf16: 13.5 -> 11.1 us with loads
 // under branches), else k_a_to_f16 (one workgroup of 8 waves per row: fewer
 // rows keep more waves busy) with the runs per thread the row needs
-template <int DT>
-int launch_a_to_f16_t(const void *a, _Float16 *o, float *rs, int M, int K, int ldo, int q4perm, hipStream_t s) {
+template <int DT, bool WIN>
+int launch_a_to_f16_t(const void *a, _Float16 *o, float *rs, int M, int K, int ldo, int q4perm, uint8_t *wsh,
+                      hipStream_t s) {
   const unsigned g4 = (unsigned)((M + 3) / 4);
-  if (M >= 1024 && ldo <= 2048)
-    hipLaunchKernelGGL((k_a_to_f16_w<4, DT>), dim3(g4), dim3(256), 0, s, a, o, rs, M, K, ldo, q4perm);
-  else if (M >= 1024 && ldo <= 4096)
-    hipLaunchKernelGGL((k_a_to_f16_w<8, DT>), dim3(g4), dim3(256), 0, s, a, o, rs, M, K, ldo, q4perm);
-  else if (M >= 1024 && ldo <= 8192)
-    hipLaunchKernelGGL((k_a_to_f16_w<16, DT>), dim3(g4), dim3(256), 0, s, a, o, rs, M, K, ldo, q4perm);
-  else if (K <= 8 * kConvThreads)
-    hipLaunchKernelGGL((k_a_to_f16<DT, 1>), dim3((unsigned)M), dim3(kConvThreads), 0, s, a, o, rs, K, ldo, q4perm);
-  else if (K <= 2 * 8 * kConvThreads)
-    hipLaunchKernelGGL((k_a_to_f16<DT, 2>), dim3((unsigned)M), dim3(kConvThreads), 0, s, a, o, rs, K, ldo, q4perm);
-  else if (K <= 4 * 8 * kConvThreads)
-    hipLaunchKernelGGL((k_a_to_f16<DT, 4>), dim3((unsigned)M), dim3(kConvThreads), 0, s, a, o, rs, K, ldo, q4perm);
-  else
-    hipLaunchKernelGGL((k_a_to_f16<DT, kConvRuns>), dim3((unsigned)M), dim3(kConvThreads), 0, s, a, o, rs, K, ldo,
-                       q4perm);
+#define GQ_CONV_W(R) \
+  hipLaunchKernelGGL((k_a_to_f16_w<R, DT, WIN>), dim3(g4), dim3(256), 0, s, a, o, rs, M, K, ldo, q4perm, wsh)
+#define GQ_CONV(RUNS)                                                                                                \
+  hipLaunchKernelGGL((k_a_to_f16<DT, RUNS, WIN>), dim3((unsigned)M), dim3(kConvThreads), 0, s, a, o, rs, K, ldo, q4perm, \
+                     wsh)
+  if (M >= 1024 && ldo <= 2048) GQ_CONV_W(4);
+  else if (M >= 1024 && ldo <= 4096) GQ_CONV_W(8);
+  else if (M >= 1024 && ldo <= 8192) GQ_CONV_W(16);
+  else if (K <= 8 * kConvThreads) GQ_CONV(1);
+  else if (K <= 2 * 8 * kConvThreads) GQ_CONV(2);
+  else if (K <= 4 * 8 * kConvThreads) GQ_CONV(4);
+  else GQ_CONV(kConvRuns);
+#undef GQ_CONV
+#undef GQ_CONV_W
   return gq_last_launch();
 }
 
+// wsh: the window shifts (ldo whole windows, A in fp32); NULL: one scale per row
 int launch_a_to_f16(const void *a, int a_dtype, _Float16 *o, float *rs, int M, int K, int ldo, int q4perm,
-                    hipStream_t s) {
-  if (a_dtype == GQ_DT_BF16) return launch_a_to_f16_t<GQ_DT_BF16>(a, o, rs, M, K, ldo, q4perm, s);
-  if (a_dtype == GQ_DT_F16) return launch_a_to_f16_t<GQ_DT_F16>(a, o, rs, M, K, ldo, q4perm, s);
-  return launch_a_to_f16_t<GQ_DT_F32>(a, o, rs, M, K, ldo, q4perm, s);
+                    hipStream_t s, uint8_t *wsh = nullptr) {
+  if (wsh) {
+    GQ_CHECK(a_dtype == GQ_DT_F32 && ldo % 256 == 0, GQ_ERR_INVALID_ARGS);
+    return launch_a_to_f16_t<GQ_DT_F32, true>(a, o, rs, M, K, ldo, q4perm, wsh, s);
+  }
+  if (a_dtype == GQ_DT_BF16) return launch_a_to_f16_t<GQ_DT_BF16, false>(a, o, rs, M, K, ldo, q4perm, nullptr, s);
+  if (a_dtype == GQ_DT_F16) return launch_a_to_f16_t<GQ_DT_F16, false>(a, o, rs, M, K, ldo, q4perm, nullptr, s);
+  return launch_a_to_f16_t<GQ_DT_F32, false>(a, o, rs, M, K, ldo, q4perm, nullptr, s);
 }
 
 template <int FMT, int CBF16, int BM, int BN>
@@ -1211,7 +1348,7 @@ template <int CBF16>
 __global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ part, const float *__restrict__ rs,
                                                    void *__restrict__ c, size_t mn, int N, int splits) {
   auto put = [&](size_t j, float v) {
-    if (rs) v *= rs[j / (size_t)N];
+    if (rs) v *= fabsf(rs[j / (size_t)N]);
     if constexpr (CBF16) reinterpret_cast<uint16_t *>(c)[j] = f32_to_bf16_rne(v);
     else reinterpret_cast<float *>(c)[j] = v;
   };
@@ -1242,7 +1379,7 @@ __global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ par
 // parts' sums [splits][M][N] in fp32
 template <int FMT, int CBF16, int BM, int BN, int WM, int WN, int KG = 1, bool SP = false>
 int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
-              hipStream_t s, int pd_default = 4, int splits = 1) {
+              hipStream_t s, int pd_default = 4, int splits = 1, const uint8_t *wsh = nullptr) {
   const int C = FMT == GQ_FMT_F16 ? K : (int)gq_chunks(FMT, K);
   const uint32_t sc_off = FMT == GQ_FMT_F16 ? (uint32_t)N * (uint32_t)K * 2u : (uint32_t)gq_sc_plane_offset(FMT, N, K);
   const int nsteps = (int)((FMT == GQ_FMT_F16 ? gq_f16w_kpad(K) : gq_kpad(FMT, K)) / BK);
@@ -1260,7 +1397,7 @@ int launch_rb(const void *packed, const _Float16 *a16, int lda, void *c, const f
   hipLaunchKernelGGL((k_gemm_rb<FMT, CBF16, BM, BN, WM, WN, PD, KG, SP>),                                           \
                      dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits),                                     \
                      dim3(64 * WM * WN * KG), 0, s, (const uint8_t *)packed, sc_off, a16,      \
-                     lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps)
+                     lda, c, rs, M, N, C, nsteps, tiles_m, gm, sps, wsh)
   // the depths whose LDS fits (operand buffers, the K groups' exchange,
   // the row scales); a deeper request falls back to the deepest that fits
   constexpr auto lds = [](int d) {
@@ -1369,16 +1506,17 @@ int launch_fmt(const void *packed, const _Float16 *a16, int lda, void *c, const 
 // Q6_K and fp16 weights: the shapes pick_tile chooses by itself for whole
 // chunks of 256 k (the step count is then a multiple of 4)
 template <int FMT, int CBF16>
-int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int M, int N, int K,
-                  hipStream_t s) {
+int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, const uint8_t *wsh, int M,
+                  int N, int K, hipStream_t s) {
   switch (pick_tile(FMT, M, N, K)) {
   // (fp16 weights: both tiles are in LDS, launch_rb takes the depth that fits, and
   // the smallest tile runs two K groups, whose buffers leave room for depth 2)
-  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 3);
-  case 13: return launch_rb<FMT, CBF16, 128, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s);
-  case 17: return launch_rb<FMT, CBF16, 128, 128, 1, 4, 2>(packed, a16, lda, c, rs, M, N, K, s);
+  case 12: return launch_rb<FMT, CBF16, 256, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 3, 1, wsh);
+  case 13: return launch_rb<FMT, CBF16, 128, 256, 1, 8>(packed, a16, lda, c, rs, M, N, K, s, 4, 1, wsh);
+  case 17: return launch_rb<FMT, CBF16, 128, 128, 1, 4, 2>(packed, a16, lda, c, rs, M, N, K, s, 4, 1, wsh);
   default:
-    return launch_rb<FMT, CBF16, 64, 128, 1, 4, FMT == GQ_FMT_F16 ? 2 : 4>(packed, a16, lda, c, rs, M, N, K, s);
+    return launch_rb<FMT, CBF16, 64, 128, 1, 4, FMT == GQ_FMT_F16 ? 2 : 4>(packed, a16, lda, c, rs, M, N, K, s, 4, 1,
+                                                                           wsh);
   }
 }
 
@@ -1397,13 +1535,13 @@ SplitPlan split_plan(int M, int N, int nsteps) {
   if (want > nsteps / 8) want = nsteps / 8;
   return SplitPlan{bm, want > 1 ? split_parts(nsteps, (int)want) : 1};
 }
-template <int FMT>
-int launch_split(const void *packed, const _Float16 *a16, int lda, float *c, const float *rs, float *part, SplitPlan p,
-                 int M, int N, int K, hipStream_t s) {
+int launch_split_f16w(const void *w, const _Float16 *a16, int lda, float *c, const float *rs, const uint8_t *wsh,
+                      float *part, SplitPlan p, int M, int N, int K, hipStream_t s) {
+  constexpr int F = GQ_FMT_F16;
   if (p.bm == 128)
-    GQ_TRY((launch_rb<FMT, 0, 128, 128, 1, 4, 2, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
+    GQ_TRY((launch_rb<F, 0, 128, 128, 1, 4, 2, true>(w, a16, lda, part, rs, M, N, K, s, 4, p.splits, wsh)));
   else
-    GQ_TRY((launch_rb<FMT, 0, 64, 128, 1, 4, 2, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, p.splits)));
+    GQ_TRY((launch_rb<F, 0, 64, 128, 1, 4, 2, true>(w, a16, lda, part, rs, M, N, K, s, 4, p.splits, wsh)));
   const size_t mn = (size_t)M * (size_t)N;
   hipLaunchKernelGGL(k_split_sum<0>, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, part, rs, c, mn, N, p.splits);
   return gq_last_launch();
@@ -1426,8 +1564,9 @@ int gemm_splits(int fmt, size_t M, size_t N, size_t K) {
   return split_parts((int)nsteps, (int)want);
 }
 int launch_gemm_split(int fmt, const void *packed, const _Float16 *a16, int lda, void *c, int c_dtype, const float *rs,
-                      float *part, int splits, int M, int N, int K, hipStream_t s) {
-#define GQ_PARTS(F) launch_rb<F, 0, 64, 128, 1, 4, 4, true>(packed, a16, lda, part, nullptr, M, N, K, s, 4, splits)
+                      const uint8_t *wsh, float *part, int splits, int M, int N, int K, hipStream_t s) {
+#define GQ_PARTS(F) \
+  launch_rb<F, 0, 64, 128, 1, 4, 4, true>(packed, a16, lda, part, wsh ? rs : nullptr, M, N, K, s, 4, splits, wsh)
   if (fmt == GQ_FMT_Q4_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q4_0));
   else if (fmt == GQ_FMT_Q8_0) GQ_TRY(GQ_PARTS(GQ_FMT_Q8_0));
   else if (gq_fmt_is_q6k(fmt)) GQ_TRY(GQ_PARTS(GQ_FMT_Q6_K));
@@ -1443,14 +1582,14 @@ int launch_gemm_split(int fmt, const void *packed, const _Float16 *a16, int lda,
 }
 
 template <int FMT>
-int launch_gemm(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, int c_dtype, int M, int N,
-                int K, hipStream_t s) {
+int launch_gemm(const void *packed, const _Float16 *a16, int lda, void *c, const float *rs, const uint8_t *wsh,
+                int c_dtype, int M, int N, int K, hipStream_t s) {
   if constexpr (FMT == GQ_FMT_Q6_K)
-    return c_dtype == GQ_DT_BF16 ? launch_fmt_kg<FMT, 1>(packed, a16, lda, c, rs, M, N, K, s)
-                                 : launch_fmt_kg<FMT, 0>(packed, a16, lda, c, rs, M, N, K, s);
+    return c_dtype == GQ_DT_BF16 ? launch_fmt_kg<FMT, 1>(packed, a16, lda, c, rs, wsh, M, N, K, s)
+                                 : launch_fmt_kg<FMT, 0>(packed, a16, lda, c, rs, wsh, M, N, K, s);
   else
-  return c_dtype == GQ_DT_BF16 ? launch_fmt<FMT, 1>(packed, a16, lda, c, rs, M, N, K, s)
-                               : launch_fmt<FMT, 0>(packed, a16, lda, c, rs, M, N, K, s);
+    return c_dtype == GQ_DT_BF16 ? launch_fmt<FMT, 1>(packed, a16, lda, c, rs, M, N, K, s)
+                                 : launch_fmt<FMT, 0>(packed, a16, lda, c, rs, M, N, K, s);
 }
 
 }  // namespace
@@ -1482,7 +1621,7 @@ static bool gemm_converts_a(int fmt, size_t M, size_t N, size_t K, int a_dtype) 
 }
 
 static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
-                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed = false);
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed = false, uint8_t *wsh = nullptr);
 
 static int gemm_checked(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M,
                         size_t N, size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed) {
@@ -1511,15 +1650,15 @@ extern "C" int gq_gemm(int fmt, const void *packed, const void *a, int a_dtype, 
 // tiled kernel's 32-bit offsets do not reach; nothing is launched then.
 int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, size_t M, size_t N, size_t K,
                          hipStream_t s) {
-  const size_t row = gq_kpad(fmt, K) * 2;
+  const size_t Kp = gq_kpad(fmt, K), row = Kp * 2 + Kp / 256;
   GQ_CHECK(gq_packed_bytes(fmt, N, K) < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
   const size_t fit = ((kGqScratchMax - (1 << 20)) / (row + 20)) & ~(size_t)255, mb = M < fit ? M : fit;
   const size_t bytes = gq_gemm_workspace_bytes(fmt, mb, K);
-  GqScratch ws(bytes, s);
+  GqScratch ws(bytes + (mb + 3) / 4 * 4 * (Kp / 256), s);
   GQ_CHECK(ws.ptr, GQ_ERR_WORKSPACE);
   for (size_t m0 = 0; m0 < M; m0 += mb)
     GQ_TRY(gemm_core(fmt, packed, a + m0 * K, GQ_DT_F32, c + m0 * N, GQ_DT_F32, M - m0 < mb ? M - m0 : mb, N, K,
-                     ws.ptr, bytes, s));
+                     ws.ptr, bytes, s, false, (uint8_t *)ws.ptr + bytes));
   return GQ_OK;
 }
 
@@ -1527,35 +1666,38 @@ int gq_launch_matmul_q6k(int fmt, const void *packed, const float *a, float *c, 
 // aligned): A to fp16 with row scales in a scratch buffer, then the register-B
 // kernel on the fp16 rows of W.  Status as gq_launch_matmul_q6k.
 int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_t N, size_t K, hipStream_t s) {
-  const size_t Kp = gq_f16w_kpad(K), row = Kp * 2;
+  const size_t Kp = gq_f16w_kpad(K), row = Kp * 2 + Kp / 256;
   // 32-bit weight offsets, with room for the columns read past a row's end
-  GQ_CHECK(N * K * 2 + row < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
+  GQ_CHECK(N * K * 2 + Kp * 2 < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
   const size_t fit = ((kGqScratchMax - (1 << 20)) / (row + 20)) & ~(size_t)255, mb = M < fit ? M : fit;
-  const size_t abytes = gq_align256(mb * row), rbytes = gq_align256((mb + 256) * 4);  // (row scales read by the tile)
+  // (row scales read by the tile, window shifts)
+  const size_t abytes = gq_align256(mb * Kp * 2), rbytes = gq_align256((mb + 256) * 4), hbytes = gq_align256((mb + 3) / 4 * 4 * (Kp / 256));
   const SplitPlan sp = split_plan((int)mb, (int)N, (int)(Kp / BK));
   const size_t pbytes = sp.splits > 1 ? (size_t)sp.splits * M * N * 4 : 0;
-  const bool split = sp.splits > 1 && mb == M && abytes + rbytes + pbytes <= kGqScratchMax;
-  GqScratch ws(abytes + rbytes + (split ? pbytes : 0), s);
+  const bool split = sp.splits > 1 && mb == M && abytes + rbytes + hbytes + pbytes <= kGqScratchMax;
+  GqScratch ws(abytes + rbytes + hbytes + (split ? pbytes : 0), s);
   GQ_CHECK(ws.ptr, GQ_ERR_WORKSPACE);
   float *rs = (float *)((uint8_t *)ws.ptr + abytes);
+  uint8_t *wsh = (uint8_t *)rs + rbytes;
   if (split) {
-    GQ_TRY(launch_a_to_f16(a, GQ_DT_F32, (_Float16 *)ws.ptr, rs, (int)M, (int)K, (int)Kp, 0, s));
-    return launch_split<GQ_FMT_F16>(w, (const _Float16 *)ws.ptr, (int)Kp, c, rs, (float *)((uint8_t *)rs + rbytes), sp,
-                                    (int)M, (int)N, (int)K, s);
+    GQ_TRY(launch_a_to_f16(a, GQ_DT_F32, (_Float16 *)ws.ptr, rs, (int)M, (int)K, (int)Kp, 0, s, wsh));
+    return launch_split_f16w(w, (const _Float16 *)ws.ptr, (int)Kp, c, rs, wsh, (float *)(wsh + hbytes), sp, (int)M, (int)N,
+                             (int)K, s);
   }
   for (size_t m0 = 0; m0 < M; m0 += mb) {
     const int m = (int)(M - m0 < mb ? M - m0 : mb);
-    GQ_TRY(launch_a_to_f16(a + m0 * K, GQ_DT_F32, (_Float16 *)ws.ptr, rs, m, (int)K, (int)Kp, 0, s));
-    GQ_TRY((launch_fmt_kg<GQ_FMT_F16, 0>(w, (const _Float16 *)ws.ptr, (int)Kp, c + m0 * N, rs, m, (int)N, (int)K, s)));
+    GQ_TRY(launch_a_to_f16(a + m0 * K, GQ_DT_F32, (_Float16 *)ws.ptr, rs, m, (int)K, (int)Kp, 0, s, wsh));
+    GQ_TRY((launch_fmt_kg<GQ_FMT_F16, 0>(w, (const _Float16 *)ws.ptr, (int)Kp, c + m0 * N, rs, wsh, m, (int)N, (int)K, s)));
   }
   return GQ_OK;
 }
 
 // fixed: ws holds all memory there is (the K parts' sums go behind the
 // conversion); otherwise the sums take a scratch block, and there is no split
-// without one.
+// without one.  wsh: room for the conversion's window shifts (Q6_K: a byte per row, of
+// rows padded to 4, and 256 k; NULL: one scale per row).
 static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, void *c, int c_dtype, size_t M, size_t N,
-                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed) {
+                     size_t K, void *ws, size_t ws_bytes, hipStream_t s, bool fixed, uint8_t *wsh) {
   const int splits = gemm_splits(fmt, M, N, K);
   if (splits > 1) {
     const size_t Kp = gq_kpad(fmt, K), conv = gq_gemm_workspace_bytes(fmt, M, K), pbytes = (size_t)splits * M * N * 4;
@@ -1572,11 +1714,12 @@ static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, vo
         }
         GQ_CHECK(ws_bytes >= conv, GQ_ERR_WORKSPACE);
         float *rsw = (float *)((uint8_t *)ws + gq_align256(M * Kp * 2));
-        GQ_TRY(launch_a_to_f16(a, a_dtype, (_Float16 *)ws, rsw, (int)M, (int)K, (int)Kp, q4, s));
+        GQ_TRY(launch_a_to_f16(a, a_dtype, (_Float16 *)ws, rsw, (int)M, (int)K, (int)Kp, q4, s, wsh));
         a16 = (const _Float16 *)ws;
         rs = rsw;
       }
-      return launch_gemm_split(fmt, packed, a16, (int)Kp, c, c_dtype, rs, part, splits, (int)M, (int)N, (int)K, s);
+      return launch_gemm_split(fmt, packed, a16, (int)Kp, c, c_dtype, rs, wsh, part, splits, (int)M, (int)N, (int)K,
+                               s);
     }
   }
   // Few rows: the tiled GEMM gives N / 64 .. N / 128 workgroups, each walking
@@ -1623,17 +1766,17 @@ static int gemm_core(int fmt, const void *packed, const void *a, int a_dtype, vo
     }
     GQ_CHECK(ws_bytes >= need, GQ_ERR_WORKSPACE);
     float *rsw = (float *)((uint8_t *)ws + gq_align256(M * Kp * 2));
-    GQ_TRY(launch_a_to_f16(a, a_dtype, (_Float16 *)ws, rsw, (int)M, (int)K, (int)Kp, q4, s));
+    GQ_TRY(launch_a_to_f16(a, a_dtype, (_Float16 *)ws, rsw, (int)M, (int)K, (int)Kp, q4, s, wsh));
     a16 = (const _Float16 *)ws;
     rs = rsw;
   }
   const int lda = (int)Kp;
   switch (fmt) {
-  case GQ_FMT_Q4_0: return launch_gemm<GQ_FMT_Q4_0>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
-  case GQ_FMT_Q8_0: return launch_gemm<GQ_FMT_Q8_0>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
+  case GQ_FMT_Q4_0: return launch_gemm<GQ_FMT_Q4_0>(packed, a16, lda, c, rs, wsh, c_dtype, (int)M, (int)N, (int)K, s);
+  case GQ_FMT_Q8_0: return launch_gemm<GQ_FMT_Q8_0>(packed, a16, lda, c, rs, wsh, c_dtype, (int)M, (int)N, (int)K, s);
   case GQ_FMT_Q6_K:
-  case GQ_FMT_Q6_K_GGML: return launch_gemm<GQ_FMT_Q6_K>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
-  default: return launch_gemm<GQ_FMT_Q4_K>(packed, a16, lda, c, rs, c_dtype, (int)M, (int)N, (int)K, s);
+  case GQ_FMT_Q6_K_GGML: return launch_gemm<GQ_FMT_Q6_K>(packed, a16, lda, c, rs, wsh, c_dtype, (int)M, (int)N, (int)K, s);
+  default: return launch_gemm<GQ_FMT_Q4_K>(packed, a16, lda, c, rs, wsh, c_dtype, (int)M, (int)N, (int)K, s);
   }
 }
 

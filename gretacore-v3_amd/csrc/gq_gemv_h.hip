@@ -1103,8 +1103,8 @@ int gq_launch_gemv_h(int fmt, const void *packed, const float *x, float *y, int 
 // C[M][N] = A[M][K] W^T with fp32 A, fp16 W and fp32 accumulation: up to 16 rows
 // of A on the fp16 batch kernels (the weights need no dequantization; A is
 // rounded to fp16 after the per-window power-of-two scaling, as every batch
-// GEMV here does), more on the tiled GEMM (A scaled by row), or in batches of
-// 16 where that has no scratch memory or would not pay.
+// GEMV here does), more on the tiled GEMM (A scaled by row, far smaller
+// windows by themselves), or in batches of 16 where that has no scratch memory or would not pay.
 namespace {
 // fp16 weights of any K or alignment (the matrix-core kernel needs K % 32 == 0
 // and 16-byte rows): one workgroup of 4 waves per output column n, each wave

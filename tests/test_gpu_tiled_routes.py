@@ -196,6 +196,97 @@ def test_f16w_tiled(dev, m, n, k):
     assert bool((c[m] == 7.0).all())
 
 
+# Rows of every tile shape and conversion kernel of the two routes that scale
+# windows of 256 k by themselves: (fp16 weights?, m, n, k)
+WINDOW_SHAPES = [
+    (True, 300, 4100, 512), (True, 641, 4200, 1024), (True, 700, 8300, 512), (True, 4865, 5300, 512),  # tiles
+    (True, 50, 130, 4064), (True, 100, 300, 4096),      # K parts, 64 and 128 rows
+    (True, 64, 300, 16384), (True, 1030, 600, 5120), (True, 50, 100, 33024),  # conversions
+    (False, 49, 33, 4352), (False, 300, 4100, 4352), (False, 641, 4200, 4352), (False, 700, 8300, 4352),
+    (False, 4865, 5300, 4352), (False, 64, 1000, 14336),  # (the last: K parts)
+]
+
+
+def _window_weights(f16, n, k, live):
+    """Weights that are zero outside of row n's window live[n] (None: none zero):
+    as the call takes them, and in float64."""
+    import gq
+    import torch
+    if f16:
+        w = torch.randn(n, k, generator=torch.Generator().manual_seed(n)).cuda().half()
+        if live is not None:
+            w *= live.cuda()[:, None] == torch.arange(k, device="cuda")[None] // 256
+        return w, w.double()
+    b = O.gen_weights(O.Q6_K, n, k, seed=n).reshape(n, k // 256, 210)
+    if live is not None:
+        dead = live.numpy()[:, None] != np.arange(k // 256)[None]
+        b[dead, :128] = 0      # code 32 in all places: weight 0
+        b[dead, 128:192] = 0xAA
+    b = b.reshape(-1)
+    return (torch.from_numpy(gq.repack_host(O.Q6_K, b, n, k)).cuda(),
+            torch.from_numpy(O.dequant(O.Q6_K, b).reshape(n, k)).cuda().double())
+
+
+def _window_run(f16, w, a, n, k):
+    import gq
+    return gq.gemm_f16w(w, a, n, k) if f16 else gq.matmul(O.Q6_K, w, a, n, k)
+
+
+@pytest.mark.parametrize("f16,m,n,k", WINDOW_SHAPES)
+def test_small_windows_beside_large_ones(dev, f16, m, n, k):
+    """Windows of a row up to 2^80 apart, each output from one of them alone: all
+    keep their bits.  A is rounded once to fp16, 2^-11 of each product (Q6_K: its
+    scales and weights once each too), and an entry 2^-29 or less of the row's, where
+    its window is not scaled up, to 2^-19 of the window's largest."""
+    import torch
+    g = torch.Generator().manual_seed(m)
+    nw = -(-k // 256)
+    w, wd = _window_weights(f16, n, k, torch.arange(n) % nw)
+    a = torch.randn(m, k, generator=g).cuda()
+    down = torch.randint(0, 81, (m, nw), generator=g).cuda()
+    down[torch.arange(m) % 3 == 1] //= 8   # up to 10: not scaled
+    down[torch.arange(m) % 3 == 2] //= 3   # around the limit of 20
+    a *= torch.exp2(-down.double()).float().repeat_interleave(256, 1)[:, :k]
+    a[3 % m] = 0.0
+    ref = a.double() @ wd.t()
+    top = torch.nn.functional.pad(a.double().abs(), (0, 256 * nw - k)).reshape(m, nw, 256).amax(2)
+    tol = (2.0**-10 if f16 else 2.0**-9) * (a.double().abs() @ wd.abs().t())
+    tol += 2.0**-18 * top[:, torch.arange(n, device="cuda") % nw] * wd.abs().sum(1)
+    c = _window_run(f16, w, a, n, k)
+    bad = (c.double() - ref).abs() > tol
+    assert not bool(bad.any()), (int(bad.sum()), bad.nonzero()[:4])
+    # rows without such windows: the bits they have in a call of their own kind
+    if m > 64:
+        b = torch.randn(m, k, generator=g).cuda()
+        x = b.clone()
+        x[5] = a[0]
+        y, z = _window_run(f16, w, b, n, k), _window_run(f16, w, x, n, k)
+        y[5] = z[5]
+        assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("f16,m,n,k", WINDOW_SHAPES[3:10])
+def test_large_values_beside_an_inf(dev, f16, m, n, k):
+    """Finite values past fp16's range in a row with an Inf stay finite: the outputs
+    are Infs by the sign of the Inf's weight, not the NaN of two Infs."""
+    import torch
+    g = torch.Generator().manual_seed(m)
+    w, wd = _window_weights(f16, n, k, None)
+    a = torch.randn(m, k, generator=g).cuda()
+    rows = torch.arange(0, m, 7, device="cuda")
+    a[rows] *= 1e9
+    col = (rows * 131) % k
+    a[rows, col] = float("inf")
+    c = _window_run(f16, w, a, n, k)
+    at = wd[:, col].t()
+    want = torch.sign(at) * float("inf")  # (0: NaN)
+    assert torch.equal(torch.nan_to_num(c[rows].double(), nan=0.0, posinf=1.0, neginf=-1.0),
+                       torch.nan_to_num(want, nan=0.0, posinf=1.0, neginf=-1.0))
+    rest = torch.ones(m, dtype=torch.bool, device="cuda")
+    rest[rows] = False
+    assert _rel(c[rest], a[rest].double() @ wd.t()) <= TOL
+
+
 @pytest.mark.parametrize("m,n,k", [(49, 1, 32), (64, 3, 64), (50, 7, 32), (70, 1, 288), (300, 2, 96)])
 def test_f16w_fewer_weights_than_a_padded_row(dev, m, n, k):
     """Steps past K start beyond the matrix's end: they read zeros, not the Inf
