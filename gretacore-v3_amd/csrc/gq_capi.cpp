@@ -364,12 +364,16 @@ int gq_matmul(int fmt, const void *packed, const float *a, float *c, size_t M, s
     return gq_gemv(fmt, packed, a, c, N, K, (int)M, nullptr, 0, stream);
   if (gq_fmt_is_q6k(fmt) && (K > 4096 || M == 0 || N == 0 || K == 0)) {
     // gq_gemm refuses Q6_K past K = 4096: the tiled kernel on scratch memory,
-    // or batches of 16 rows through the GEMV where there is none.  Two or three
-    // GEMV passes over few columns also beat the tiled kernel, whose few
-    // workgroups each walk K in steps (17 / 33 / 48 / 64 rows, 4096 x 14336: GEMVs
-    // 38 / 66 / 82 / 109 us, tiled 79 / 79 / 80 / 82; 14336 x 14336: 83 / 132 / 143 /
-    // 190 against 95 / 96 / 98 / 100; 512 x 4096 x 14336: 861 against 99)
-    if ((M > 48 || (M > 32 && N >= 8192)) && M <= GQ_MAX_DIM && N > 0 && K > 0 && packed && a && c &&
+    // or batches of 16 rows through the GEMV where there is none.  Up to K = 8192, where
+    // the tiled kernel's workgroups each walk all of K, two or three GEMV passes beat
+    // it over few columns; past that K is split over workgroups, and they do so only
+    // up to 23 rows of a small matrix (17 / 24 / 32 / 33 / 48 rows, GEMVs | tiled, us: 4096 x
+    // 4352 17 / 22 / 25 / 29 / 36 | 33, 4096 x 8192 22 / 29 / 33 / 38 / 48 | 50, 14336 x 8192 48 /
+    // 53 / 56 / - | 53 / 52 / 52 / 52, 1024 x 14336 24 / 34 / 34 / 41 / 51 | 30, 4096 x 14336 35 / 44 /
+    // 51 / 61 / 79 | 35, 2048 x 28672 58 / 61 / 57 / 87 / 85 | 39, 14336 x 14336 81 / 82 / 91 / - |
+    // 58 / 58 / 59 / 59)
+    const bool few = K > 8192 ? M < 24 && N * K < (size_t)56 << 20 : M <= 32 || (M <= 48 && N < 8192);
+    if (!few && M <= GQ_MAX_DIM && N > 0 && K > 0 && packed && a && c &&
         gq_check_shape(fmt, N, K) == GQ_OK) {
       const int r = gq_launch_matmul_q6k(fmt, packed, a, c, M, N, K, (hipStream_t)stream);
       if (r != GQ_ERR_WORKSPACE && r != GQ_ERR_UNSUPPORTED) return r;

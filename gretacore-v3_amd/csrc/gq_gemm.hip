@@ -835,7 +835,7 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
   // the group's l-th step of K
   // fp16 rows at a power-of-two stride put every workgroup's step on the same
   // few memory channels: each weight column tile starts its walk one step
-  // further on (fragments loaded into registers, 17 / 100 rows x 32000 x 4096: 70.5 / 80.2 -> 62.3 / 75.1 us; the T16
+  // further on (17 / 100 rows x 32000 x 4096: 55.4 / 62.2 -> 54.6 / 61.2 us; the T16
   // formats, whose tiles are contiguous, gain nothing)
   const int off = FMT == GQ_FMT_F16 ? nt % nl : 0;
   auto gstep = [&](int l) {
@@ -1523,8 +1523,9 @@ int launch_fmt_kg(const void *packed, const _Float16 *a16, int lda, void *c, con
 // Few workgroups (a short, narrow C over a long K): K in parts over workgroups,
 // each part's sums in fp32 in `part`, added by k_split_sum.  About one
 // workgroup per CU, at least 8 steps a part, and only from 32 steps on: fp16 weights,
-// 64 rows, unsplit / split (weights loaded into registers): 4096 x 14336 174 / 47 us, 4096 x 4096 46 / 24, 300 x 14336
-// 130 / 28; 4096 x 1120 (20 steps) 18.6 / 20.3.
+// 64 rows, unsplit / split: 4096 x 14336 99 / 35 us, 4096 x 4096 34 / 21.5, 300 x 14336
+// 99.5 / 24.5; 100 rows of 4096 x 2048 (32 steps) 21.0 / 21.6; 4096 x 1120 (20 steps) 17.3 /
+// 18.1.
 struct SplitPlan {
   int bm, splits;  // tile rows (64 x 128 or 128 x 128, in two K groups)
 };

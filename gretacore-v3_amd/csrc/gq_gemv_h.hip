@@ -1103,8 +1103,9 @@ int gq_launch_gemv_h(int fmt, const void *packed, const float *x, float *y, int 
 // C[M][N] = A[M][K] W^T with fp32 A, fp16 W and fp32 accumulation: up to 16 rows
 // of A on the fp16 batch kernels (the weights need no dequantization; A is
 // rounded to fp16 after the per-window power-of-two scaling, as every batch
-// GEMV here does), more on the tiled GEMM (A scaled by row, far smaller
-// windows by themselves), or in batches of 16 where that has no scratch memory or would not pay.
+// GEMV here does), more on the tiled GEMM (A scaled by row, far smaller windows
+// by themselves), or in batches of 16 where that has no scratch memory or would
+// not pay.
 namespace {
 // fp16 weights of any K or alignment (the matrix-core kernel needs K % 32 == 0
 // and 16-byte rows): one workgroup of 4 waves per output column n, each wave
@@ -1140,13 +1141,13 @@ extern "C" int gq_gemm_f16w(const void *w, const float *a, float *c, size_t M, s
                        (int)K);
     return gq_last_launch();
   }
-  // two or three passes over a small matrix cost less than the conversion, the
-  // scratch and a grid of few workgroups (17 rows, tiled against two GEMVs: 300 x
-  // 512 18.0 / 11.6 us, 14336 x 1024 22.4 / 18.2, 4096 x 1120 18.0 / 18.6, 4096 x 2048
-  // 21.6 / 19.1, 14336 x 2048 26.5 / 31.1, 4096 x 4096 23.9 / 23.3; 33 rows: 4096 x 512
-  // 17.9 / 15.8, 14336 x 512 18.3 / 23.2)
-  const size_t pass = (M + 15) / 16, nk = N * K, m1 = (size_t)1 << 20;
-  const bool small = pass == 2 ? K <= 2048 && nk <= (K <= 1024 ? 16 : 9) * m1 : pass == 3 && K <= 1024 && nk <= 5 * m1;
+  // two passes over a small matrix cost less than the conversion, the scratch and a
+  // grid of few workgroups (17 / 32 rows, two GEMVs | tiled, us: 300 x 512 10.0 / 10.5 |
+  // 13.2, 4096 x 512 10.3 / 10.9 | 12.8, 1024 x 1024 14.1 / 15.0 | 15.8, 4096 x 1024 14.8 /
+  // 15.8 | 15.4, 4096 x 1120 15.7 / 16.8 | 16.7, 1024 x 2048 14.4 / 15.4 | 16.3, 14336 x 512
+  // 15.2 / 14.9 | 13.3, 4096 x 2048 17.7 / 19.6 | 16.6; three passes lose: 300 x 512 15.1 |
+  // 13.2, 1024 x 1024 21.7 | 15.9)
+  const bool small = M <= 2 * GQ_MAX_BATCH && K <= 2048 && N * K <= (size_t)5 << 20;
   if (M > GQ_MAX_BATCH && !small) {
     const int r = gq_launch_gemm_f16w(w, a, c, M, N, K, s);
     if (r != GQ_ERR_WORKSPACE && r != GQ_ERR_UNSUPPORTED) return r;

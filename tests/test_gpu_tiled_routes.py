@@ -59,7 +59,10 @@ def test_q6k_gemm_skinny_or_tiled(dev, m, n, k):
     assert _rel(gq.gemm(O.Q6_K, packed, a, n, k), _ref(O.Q6_K, w, a, n, k)) <= TOL
 
 
-@pytest.mark.parametrize("m,n,k", [(49, 33, 4352), (33, 8192, 4352), (130, 8200, 4608), (300, 100, 14336)])
+@pytest.mark.parametrize("m,n,k", [
+    (49, 33, 4352), (33, 8192, 4352), (130, 8200, 4608), (300, 100, 14336),
+    (48, 33, 4352), (23, 1000, 14336), (24, 1000, 14336), (17, 4200, 14336),  # about the GEMV passes' limits
+])
 def test_q6k_matmul_long_k(dev, m, n, k):
     """K > 4096: the tiled kernel on scratch memory, the 16-row GEMVs under
     capture; the same within the bound, replayed with eager calls between."""
@@ -176,6 +179,7 @@ def test_scratch_of_many_streams_and_sizes(dev):
     (17, 33, 4128),       # K in parts, 64-row tiles, an odd count of outputs
     (131, 300, 14304),    # K in parts of unequal length, 128-row tiles
     (17, 100, 64), (40, 64, 512), (49, 64, 512),  # about the batch GEMVs' limits
+    (32, 64, 512), (33, 64, 512), (17, 2560, 2048), (17, 2561, 2048),
 ])
 def test_f16w_tiled(dev, m, n, k):
     """Columns past K hold Inf in the next row's weights: they must not count."""
