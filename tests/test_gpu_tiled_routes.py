@@ -291,6 +291,24 @@ def test_large_values_beside_an_inf(dev, f16, m, n, k):
     assert _rel(c[rest], a[rest].double() @ wd.t()) <= TOL
 
 
+@pytest.mark.parametrize("f16,k,fit", [(True, 16384, 3840), (False, 16128, 4096)])
+@pytest.mark.parametrize("extra", [1, 70])
+def test_second_block_of_rows(dev, f16, k, fit, extra):
+    """More rows than one scratch block converts at a time: the last block, of a few
+    rows, takes another tile (and could split K).  Every row against float64."""
+    import torch
+    m, n = fit + extra, 70
+    w, wd = _window_weights(f16, n, k, None)
+    a = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(extra), device="cuda")
+    c = _window_run(f16, w, a, n, k)
+    worst = 0.0
+    for r in range(0, m, 512):
+        ref = a[r:r + 512].double() @ wd.t()
+        worst = max(worst, float(((c[r:r + 512].double() - ref).norm(dim=1) / ref.norm(dim=1)).max()))
+    # one row of 70 outputs: a little over the bound of a long row
+    assert worst <= 2 * TOL, worst
+
+
 @pytest.mark.parametrize("m,n,k", [(49, 1, 32), (64, 3, 64), (50, 7, 32), (70, 1, 288), (300, 2, 96)])
 def test_f16w_fewer_weights_than_a_padded_row(dev, m, n, k):
     """Steps past K start beyond the matrix's end: they read zeros, not the Inf
