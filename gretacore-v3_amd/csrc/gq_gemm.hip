@@ -509,8 +509,7 @@ GQ_DEV void load_rstep(const uint8_t *w, const uint32_t (&qo)[NJ], const uint32_
                        RStep<FMT, NJ> &st) {
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if constexpr (FMT == GQ_FMT_F16) {
-    } else if constexpr (FMT == GQ_FMT_Q4_0) {
+    if constexpr (FMT == GQ_FMT_Q4_0) {
       const uint32_t b = ((uint32_t)(step >> 1) << 10) + 8u * (uint32_t)(step & 1);
       st.q[j][0] = ld8_b(w, qo[j], b);
       st.q[j][1] = ld8_b(w, qo[j] + 512u, b);
@@ -658,8 +657,6 @@ GQ_DEV void q6k_factors(const RStep<GQ_FMT_Q6_K, NJ> &st, int kh, gq_half2 (&f)[
 template <int FMT, int NJ>
 GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const QKf *qk, const gq_half2 *q6,
                       uint32_t mg) {
-  if constexpr (FMT == GQ_FMT_F16) return gq_half8{};  // (read from LDS)
-  else {
   const int h = ks >> 1;
   gq_half2 p[4];
   if constexpr (FMT == GQ_FMT_Q6_K) {
@@ -708,7 +705,6 @@ GQ_DEV gq_half8 rfrag(const RStep<FMT, NJ> &st, int j, int ks, int step, const Q
     o[2 * i + 1] = p[i][1];
   }
   return o;
-  }
 }
 
 // Workgroup tile BM x BN, WM x WN waves; a wave owns (BM / WM) x (BN / WN) of C
@@ -911,7 +907,9 @@ k_gemm_rb(const uint8_t *__restrict__ w, uint32_t sc_off, const _Float16 *__rest
       if (ks + 1 < KS) read_a(ks + 1, (ks + 1) & 1);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const gq_half8 bf = LB ? bl[ks & 1][j] : rfrag<FMT, NJ>(cur, j, ks, step, qk[j], q6[j], mg);
+        gq_half8 bf;
+        if constexpr (LB) bf = bl[ks & 1][j];
+        else bf = rfrag<FMT, NJ>(cur, j, ks, step, qk[j], q6[j], mg);
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[i][j] = gq_mfma32(af[ks & 1][i], bf, acc[i][j]);
       }

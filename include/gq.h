@@ -51,8 +51,9 @@ extern "C" {
    kernel); gq_gemv_multi / gq_gemv_swiglu run their fallback for it (RMSNorm,
    one gq_gemv per matrix); gq_gemm with longer K and gq_gemv_prep / prepped
    return GQ_ERR_UNSUPPORTED for it.  gq_matmul takes any K: beyond 4096 the tiled
-   kernel on scratch memory of the call's own (stream-ordered), or 16-row GEMV
-   batches up to 48 rows and while the stream is being captured. */
+   kernel on scratch memory of the call's own, or 16-row GEMV batches where these
+   are the quicker (up to 48 rows and K = 8192, 23 rows of a small matrix beyond) and
+   while the stream is being captured. */
 
 /* activation / output dtypes */
 #define GQ_DT_F32 0
@@ -187,7 +188,7 @@ int gq_gemv_swiglu_plan(int fmt, size_t N, size_t K, int batch, int *ksplit, int
  * (M <= 256 where the grid stays within one workgroup per CU, or two for K
  * beyond 4096) run on a skinny kernel that splits K over the waves of a
  * workgroup; small tiled grids split K over 2 or 4 wave groups of a
- * workgroup, and few tiles on a K of 8192 or more over workgroups as well (the
+ * workgroup, and few tiles on a K beyond 8192 over workgroups as well (the
  * parts' fp32 sums in scratch memory of the call's own; not while the stream is
  * being captured, where the sums round in another order). */
 size_t gq_gemm_workspace_bytes(int fmt, size_t M, size_t K);
