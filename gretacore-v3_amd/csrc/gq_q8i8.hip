@@ -5,8 +5,9 @@
 // products (oracle gqo_gemm_q8_i8).
 //
 // Both operands carry a scale per 32-block, so every block of every output
-// costs VALU work after its MFMA: the route is VALU-bound, not MFMA-bound.  Two
-// instructions per output remain (32 per 32 x 32 x 32 MFMA): the MFMA
+// costs VALU work after its MFMA (at 512 x 14336 x 4096 the VALU issues in 50 % of
+// the cycles, the MFMA is busy in 10 %; 448 tiles on 512 places and waits are the
+// rest).  Two instructions per output remain (32 per 32 x 32 x 32 MFMA): the MFMA
 // accumulates onto the bits of 1.5 * 2^23, so its int32 result m + p (|p| < 2^20)
 // read as a float is 1.5 * 2^23 + p; fma(d_w, that, -1.5 * 2^23 d_w) is d_w p rounded
 // once (the constant is exact: d_w has 11 bits), and a second fma multiplies by
