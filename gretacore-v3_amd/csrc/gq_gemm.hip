@@ -1670,7 +1670,8 @@ int gq_launch_gemm_f16w(const void *w, const float *a, float *c, size_t M, size_
   GQ_CHECK(N * K * 2 + Kp * 2 < ((size_t)1 << 32) && 256 * (row + 20) <= kGqScratchMax - (1 << 20), GQ_ERR_UNSUPPORTED);
   const size_t fit = ((kGqScratchMax - (1 << 20)) / (row + 20)) & ~(size_t)255, mb = M < fit ? M : fit;
   // (row scales read by the tile, window shifts)
-  const size_t abytes = gq_align256(mb * Kp * 2), rbytes = gq_align256((mb + 256) * 4), hbytes = gq_align256((mb + 3) / 4 * 4 * (Kp / 256));
+  const size_t abytes = gq_align256(mb * Kp * 2), rbytes = gq_align256((mb + 256) * 4);
+  const size_t hbytes = gq_align256((mb + 3) / 4 * 4 * (Kp / 256));
   const SplitPlan sp = split_plan((int)mb, (int)N, (int)(Kp / BK));
   const size_t pbytes = sp.splits > 1 ? (size_t)sp.splits * M * N * 4 : 0;
   const bool split = sp.splits > 1 && mb == M && abytes + rbytes + hbytes + pbytes <= kGqScratchMax;
